@@ -244,39 +244,191 @@ __global__ void k_zero_out(double *phi, int64_t n, double *acc)
 }
 
 // Direct sum in input order over all n mass-set bodies (self skipped by
-// index), for the targets idx[0..nt) of the mass set.
-constexpr int kDirTile = 256;
-__global__ __launch_bounds__(kTpb) void k_direct(const double *__restrict__ pos, const double *__restrict__ mass,
-                                                 int64_t n, const int64_t *__restrict__ idx, int64_t nt, double eps,
-                                                 double *phi_out, double *acc_out)
+// index), for the targets idx[0..nt) of the mass set.  Every target's sums
+// run over the sources in input order (bit for bit directcode's), so a
+// target's additions are one serial chain of n; the terms of that chain (a
+// square root and two divisions each, ~60 FP64 instructions) are independent.
+// A block takes TB targets: its first kDirProd waves compute the terms of K
+// sources x TB targets per stage into LDS while the other waves add the
+// previous stage's terms, one thread per (target, component) in source order
+// and fetch the next stage's sources.  A self pair adds a zero, which
+// leaves every sum as it is (no sum is ever -0.0: it starts at +0.0).
+// Bound: the FP64 vector ALU (about 45 instructions a pair).  One thread per
+// target, each with its own chain of roots and divisions, kept 8192 targets on
+// 32 of the 256 CUs: 8192 targets of 2^20 bodies took 222 ms; this layout with
+// plain roots and divisions 31 ms, with the sources loaded a stage ahead and
+// softened()'s shared reciprocals 21.8 ms (3.9e11 pairs/s).  Six term and two
+// adding waves in blocks of half the size, two to a CU, measured alike.
+constexpr int kDirProd = 12, kDirCons = 4;              // waves computing terms, waves adding them
+constexpr int kDirPer = 2;                              // terms per thread and stage
+constexpr int kDirTerms = 64 * kDirProd * kDirPer;      // terms per stage
+constexpr int kDirTpb = 64 * (kDirProd + kDirCons);
+constexpr int kDirRun = 24;                             // terms an adding thread reads ahead
+
+// Magnitudes the short form of softened() handles: 2^-400 .. 2^400.
+constexpr int kExpLo = (1023 - 400) << 20, kExpSpan = 800 << 20;
+__device__ __forceinline__ bool mid_range(double a)
 {
-    __shared__ double4 tile[kDirTile];
-    int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    const bool act = t < nt;
-    int64_t i = act ? idx[t] : 0;
-    double x = pos[3 * i], y = pos[3 * i + 1], z = pos[3 * i + 2];
-    Acc64 a;
-    for (int64_t base = 0; base < n; base += kDirTile) {
-        __syncthreads();
-        int64_t j = base + threadIdx.x;
-        if (j < n) tile[threadIdx.x] = make_double4(pos[3 * j], pos[3 * j + 1], pos[3 * j + 2], mass[j]);
-        __syncthreads();
-        int lim = (int)std::min<int64_t>(kDirTile, n - base);
-        for (int k = 0; k < lim; k++) {
-            if (base + k == i) continue;
-            double4 b = tile[k];
-            double dx = b.x - x, dy = b.y - y, dz = b.z - z;
-            double drsq = dx * dx;
-            drsq += dy * dy;
-            drsq += dz * dz;
-            gravsub64(a, dx, dy, dz, drsq, b.w, eps, nullptr);
+    return (unsigned)((__double2hiint(a) & 0x7fffffff) - kExpLo) < (unsigned)kExpSpan;
+}
+
+// phii = m / sqrt(a) and mor3 = phii / a, each operation correctly rounded as
+// the plain expressions are.  The short form shares one reciprocal square
+// root: Goldschmidt's iteration on the hardware estimate gives g ~ sqrt(a)
+// and h ~ 1/(2 sqrt(a)), the exact residual a - g^2 rounds the root, and each
+// quotient is corrected by its exact residual with a reciprocal accurate to
+// the last bit (Markstein, IBM J. Res. Dev. 34, 1990): 24 multiply-adds and
+// one estimate in the place of a root and two divisions of ~18 instructions
+// and an estimate each.  It needs magnitudes far from overflow and underflow;
+// others (and a self pair at eps = 0) take the plain expressions.  odd: some
+// mass of the stage is neither 0 nor of such a magnitude.  A pair that is off
+// gives zeros (the short form by a mass of 0).  Returns whether the short
+// form was taken.
+template <int N>
+__device__ __forceinline__ bool softened(const double *a, double *m, const bool *on, int odd, double *phii,
+                                         double *mor3)
+{
+    bool mid = !odd;
+#pragma unroll
+    for (int u = 0; u < N; u++) mid = mid && mid_range(a[u]);
+    if (__builtin_expect(!__all(mid), 0)) {
+        for (int u = 0; u < N; u++) {
+            phii[u] = on[u] ? m[u] / sqrt(a[u]) : 0.0;
+            mor3[u] = on[u] ? phii[u] / a[u] : 0.0;
         }
+        return false;
     }
-    if (act) {
-        phi_out[t] = a.phi;
-        acc_out[3 * t] = a.ax;
-        acc_out[3 * t + 1] = a.ay;
-        acc_out[3 * t + 2] = a.az;
+    double g[N], h[N], s[N], y[N], z[N], q[N];
+    // (one operation on all N pairs at a time: N independent chains)
+#define BH_EACH _Pragma("unroll") for (int u = 0; u < N; u++)
+    BH_EACH m[u] = on[u] ? m[u] : 0.0;
+    BH_EACH h[u] = __builtin_amdgcn_rsq(a[u]);
+    BH_EACH g[u] = a[u] * h[u];
+    BH_EACH h[u] = 0.5 * h[u];
+#pragma unroll
+    for (int it = 0; it < 2; it++) {
+        BH_EACH q[u] = fma(-h[u], g[u], 0.5);
+        BH_EACH g[u] = fma(g[u], q[u], g[u]);
+        BH_EACH h[u] = fma(h[u], q[u], h[u]);
+    }
+    BH_EACH q[u] = fma(-g[u], g[u], a[u]);
+    BH_EACH s[u] = fma(q[u], h[u], g[u]);               // sqrt(a)
+    BH_EACH y[u] = h[u] + h[u];
+    BH_EACH q[u] = fma(-s[u], y[u], 1.0);
+    BH_EACH y[u] = fma(q[u], y[u], y[u]);               // 1 / s
+    BH_EACH g[u] = m[u] * y[u];
+    BH_EACH z[u] = y[u] * y[u];
+    BH_EACH q[u] = fma(-g[u], s[u], m[u]);
+    BH_EACH h[u] = fma(-a[u], z[u], 1.0);
+    BH_EACH phii[u] = fma(q[u], y[u], g[u]);            // m / s
+    BH_EACH z[u] = fma(h[u], z[u], z[u]);               // 1 / a
+    BH_EACH g[u] = phii[u] * z[u];
+    BH_EACH q[u] = fma(-g[u], a[u], phii[u]);
+    BH_EACH mor3[u] = fma(q[u], z[u], g[u]);            // phii / a
+#undef BH_EACH
+    return true;
+}
+
+template <int TB>
+__global__ __launch_bounds__(kDirTpb) void k_direct(const double *__restrict__ pos, const double *__restrict__ mass,
+                                                    int64_t n, const int64_t *__restrict__ idx, int64_t nt, double eps,
+                                                    double *phi_out, double *acc_out)
+{
+    constexpr int K = kDirTerms / TB;                   // sources per stage
+    static_assert(kDirTerms % TB == 0 && K % kDirRun == 0 && 64 % TB == 0 && K <= 64 * kDirCons && 4 * TB <= 64 * kDirCons, "stage shape");
+    __shared__ double4 src[2][K];
+    __shared__ int odd[2];                              // a mass of the stage outside softened()'s short form
+    __shared__ double term[2][4][kDirTerms];            // [buffer][-phi, ax, ay, az][source * TB + target]
+    const int tid = threadIdx.x;
+    const int64_t t0 = (int64_t)blockIdx.x * TB;
+    const int64_t nstage = (n + K - 1) / K;
+    const bool prod = tid < 64 * kDirProd;
+    const int q = tid - 64 * kDirProd;                  // adding threads: 0 ..
+    const int tl = prod ? tid % TB : q % TB;            // target in the block
+    const int64_t t = t0 + tl;
+    const int64_t i = t < nt ? idx[t] : idx[t0];
+    const double x = pos[3 * i], y = pos[3 * i + 1], z = pos[3 * i + 2];
+    auto source = [&](int64_t j) {
+        return j < n ? make_double4(pos[3 * j], pos[3 * j + 1], pos[3 * j + 2], mass[j]) : make_double4(0, 0, 0, 0);
+    };
+    auto odd_mass = [](double m) { return m != 0.0 && !mid_range(m); };
+    if (tid < 2) odd[tid] = 0;
+    __syncthreads();
+    if (!prod && q < K) {
+        src[0][q] = source(q);
+        if (odd_mass(src[0][q].w)) odd[0] = 1;
+    }
+    __syncthreads();
+    double sum = 0.0;
+    // the sources of stage s + 1, loaded during stage s - 1 (a global load takes
+    // longer than a stage)
+    double4 o = make_double4(0, 0, 0, 0);
+    if (!prod && q < K) o = source(K + q);
+    if (!prod) __builtin_amdgcn_s_setprio(3);           // the serial chain first, the terms around it
+    for (int64_t s = 0; s <= nstage; s++) {
+        const int b = (int)(s & 1);
+        // the stage's sources, and the target's own body among them
+        const int left = (int)min<int64_t>(K, n - s * K);
+        const int self = (int)max<int64_t>(-1, min<int64_t>(K, i - s * K));
+        if (prod) {
+            if (s < nstage) {
+                double dx[kDirPer], dy[kDirPer], dz[kDirPer], r2[kDirPer], m[kDirPer], phii[kDirPer], mor3[kDirPer];
+                bool on[kDirPer];
+#pragma unroll
+                for (int u = 0; u < kDirPer; u++) {
+                    const int k = (tid + u * 64 * kDirProd) / TB;
+                    const double4 c = src[b][k];
+                    dx[u] = c.x - x;
+                    dy[u] = c.y - y;
+                    dz[u] = c.z - z;
+                    m[u] = c.w;
+                    double drsq = dx[u] * dx[u];
+                    drsq += dy[u] * dy[u];
+                    drsq += dz[u] * dz[u];
+                    r2[u] = drsq + eps * eps;
+                    on[u] = k != self && k < left;
+                }
+                if (!softened<kDirPer>(r2, m, on, odd[b], phii, mor3)) {
+#pragma unroll
+                    for (int u = 0; u < kDirPer; u++)   // (a non-finite offset times 0 is no zero)
+                        if (!on[u]) dx[u] = dy[u] = dz[u] = 0.0;
+                }
+#pragma unroll
+                for (int u = 0; u < kDirPer; u++) {
+                    const int e = tid + u * 64 * kDirProd;
+                    term[b][0][e] = -phii[u];
+                    term[b][1][e] = dx[u] * mor3[u];
+                    term[b][2][e] = dy[u] * mor3[u];
+                    term[b][3][e] = dz[u] * mor3[u];
+                }
+            }
+        } else {
+            if (q < K) {
+                src[b ^ 1][q] = o;
+                if (odd_mass(o.w)) odd[b ^ 1] = 1;      // (stays set: later stages only lose the short form)
+                o = source((s + 2) * K + q);
+            }
+            if (s > 0 && q < 4 * TB) {
+                // the next kDirRun terms are read while these are added
+                const double *v = term[b ^ 1][q / TB] + tl;
+                double c[2][kDirRun];
+#pragma unroll
+                for (int k = 0; k < kDirRun; k++) c[0][k] = v[k * TB];
+#pragma unroll
+                for (int r = 0; r < K / kDirRun; r++) {
+                    if (r + 1 < K / kDirRun)
+#pragma unroll
+                        for (int k = 0; k < kDirRun; k++) c[(r + 1) & 1][k] = v[((r + 1) * kDirRun + k) * TB];
+#pragma unroll
+                    for (int k = 0; k < kDirRun; k++) sum = sum + c[r & 1][k];
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (!prod && q < 4 * TB && t < nt) {
+        if (q / TB == 0) phi_out[t] = sum;
+        else acc_out[3 * t + q / TB - 1] = sum;
     }
 }
 
@@ -307,11 +459,30 @@ double *cell_rcrit(bh_ctx *ctx, const bh_params &p, const uint64_t *keys, const 
     return rc2;
 }
 
+// Targets per block: the split with the least work on the busiest CU (one
+// block per CU at a time: ~110 KB of LDS), TB times the rounds of blocks.  Not
+// below 8 targets, where the serial additions are the bound (2^20 bodies: 9.6
+// ms for 256 targets, 9.2 ms for 1024, 21.8 ms for 8192).
 void direct_sum(bh_ctx *ctx, double eps, int64_t nidx, const int64_t *d_idx, double *d_phi, double *d_acc)
 {
-    int grid = (int)std::max<int64_t>(1, (nidx + kTpb - 1) / kTpb);
-    k_direct<<<grid, kTpb, 0, ctx->stream>>>(ptr<double>(ctx->pos), ptr<double>(ctx->mass), ctx->nmass, d_idx, nidx, eps,
-                                             d_phi, d_acc);
+    int best = 64;
+    int64_t cost = INT64_MAX;
+    for (int tb : {64, 32, 16, 8}) {
+        const int64_t blocks = (nidx + tb - 1) / tb, c = (blocks + ctx->ncu - 1) / ctx->ncu * tb;
+        if (c < cost) {
+            cost = c;
+            best = tb;
+        }
+    }
+    const int grid = (int)((nidx + best - 1) / best);
+    const double *pos = ptr<double>(ctx->pos), *mass = ptr<double>(ctx->mass);
+    auto go = [&](auto kernel) {
+        kernel<<<grid, kDirTpb, 0, ctx->stream>>>(pos, mass, ctx->nmass, d_idx, nidx, eps, d_phi, d_acc);
+    };
+    if (best == 64) go(k_direct<64>);
+    else if (best == 32) go(k_direct<32>);
+    else if (best == 16) go(k_direct<16>);
+    else go(k_direct<8>);
     BH_HIP(hipGetLastError());
 }
 
