@@ -41,7 +41,7 @@
 // A body's own contribution is removed exactly: with eps > 0 the self pair
 // adds m*rsq(eps^2) to the potential sum and nothing to the acceleration, so
 // that term is subtracted at the end; with eps == 0 the kernel masks r = 0.
-#include "bh_ctx.h"
+#include "bh_walk.h"
 
 #include <algorithm>
 
@@ -51,317 +51,6 @@ namespace {
 constexpr int kWaves = 4;          // waves per block
 constexpr int kTpb = 64 * kWaves;
 constexpr int kListCap = 128;      // entries per list (a tile is 64)
-
-__device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
-
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ __forceinline__ float wave_min(float v)
-{
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = fminf(v, __shfl_xor(v, d, 64));
-    return v;
-}
-__device__ __forceinline__ float wave_max(float v)
-{
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = fmaxf(v, __shfl_xor(v, d, 64));
-    return v;
-}
-__device__ __forceinline__ int wave_min_i(int v)
-{
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = min(v, __shfl_xor(v, d, 64));
-    return v;
-}
-__device__ __forceinline__ int wave_max_i(int v)
-{
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = max(v, __shfl_xor(v, d, 64));
-    return v;
-}
-__device__ __forceinline__ int wave_excl_scan(int v, int *total)
-{
-    const int lane = lane_id();
-    int x = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        int t = __shfl_up(x, d, 64);
-        if (lane >= d) x += t;
-    }
-    *total = __shfl(x, 63, 64);
-    return x - v;
-}
-__device__ __forceinline__ int mbcnt(unsigned long long m)
-{
-    return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
-}
-
-// TwoSum fold of a tile sum into a compensated accumulator.
-__device__ __forceinline__ void fold(float &hi, float &lo, float v)
-{
-    float s = hi + v;
-    float bb = s - hi;
-    float err = (hi - (s - bb)) + (v - bb);
-    hi = s;
-    lo += err;
-}
-
-__device__ __forceinline__ float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
-
-template <int NPL>
-struct Lane {
-    float px[NPL], py[NPL], pz[NPL];
-    float axh[NPL], axl[NPL], ayh[NPL], ayl[NPL], azh[NPL], azl[NPL], ph[NPL], pl[NPL];
-};
-
-// NQ <= NPL: the particle slots in use (a group of at most 64 points uses
-// one slot per lane).
-template <int NPL, int NQ, bool SOFT0>
-__device__ __forceinline__ void eval_p2p(Lane<NPL> &L, const float4 *src, int cnt, float eps2)
-{
-    float sx[NPL], sy[NPL], sz[NPL], sp[NPL];
-#pragma unroll
-    for (int q = 0; q < NQ; q++) sx[q] = sy[q] = sz[q] = sp[q] = 0.f;
-#pragma unroll 4
-    for (int j = 0; j < cnt; j++) {
-        const float4 s = src[j];
-#pragma unroll
-        for (int q = 0; q < NQ; q++) {
-            float dx = s.x - L.px[q], dy = s.y - L.py[q], dz = s.z - L.pz[q];
-            float r2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
-            float ri = rsq(r2);
-            if (SOFT0) ri = r2 > 0.f ? ri : 0.f;
-            float mr = s.w * ri;
-            sp[q] += mr;
-            float mr3 = mr * ri * ri;
-            sx[q] = fmaf(dx, mr3, sx[q]);
-            sy[q] = fmaf(dy, mr3, sy[q]);
-            sz[q] = fmaf(dz, mr3, sz[q]);
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-        fold(L.axh[q], L.axl[q], sx[q]);
-        fold(L.ayh[q], L.ayl[q], sy[q]);
-        fold(L.azh[q], L.azl[q], sz[q]);
-        fold(L.ph[q], L.pl[q], sp[q]);
-    }
-}
-
-// P2C entry: e[0] = (dx0, dy0, dz0, m) relative to the group centre,
-// e[1] = (qxx, qxy, qxz, qyy), e[2] = (qyz, qzz, -, -).
-template <int NPL, int NQ, bool QUAD, bool SOFT0>
-__device__ __forceinline__ void eval_p2c(Lane<NPL> &L, const float4 *src, int cnt, float eps2)
-{
-    constexpr int S = QUAD ? 3 : 1;
-    float sx[NPL], sy[NPL], sz[NPL], sp[NPL];
-#pragma unroll
-    for (int q = 0; q < NQ; q++) sx[q] = sy[q] = sz[q] = sp[q] = 0.f;
-#pragma unroll 2
-    for (int j = 0; j < cnt; j++) {
-        const float4 s = src[S * j];
-        float4 q0, q1;
-        if (QUAD) {
-            q0 = src[S * j + 1];
-            q1 = src[S * j + 2];
-        }
-#pragma unroll
-        for (int q = 0; q < NQ; q++) {
-            float dx = s.x - L.px[q], dy = s.y - L.py[q], dz = s.z - L.pz[q];
-            float r2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
-            float ri = rsq(r2);
-            if (SOFT0) ri = r2 > 0.f ? ri : 0.f;
-            float ri2 = ri * ri;
-            float mr = s.w * ri;
-            if (QUAD) {
-                float qx = fmaf(q0.x, dx, fmaf(q0.y, dy, q0.z * dz));
-                float qy = fmaf(q0.y, dx, fmaf(q0.w, dy, q1.x * dz));
-                float qz = fmaf(q0.z, dx, fmaf(q1.x, dy, q1.y * dz));
-                float dqd = fmaf(dx, qx, fmaf(dy, qy, dz * qz));
-                float r5 = ri2 * ri2 * ri;
-                float phq = -0.5f * r5 * dqd;          // quadrupole potential term
-                float coef = (mr - 5.f * phq) * ri2;   // radial factor of a
-                sp[q] += mr - phq;
-                sx[q] = fmaf(dx, coef, fmaf(-qx, r5, sx[q]));
-                sy[q] = fmaf(dy, coef, fmaf(-qy, r5, sy[q]));
-                sz[q] = fmaf(dz, coef, fmaf(-qz, r5, sz[q]));
-            } else {
-                float mr3 = mr * ri2;
-                sp[q] += mr;
-                sx[q] = fmaf(dx, mr3, sx[q]);
-                sy[q] = fmaf(dy, mr3, sy[q]);
-                sz[q] = fmaf(dz, mr3, sz[q]);
-            }
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-        fold(L.axh[q], L.axl[q], sx[q]);
-        fold(L.ayh[q], L.ayl[q], sy[q]);
-        fold(L.azh[q], L.azl[q], sz[q]);
-        fold(L.ph[q], L.pl[q], sp[q]);
-    }
-}
-
-// Tiles for the first nq particle slots of each lane (groups of at most
-// 64 nq points leave the other slots idle).
-template <int NPL, bool SOFT0>
-__device__ __forceinline__ void p2p_slots(int nq, Lane<NPL> &L, const float4 *src, int cnt, float eps2)
-{
-    if (nq <= 1) eval_p2p<NPL, 1, SOFT0>(L, src, cnt, eps2);
-    else if (NPL > 2 && nq == 2) eval_p2p<NPL, (NPL > 2 ? 2 : NPL), SOFT0>(L, src, cnt, eps2);
-    else if (NPL > 3 && nq == 3) eval_p2p<NPL, (NPL > 3 ? 3 : NPL), SOFT0>(L, src, cnt, eps2);
-    else eval_p2p<NPL, NPL, SOFT0>(L, src, cnt, eps2);
-}
-
-template <int NPL, bool QUAD, bool SOFT0>
-__device__ __forceinline__ void p2c_slots(int nq, Lane<NPL> &L, const float4 *src, int cnt, float eps2)
-{
-    if (nq <= 1) eval_p2c<NPL, 1, QUAD, SOFT0>(L, src, cnt, eps2);
-    else if (NPL > 2 && nq == 2) eval_p2c<NPL, (NPL > 2 ? 2 : NPL), QUAD, SOFT0>(L, src, cnt, eps2);
-    else if (NPL > 3 && nq == 3) eval_p2c<NPL, (NPL > 3 ? 3 : NPL), QUAD, SOFT0>(L, src, cnt, eps2);
-    else eval_p2c<NPL, NPL, QUAD, SOFT0>(L, src, cnt, eps2);
-}
-
-// Local expansion coefficients, in the order G0, G1 (x y z), G2 (xx xy xz yy
-// yz zz), G3 (xxx xxy xxz xyy xyz xzz yyy yyz yzz zzz).
-constexpr int kLoc = 20;
-
-// v + (v of another lane chosen by the DPP control CTRL); rows outside RM add 0.
-template <int CTRL, int RM = 0xF>
-__device__ __forceinline__ float dpp_add(float v)
-{
-    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, RM, 0xF, true));
-}
-
-// Sum over the wave, valid in lane 63: quad swaps (xor 1, xor 2), half-row
-// and row mirrors (sums of 8 and 16 lanes), then row 15 -> next row and
-// lane 31 -> rows 2-3 broadcasts.  All VALU, no LDS round trips.
-__device__ __forceinline__ float wave_sum63(float v)
-{
-    v = dpp_add<0xB1>(v);          // quad_perm [1,0,3,2]
-    v = dpp_add<0x4E>(v);          // quad_perm [2,3,0,1]
-    v = dpp_add<0x141>(v);         // row_half_mirror
-    v = dpp_add<0x140>(v);         // row_mirror
-    v = dpp_add<0x142, 0xA>(v);    // row_bcast:15 into rows 1 and 3
-    v = dpp_add<0x143, 0xC>(v);    // row_bcast:31 into rows 2 and 3
-    return v;
-}
-
-// Adds the first cnt far cells of F (c.o.m. relative to the centre, mass) to
-// the group's coefficients row[kLoc]: lane k takes cell k, then the wave sums.
-__device__ __forceinline__ void local_flush(const float4 *F, int cnt, float *row, float eps2, float ell)
-{
-    const int lane = lane_id();
-    const float4 e = lane < cnt ? F[lane] : make_float4(1.f, 0.f, 0.f, 0.f);   // massless: no terms
-    const float rho2 = fmaf(e.x, e.x, fmaf(e.y, e.y, fmaf(e.z, e.z, eps2)));
-    const float ri = rsq(rho2);
-    const float nx = e.x * ri, ny = e.y * ri, nz = e.z * ri;
-    const float F0 = e.w * ri * ri;
-    const float sc = ell * ri;
-    const float Fs = F0 * sc, Fs2 = Fs * sc;
-    const float e3 = 3.f * Fs, t15 = 15.f * Fs2, f3 = 3.f * Fs2;
-    // one coefficient at a time: its wave sum, added by lane 63
-    auto put = [&](int k, float v) {
-        v = wave_sum63(v);
-        if (lane == 63) row[k] += v;
-    };
-    put(0, e.w * ri);
-    put(1, F0 * nx);
-    put(2, F0 * ny);
-    put(3, F0 * nz);
-    put(4, fmaf(e3 * nx, nx, -Fs));
-    put(5, e3 * nx * ny);
-    put(6, e3 * nx * nz);
-    put(7, fmaf(e3 * ny, ny, -Fs));
-    put(8, e3 * ny * nz);
-    put(9, fmaf(e3 * nz, nz, -Fs));
-    put(10, fmaf(t15 * nx, nx * nx, -3.f * f3 * nx));
-    put(11, fmaf(t15 * nx, nx * ny, -f3 * ny));
-    put(12, fmaf(t15 * nx, nx * nz, -f3 * nz));
-    put(13, fmaf(t15 * nx, ny * ny, -f3 * nx));
-    put(14, t15 * nx * (ny * nz));
-    put(15, fmaf(t15 * nx, nz * nz, -f3 * nx));
-    put(16, fmaf(t15 * ny, ny * ny, -3.f * f3 * ny));
-    put(17, fmaf(t15 * ny, ny * nz, -f3 * nz));
-    put(18, fmaf(t15 * ny, nz * nz, -f3 * ny));
-    put(19, fmaf(t15 * nz, nz * nz, -3.f * f3 * nz));
-}
-
-// Field and potential sum (+m/r convention of the tiles) of the summed
-// coefficients G at the member u = (x - centre)/l.
-__device__ __forceinline__ void local_eval(const float *G, float ux, float uy, float uz, float ell, float &ax,
-                                           float &ay, float &az, float &ph)
-{
-    const float gx = fmaf(G[4], ux, fmaf(G[5], uy, G[6] * uz));
-    const float gy = fmaf(G[5], ux, fmaf(G[7], uy, G[8] * uz));
-    const float gz = fmaf(G[6], ux, fmaf(G[8], uy, G[9] * uz));
-    const float xx = ux * ux, yy = uy * uy, zz = uz * uz;
-    const float xy2 = 2.f * ux * uy, xz2 = 2.f * ux * uz, yz2 = 2.f * uy * uz;
-    const float hx = fmaf(G[10], xx, fmaf(G[11], xy2, fmaf(G[12], xz2, fmaf(G[13], yy, fmaf(G[14], yz2, G[15] * zz)))));
-    const float hy = fmaf(G[11], xx, fmaf(G[13], xy2, fmaf(G[14], xz2, fmaf(G[16], yy, fmaf(G[17], yz2, G[18] * zz)))));
-    const float hz = fmaf(G[12], xx, fmaf(G[14], xy2, fmaf(G[15], xz2, fmaf(G[17], yy, fmaf(G[18], yz2, G[19] * zz)))));
-    ax = fmaf(0.5f, hx, G[1] + gx);
-    ay = fmaf(0.5f, hy, G[2] + gy);
-    az = fmaf(0.5f, hz, G[3] + gz);
-    const float px = fmaf(1.f / 6.f, hx, fmaf(0.5f, gx, G[1]));
-    const float py = fmaf(1.f / 6.f, hy, fmaf(0.5f, gy, G[2]));
-    const float pz = fmaf(1.f / 6.f, hz, fmaf(0.5f, gz, G[3]));
-    ph = fmaf(ell, fmaf(ux, px, fmaf(uy, py, uz * pz)), G[0]);
-}
-
-struct WalkArgs {
-    const float4 *thi, *tlo;
-    const int *tself, *tinv;
-    int selfmode;
-    const uint32_t *tperm;
-    int64_t ntest;
-    const unsigned long long *stat;
-    const int *gfirst, *gcount;
-    const float4 *bhi, *blo;
-    const float4 *cA, *cB, *cQ0, *cQ1;
-    const int *sub, *nkids;
-    const int2 *fnb;
-    int nleaf;
-    const uint8_t *level;
-    int nb;
-    const unsigned long long *ncellp;
-    float tolsq, eps2;
-    int *frontier;
-    int fcap;
-    int *gctr;
-    unsigned long long *counters;
-    double *phi, *acc;
-    double4 *sacc;        // lmode 1: (a, phi) per test point in sorted order (the correction pass writes phi, acc)
-    // learned correction: record, per group, the accepted cells whose
-    // size/distance lies in [lr_lo, lr_hi] (squared bounds) into a per-wave
-    // region: [used][g, n, cx, cy, cz, cell ids ...] ...
-    int lmode;            // 0 off, 1 every group, 2 every lstride-th group
-    int lstride;
-    float lr_lo2, lr_hi2;
-    int *lrec;
-    int lcap;
-    // batches: system offsets, per-system (tol^2, eps^2) and walk roots
-    int nsys;
-    const int64_t *boff;
-    const float2 *sysp;
-    const int *sysroot;
-    // treecode1 criteria: root box; cB.w holds each cell's Rcrit2
-    const double4 *box;
-    // super-groups: K consecutive groups share one traversal; per-wave
-    // scratch for the shared lists (shcap entries each)
-    int K;
-    float lalpha2;        // local expansions: local_alpha^2 (0 = off)
-    float4 *shlist;       // [wave][shcap P entries][shcap * S C entries]
-    int *shid;            // [wave][shcap body ids of the P entries][shcap deferred nodes]
-    int shcap;
-};
 
 // CRIT: treecode1's accept (treegrav.c:137-156) for the whole group.  With
 // U the union of the side-s cubes (s = the cell's side, cubes of the cell's
@@ -1251,6 +940,32 @@ void launch(bh_ctx *ctx, WalkArgs &a, int grid, bool crit)
     else k_walk<NPL, QUAD, SOFT0, false, false, false><<<grid, kTpb, 0, ctx->stream>>>(a);
 }
 
+// Who walks a group: one wave (waves 0: k_walk) or a team of waves
+// (k_walk_team), which may take one 64-point row of it (split).  By the groups
+// the points fill at least, e = points / group_size (a third more are cut),
+// against the device's CUs; walk times in us, quadrupole cells in brackets:
+//   one row per 8-wave team while the rows of all groups stay near one per CU
+//     (N = 10^4, groups of 128: 76 [87]; 8 waves per group 86 [111], one wave 391 [450]);
+//   8 waves per group up to 3 groups per CU (N = 5 10^4: 139 [191]; 4 waves
+//     190 [262], a row per team 177 [230], one wave 461 [626]);
+//   4 waves up to 16 per CU (N = 4 10^5: 683 [982]; 8 waves 737 [1013], one
+//     wave 749 [1028]; N = 2^20, groups of 256: 1541; one wave 1671);
+//   then one wave, whose tiles never wait for another's (N = 2^20, groups of
+//     128: 1559 [2090]; 4 waves 1595 [2251]; N = 2^22: 5640 [7070]; 6090 [8740]).
+struct Walkers {
+    int waves;
+    bool split;
+};
+Walkers walkers(const bh_ctx *ctx, const bh_params &p, int64_t nt, int K)
+{
+    if (K > 1) return {0, false};
+    const int64_t e = std::max<int64_t>(nt / p.group_size, ctx->nsys), ncu = ctx->ncu;
+    if (2 * e * (p.group_size / 64) <= 3 * ncu) return {8, p.group_size > 64};
+    if (e <= 3 * ncu) return {8, false};
+    if (e <= 16 * ncu) return {4, false};
+    return {0, false};
+}
+
 }  // namespace
 
 void walk_fast(bh_ctx *ctx, const bh_params &p, int lmode, int lstride)
@@ -1309,11 +1024,9 @@ void walk_fast(bh_ctx *ctx, const bh_params &p, int lmode, int lstride)
     grid = std::max(grid, 1);
     if (ctx->fcap == 0) ctx->fcap = 1 << 15;
     a.fcap = (int)ctx->fcap;
-    a.frontier = ensure<int>(ctx->frontier, (size_t)grid * kWaves * 2 * ctx->fcap);
     // the group counter is a status word cleared at the start of the tree
     // build (every tree build is followed by exactly one fast walk)
     a.gctr = reinterpret_cast<int *>(ptr<unsigned long long>(ctx->counters) + S_GCTR);
-    const int nwave = grid * kWaves;
     // super-groups: the plain walk of a single system with the hackcode1
     // criterion (learned recordings, treecode1 criteria, batches and local
     // expansions walk group by group)
@@ -1323,6 +1036,19 @@ void walk_fast(bh_ctx *ctx, const bh_params &p, int lmode, int lstride)
     a.K = (lmode == 0 && p.criterion == BH_CRIT_HACK && ctx->nsys == 0 && a.lalpha2 == 0.f)
               ? std::max(1, std::min(p.supergroup, kMaxK))
               : 1;
+    const Walkers by = walkers(ctx, p, nt, a.K);
+    a.grows = npl;
+    a.rows = by.split ? 1 : npl;
+    if (by.waves) {
+        // as many teams as are resident: by LDS, and 16 waves per CU (the
+        // kernels' registers)
+        const size_t lds = walk_team_lds(by.waves, p.usequad, a.lalpha2 > 0.f, a.rows);
+        const int64_t percu = std::max<int64_t>(1, std::min<int64_t>((160 << 10) / lds, 16 / by.waves));
+        grid = (int)std::min<int64_t>(nt * (by.split ? npl : 1), ctx->ncu * percu);
+    }
+    // walkers: the waves, or teams, that take groups
+    const int nwave = by.waves ? grid : grid * kWaves;
+    a.frontier = ensure<int>(ctx->frontier, (size_t)nwave * 2 * ctx->fcap);
     if (a.K > 1) {
         const int S = p.usequad ? 3 : 1;
         a.shcap = (int)std::max<int64_t>(ctx->fcap / 4, 1024);
@@ -1345,7 +1071,9 @@ void walk_fast(bh_ctx *ctx, const bh_params &p, int lmode, int lstride)
     if (!ctx->capturing && lmode) BH_HIP(hipEventRecord(ctx->ev[4], ctx->stream));
     const bool crit = p.criterion != BH_CRIT_HACK;
     a.box = T.dbox;
-    if (npl == 3) {
+    if (by.waves) {
+        walk_team(ctx, a, by.waves, grid, p.usequad, soft0, crit);
+    } else if (npl == 3) {
         if (p.usequad) soft0 ? launch<3, true, true>(ctx, a, grid, crit) : launch<3, true, false>(ctx, a, grid, crit);
         else soft0 ? launch<3, false, true>(ctx, a, grid, crit) : launch<3, false, false>(ctx, a, grid, crit);
     } else if (npl == 4) {
