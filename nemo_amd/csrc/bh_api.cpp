@@ -429,7 +429,8 @@ void bh_destroy(bh_ctx *ctx)
                           &ctx->vel,    &ctx->acc_old, &ctx->lfstep, &ctx->diag_partial, &ctx->diag_buf,
                           &ctx->n2b_buf, &ctx->nbc_buf, &ctx->lrec, &ctx->sacc,   &ctx->cF0,    &ctx->cF1,
                           &ctx->mlp.params, &ctx->mlp.wb, &ctx->mlp.bias, &ctx->mlp.gpart, &ctx->mlp.lpart,
-                          &ctx->mlp.adam_m, &ctx->mlp.adam_v, &ctx->mlp.grad, &ctx->mlp.loss, &ctx->mlp.sx,
+                          &ctx->mlp.adam_m, &ctx->mlp.adam_v, &ctx->mlp.loss,
+                          &ctx->mlp.sel, &ctx->mlp.selhist, &ctx->mlp.selpart, &ctx->mlp.sx,
                           &ctx->mlp.sy, &ctx->mlp.snew_x, &ctx->mlp.snew_y, &ctx->mlp.soff, &ctx->mlp.corr,
                           &ctx->mlp.ecell, &ctx->mlp.egrp, &ctx->mlp.gstart, &ctx->mlp.gcnt, &ctx->mlp.gcentre,
                           &ctx->mlp.res, &ctx->mlp.smeta};
@@ -1093,36 +1094,7 @@ bh_status bh_mlp_train(bh_ctx *ctx, int epochs, int batch, float lr, uint64_t se
         if (n < 64) throw ApiFail(BH_ERR_STATE, "too few training samples");
         if (epochs < 1 || batch < 64 || !(lr > 0.f)) throw ApiFail(BH_ERR_ARG, "bad training arguments");
         hipStream_t st = ctx->stream;
-        // output scales of the residual and Jacobian blocks: the rms of the
-        // targets below the block's 99th percentile of |y| on a sample of the
-        // set (a few cells reach bodies close to the group centre, where the
-        // field is far from linear; those targets are also clipped when the
-        // batches are gathered, so they cannot dominate the loss)
-        if (M.adam_step == 0) {
-            const int64_t k = std::min<int64_t>(n, 1 << 20);
-            std::vector<float> h((size_t)bh::kMlpOut * k);
-            BH_HIP(hipMemcpy(h.data(), M.sy.p, h.size() * sizeof(float), hipMemcpyDeviceToHost));
-            for (int blk = 0; blk < 2; blk++) {
-                std::vector<float> a;
-                a.reserve(h.size());
-                for (size_t i = 0; i < h.size(); i++)
-                    if (((int)(i % bh::kMlpOut) >= bh::kMlpOutR) == (blk == 1)) a.push_back(std::fabs(h[i]));
-                const size_t q = (size_t)(0.99 * (double)(a.size() - 1));
-                std::nth_element(a.begin(), a.begin() + q, a.end());
-                const float lim = a[q];
-                double s2 = 0.0;
-                size_t cnt = 0;
-                for (float v : a)
-                    if (v <= lim) {
-                        s2 += (double)v * v;
-                        cnt++;
-                    }
-                M.norm[blk == 0 ? 0 : 3] = (float)std::max(1e-12, std::sqrt(s2 / (double)std::max<size_t>(cnt, 1)));
-            }
-        }
-        float *bx = bh::ensure<float>(M.snew_x, (size_t)batch * bh::kMlpIn);
-        float *by = bh::ensure<float>(M.snew_y, (size_t)batch * bh::kMlpOut);
-        float *grad = bh::ensure<float>(M.grad, bh::kMlpParams);
+        if (M.adam_step == 0) bh::mlp_scales(ctx);
         const int64_t nb = n / batch;
         float *lossb = bh::ensure<float>(M.loss, std::max<int64_t>(nb, 1));
         uint64_t rs = seed * 0x9e3779b97f4a7c15ULL + 7;
@@ -1148,12 +1120,10 @@ bh_status bh_mlp_train(bh_ctx *ctx, int epochs, int batch, float lr, uint64_t se
             while (gcd(a, (uint64_t)n) != 1) a = (a + 2) % (uint64_t)n;
             const uint64_t c = rnd() % (uint64_t)n;
             for (int64_t b = 0; b < nb; b++) {
-                bh::mlp_gather(ctx, a, c, b * batch, batch, bx, by);
-                bh::mlp_grad(ctx, bx, by, batch, grad, lossb + b);
                 const double f = total_steps > 1 ? (double)step / (double)(total_steps - 1) : 0.0;
                 const float lr_t = (float)(lr * (0.1 + 0.45 * (1.0 + std::cos(3.141592653589793 * f))));
                 step++;
-                bh::mlp_adam(ctx, grad, lr_t, ++M.adam_step);
+                bh::mlp_train_step(ctx, a, c, b * batch, batch, lr_t, ++M.adam_step, lossb + b);
             }
             if (epoch_loss) {
                 std::vector<float> lh(std::max<int64_t>(nb, 1));

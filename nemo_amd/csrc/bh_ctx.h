@@ -10,7 +10,7 @@ namespace bh {
 // Learned-correction state: parameters (FP32 master, BF16 MFMA copy, biases),
 // optimiser moments, training samples and the per-group corrections.
 struct Mlp {
-    DevBuf params, wb, bias, gpart, lpart, adam_m, adam_v, grad, loss;
+    DevBuf params, wb, bias, gpart, lpart, adam_m, adam_v, loss, sel, selhist, selpart;
     DevBuf sx, sy, snew_x, snew_y, soff, corr, ecell, egrp, gstart, gcnt, gcentre, res;
     DevBuf smeta;               // per sample of the last collection: cell, group centre (tests)
     int64_t nsamples = 0;
@@ -162,8 +162,8 @@ void mlp_set(bh_ctx *ctx, const float *host_params, const float *norm);
 void mlp_pack(bh_ctx *ctx);
 void mlp_forward(bh_ctx *ctx, const float *d_x, int64_t n, float *d_y);
 void mlp_grad(bh_ctx *ctx, const float *d_x, const float *d_y, int64_t n, float *d_grad, float *d_loss);
-void mlp_adam(bh_ctx *ctx, const float *d_grad, float lr, int step);
-void mlp_gather(bh_ctx *ctx, uint64_t a, uint64_t c, int64_t first, int64_t cnt, float *bx, float *by);
+void mlp_scales(bh_ctx *ctx);
+void mlp_train_step(bh_ctx *ctx, uint64_t a, uint64_t c, int64_t first, int64_t cnt, float lr, int step, float *d_loss);
 void mlp_correct(bh_ctx *ctx, const bh_params &p);
 int64_t mlp_collect(bh_ctx *ctx, const bh_params &p);
 // bh_lf.hip

@@ -72,115 +72,17 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c)
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// A operand of tile (ti, kk) from a row-major bf16 matrix (row stride lda),
-// 16-byte aligned rows: rows ti*16.., columns kk..kk+31.
-__device__ __forceinline__ bf16x8 load_rows(const bf16 *M, int lda, int r0, int k0)
-{
-    const int l = lane_id();
-    return *reinterpret_cast<const bf16x8 *>(M + (r0 + (l & 15)) * lda + k0 + 8 * (l >> 4));
-}
-
-// A operand element-wise: A[i][k] = M[k*ld + i] (transposed access).
-__device__ __forceinline__ bf16x8 load_cols(const bf16 *M, int ld, int r0, int k0)
-{
-    const int l = lane_id();
-    bf16x8 v;
-    const int i = r0 + (l & 15), kb = k0 + 8 * (l >> 4);
-#pragma unroll
-    for (int e = 0; e < 8; e++) v[e] = M[(kb + e) * ld + i];
-    return v;
-}
-
-// Weight offsets inside the BF16 parameter block.
-// W4 is padded to 32 zero rows so that the transposed product in the backward
-// pass (K = 32) stays inside the block.
-constexpr int kW1b = 0, kW2b = kW1b + 64 * 32, kW3b = kW2b + 64 * 64, kW4b = kW3b + 64 * 64, kWbTotal = kW4b + 32 * 64;
-
-struct Acts {
-    bf16 *x;            // [64][32] inputs
-    bf16 *z[3];         // pre-activations of the hidden layers [64][64] (training)
-    bf16 *h[3];         // hidden activations [64][64]; may all alias (inference)
-};
-
-// One hidden layer: out[64][64] = act(in[64][K] W^T + b).  in/out may alias
-// (all reads happen before the writes).  zsave != nullptr keeps Z (bf16).
-template <int K>
-__device__ void layer_hidden(const bf16 *in, const bf16 *W, const float *b, bf16 *out, bf16 *zsave)
-{
-    const int l = lane_id();
-    f32x4 acc[4][4];
-#pragma unroll
-    for (int ti = 0; ti < 4; ti++)
-#pragma unroll
-        for (int tj = 0; tj < 4; tj++) {
-            acc[ti][tj] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kk = 0; kk < K; kk += 32)
-                acc[ti][tj] = mfma(load_rows(in, K, ti * 16, kk), load_rows(W, K, tj * 16, kk), acc[ti][tj]);
-        }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int ti = 0; ti < 4; ti++)
-#pragma unroll
-        for (int tj = 0; tj < 4; tj++) {
-            const int col = tj * 16 + (l & 15);
-            const float bias = b[col];
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int row = ti * 16 + 4 * (l >> 4) + e;
-                const float z = acc[ti][tj][e] + bias;
-                if (zsave) zsave[row * 64 + col] = (bf16)z;
-                out[row * 64 + col] = (bf16)act(z);
-            }
-        }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Output layer: y[64][kMlpOut] (rows in lanes as D fragments) = h W4^T + b4.
-// Returns for lane l the 4 rows 4*(l/16)+e of tile ti in column l%16.
-__device__ void layer_out(const bf16 *h, const bf16 *W4, const float *b4, float y[4][4])
-{
-    const int l = lane_id();
-#pragma unroll
-    for (int ti = 0; ti < 4; ti++) {
-        f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < 64; kk += 32) acc = mfma(load_rows(h, 64, ti * 16, kk), load_rows(W4, 64, 0, kk), acc);
-        const int col = l & 15;
-        const float bias = col < kMlpOut ? b4[col] : 0.f;
-#pragma unroll
-        for (int e = 0; e < 4; e++) y[ti][e] = acc[e] + bias;
-    }
-}
-
-// Forward pass of 64 rows already in a.x; y fragments as in layer_out.
-__device__ void mlp_forward_wave(const Acts &a, const bf16 *Wb, const float *bias, float y[4][4])
-{
-    layer_hidden<32>(a.x, Wb + kW1b, bias + 0, a.h[0], a.z[0]);
-    layer_hidden<64>(a.h[0], Wb + kW2b, bias + 64, a.h[1], a.z[1]);
-    layer_hidden<64>(a.h[1], Wb + kW3b, bias + 128, a.h[2], a.z[2]);
-    layer_out(a.h[2], Wb + kW4b, bias + 192, y);
-}
+// Weight offsets inside the BF16 parameter block: W1[64][32], W2, W3[64][64] and
+// W4[32][64] (rows >= kMlpOut zero), then the transposes that the backward
+// pass reads as operand rows: W2^T, W3^T [in][64] and W4^T [in][32].
+constexpr int kW1b = 0, kW2b = kW1b + 64 * 32, kW3b = kW2b + 64 * 64, kW4b = kW3b + 64 * 64, kW2t = kW4b + 32 * 64,
+              kW3t = kW2t + 64 * 64, kW4t = kW3t + 64 * 64, kWbTotal = kW4t + 64 * 32;
 
 __device__ __forceinline__ void wave_sync_lds()
 {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Stage 64 rows of 12 FP32 features (rows >= nrow are zero) into a.x.
-__device__ void stage_features(const Acts &a, const float *f, int nrow)
-{
-    const int l = lane_id();
-    for (int c = 0; c < 32; c++) {
-        float v = (l < nrow && c < kMlpIn) ? f[(int64_t)l * kMlpIn + c] : 0.f;
-        a.x[l * 32 + c] = (bf16)v;
-    }
-    wave_sync_lds();
 }
 
 // ---- register-resident inference -------------------------------------------------
@@ -315,185 +217,440 @@ __global__ __launch_bounds__(64) void k_mlp_forward(const float *__restrict__ X,
     }
 }
 
-// ---- training: forward + backward, per-wave partial gradients ----------------
+// ---- training: forward + backward, partial gradients per 64 samples ----------
 
-// dW[out][in] += sum_s dZ[s][out] * H[s][in]: A = dZ^T (transposed access of the
-// [64][ldz] dZ block), B = H rows.  Tiles: out 16*ti.., in 16*tj.., K = 64 samples.
-template <int OUT_T, int IN_T>
-__device__ void grad_w(const bf16 *dZ, int ldz, const bf16 *H, int ldh, float *gW, int in_real, int out_real)
+constexpr int kGradWaves = 16;                // waves per 64 samples: a 16 x 16 tile of each 64 x 64 product each
+constexpr int kLd = 72;                       // row stride of the staged matrices (16-byte rows, spread over the banks)
+
+// MFMA operand from a row-major bf16 matrix with 16-byte aligned rows (row
+// stride ld): rows r0.., columns k0..k0+31.
+__device__ __forceinline__ bf16x8 load_rows(const bf16 *M, int ld, int r0, int k0)
 {
     const int l = lane_id();
-#pragma unroll
-    for (int ti = 0; ti < OUT_T; ti++)
-#pragma unroll
-        for (int tj = 0; tj < IN_T; tj++) {
-            f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kk = 0; kk < 64; kk += 32) {
-                bf16x8 av = load_cols(dZ, ldz, ti * 16, kk);
-                bf16x8 bv;
-                const int j = tj * 16 + (l & 15), kb = kk + 8 * (l >> 4);
-#pragma unroll
-                for (int e = 0; e < 8; e++) bv[e] = H[(kb + e) * ldh + j];
-                acc = mfma(av, bv, acc);
-            }
-            const int in = tj * 16 + (l & 15);
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int out = ti * 16 + 4 * (l >> 4) + e;
-                if (out < out_real && in < in_real) gW[out * in_real + in] = acc[e];
-            }
-        }
+    return *reinterpret_cast<const bf16x8 *>(M + (r0 + (l & 15)) * ld + k0 + 8 * (l >> 4));
 }
 
-// dH[s][in] = sum_out dZ[s][out] W[out][in]: A = dZ rows (K = out), B[k=out][j=in]
-// = W[out][in] read element-wise from the BF16 weights (row stride ldw).
-template <int KOUT>
-__device__ void grad_h(const bf16 *dZ, int ldz, const bf16 *W, int ldw, float dH[4][4][4])
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+// The 16 x 16 tile of bf16 values v (lane l: rows 4(l/16)+e of the tile, column
+// l%16) into a row-major and a transposed matrix.
+__device__ __forceinline__ void put_tile(bf16 *M, bf16 *MT, int r0, int c0, bf16x4 v)
 {
-    const int l = lane_id();
+    const int l = lane_id(), row = r0 + 4 * (l >> 4), col = c0 + (l & 15);
 #pragma unroll
-    for (int ti = 0; ti < 4; ti++)
-#pragma unroll
-        for (int tj = 0; tj < 4; tj++) {
-            f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kk = 0; kk < KOUT; kk += 32) {
-                bf16x8 av = load_rows(dZ, ldz, ti * 16, kk);
-                bf16x8 bv;
-                const int j = tj * 16 + (l & 15), kb = kk + 8 * (l >> 4);
-#pragma unroll
-                for (int e = 0; e < 8; e++) bv[e] = W[(kb + e) * ldw + j];
-                acc = mfma(av, bv, acc);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; e++) dH[ti][tj][e] = acc[e];
-        }
+    for (int e = 0; e < 4; e++) M[(row + e) * kLd + col] = v[e];
+    *reinterpret_cast<bf16x4 *>(MT + col * kLd + row) = v;
 }
 
-// Writes dZ = dH * act'(Z) (bf16) into dz[64][64] and db[64] partial sums.
-__device__ void backprop_act(const float dH[4][4][4], const bf16 *Z, bf16 *dz, float *gb)
+// Staged matrices of one block: hidden activations transposed [feature][sample]
+// (B operands of the weight gradients), the error of every layer's
+// pre-activations transposed (A operands), and the current layer row-major (A
+// operands of the next product).
+struct GradLds {
+    bf16 xT[16 * kLd];                        // inputs
+    bf16 hT[3][64 * kLd];
+    bf16 dT[3][64 * kLd];                     // hidden layers 1..3
+    bf16 d4T[16 * kLd];                       // outputs
+    bf16 rows[2][64 * kLd];                   // row-major, alternating
+    float d4[64 * 16];                        // y - target
+};
+
+// The wave's tile of a hidden layer: z = A W^T + b (NK operands of 32 columns);
+// returns bf16 z, stores act(z).
+template <int NK>
+__device__ __forceinline__ bf16x4 grad_layer(const bf16x8 *A, const bf16x8 *Wf, float bias, int r0, int c0, bf16 *rows,
+                                             bf16 *hT)
 {
-    const int l = lane_id();
-    wave_sync_lds();
-    float colsum[4] = {0.f, 0.f, 0.f, 0.f};
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ti = 0; ti < 4; ti++)
+    for (int k = 0; k < NK; k++) acc = mfma(A[k], Wf[k], acc);
+    bf16x4 zs, h;
 #pragma unroll
-        for (int tj = 0; tj < 4; tj++) {
-            const int col = tj * 16 + (l & 15);
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int row = ti * 16 + 4 * (l >> 4) + e;
-                const float g = dH[ti][tj][e] * act_grad((float)Z[row * 64 + col]);
-                const bf16 gb16 = (bf16)g;
-                dz[row * 64 + col] = gb16;
-                colsum[tj] += (float)gb16;
-            }
-        }
-    // column sums over the 64 rows: lanes with the same l%16 hold the same columns
-#pragma unroll
-    for (int tj = 0; tj < 4; tj++) {
-        float v = colsum[tj];
-        v += __shfl_xor(v, 16, 64);
-        v += __shfl_xor(v, 32, 64);
-        if (l < 16) gb[tj * 16 + l] = v;
+    for (int e = 0; e < 4; e++) {
+        const float z = acc[e] + bias;
+        zs[e] = (bf16)z;
+        h[e] = (bf16)act(z);
     }
-    wave_sync_lds();
+    put_tile(rows, hT, r0, c0, h);
+    return zs;
 }
 
-// One wave: 64 samples -> partial gradient (kMlpParams floats, FP32 master
-// layout) and partial loss.  rows >= nrow contribute nothing.
-__global__ __launch_bounds__(64) void k_mlp_grad(const float *__restrict__ X, const float *__restrict__ Yt, int64_t n,
-                                                 float inv_batch, const bf16 *__restrict__ Wb,
-                                                 const float *__restrict__ bias, float *__restrict__ gpart,
-                                                 float *__restrict__ lpart)
+// The wave's tile of a hidden layer's error: dH = dZ W (A = rows of dZ),
+// dZ' = dH act'(z).
+template <int NK>
+__device__ __forceinline__ void grad_back(const bf16x8 *A, const bf16x8 *Wt, bf16x4 zs, int r0, int c0, bf16 *rows,
+                                          bf16 *dT)
 {
-    __shared__ __attribute__((aligned(16))) bf16 sx[64 * 32];
-    __shared__ __attribute__((aligned(16))) bf16 sz[3][64 * 64];
-    __shared__ __attribute__((aligned(16))) bf16 sh[3][64 * 64];
-    __shared__ __attribute__((aligned(16))) bf16 sd[64 * 64];
-    Acts a{sx, {sz[0], sz[1], sz[2]}, {sh[0], sh[1], sh[2]}};
-    const int l = lane_id();
-    const int64_t r0 = (int64_t)blockIdx.x * 64;
-    const int nrow = (int)std::min<int64_t>(64, n - r0);
-    stage_features(a, X + r0 * kMlpIn, nrow);
-    float y[4][4];
-    mlp_forward_wave(a, Wb, bias, y);
-    float *g = gpart + (int64_t)blockIdx.x * kMlpParams;
-    // dY = 2 (y - t) / batch on real rows/columns; kept as bf16 dZ4 [64][64] (cols < kMlpOut)
-    const int col = l & 15;
-    float lsum = 0.f, b4s = 0.f;
-    for (int i = l; i < 64 * 64; i += 64) sd[i] = (bf16)0.f;
-    wave_sync_lds();
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ti = 0; ti < 4; ti++)
+    for (int k = 0; k < NK; k++) acc = mfma(A[k], Wt[k], acc);
+    bf16x4 d;
+#pragma unroll
+    for (int e = 0; e < 4; e++) d[e] = (bf16)(acc[e] * act_grad((float)zs[e]));
+    put_tile(rows, dT, r0, c0, d);
+}
+
+// Weight gradient tile dW[out][in] = sum over the 64 samples of dZ^T H.
+__device__ __forceinline__ void grad_tile(const bf16 *dT, const bf16 *hT, int ti, int tj, float *gW, int in_real,
+                                          int out_real)
+{
+    const int l = lane_id();
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < 64; kk += 32)
+        acc = mfma(load_rows(dT, kLd, ti * 16, kk), load_rows(hT, kLd, tj * 16, kk), acc);
+    const int in = tj * 16 + (l & 15);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int out = ti * 16 + 4 * (l >> 4) + e;
+        if (out < out_real && in < in_real) gW[out * in_real + in] = acc[e];
+    }
+}
+
+// Column sums of dZ over the 64 samples, columns 16 tj.. (rows in the order
+// of a single wave's fragments, then across the lanes).
+__device__ __forceinline__ void grad_bias(const bf16 *dT, int tj, float *gb)
+{
+    const int l = lane_id();
+    float v = 0.f;
+#pragma unroll
+    for (int ti = 0; ti < 4; ti++) {
+        const bf16x4 d = *reinterpret_cast<const bf16x4 *>(dT + (tj * 16 + (l & 15)) * kLd + ti * 16 + 4 * (l >> 4));
+#pragma unroll
+        for (int e = 0; e < 4; e++) v += (float)d[e];
+    }
+    v += __shfl_xor(v, 16, 64);
+    v += __shfl_xor(v, 32, 64);
+    if (l < 16) gb[tj * 16 + l] = v;
+}
+
+// Where a batch's rows come from: rows 0.. of X and Yt, or (n > 0) rows
+// (a (first + i) + c) mod n of the sample set, its targets divided by their
+// block's scale and clipped to +-kClip.
+constexpr float kClip = 10.f;
+struct BatchOf {
+    uint64_t a, c;
+    int64_t first, n;
+    float inv_yscale, inv_jscale;
+};
+
+// (a i + c) mod n.  a i + c < 2^62 and n < 2^31 (a, i, c < n): the quotient from
+// doubles is off by at most one, which the exact remainder shows.
+__device__ __forceinline__ int64_t batch_row(const BatchOf &b, int64_t i)
+{
+    const int64_t x = (int64_t)(b.a * (uint64_t)i + b.c);
+    int64_t r = x - (int64_t)((double)x / (double)b.n) * b.n;
+    if (r < 0) r += b.n;
+    if (r >= b.n) r -= b.n;
+    return r;
+}
+
+// Partial gradient (kMlpParams floats, FP32 master layout) and loss of 64
+// samples; rows >= nrow contribute nothing.  A batch of 8192 has only 128 such
+// blocks (their sums are added in block order, which fixes the size), so a
+// block is bound by the latency of its chain of seven products: sixteen waves
+// share it, one 16 x 16 tile of every product each; the weights' operands are
+// loaded before the inputs arrive, and every operand is one 16-byte load
+// (transposed copies of the activations, the errors and the weights).  One wave
+// per block with element-wise transposed loads took 38.7 us a batch of 8192,
+// four waves with 16 rows each 16.1 us, this 13.7 us (4 of them the launch).
+__global__ __launch_bounds__(64 * kGradWaves) void k_mlp_grad(const float *__restrict__ X, const float *__restrict__ Yt,
+                                                              int64_t count, BatchOf bo, float inv_batch,
+                                                              const bf16 *__restrict__ Wb, const float *__restrict__ bias,
+                                                              float *__restrict__ gpart, float *__restrict__ lpart)
+{
+    __shared__ __attribute__((aligned(16))) GradLds S;
+    const int l = lane_id(), q = l >> 4, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t b0 = (int64_t)blockIdx.x * 64;
+    const int nrow = (int)std::min<int64_t>(64, count - b0);
+    const int r0 = 16 * (w & 3), c0 = 16 * (w >> 2);     // the wave's tile
+    const int col = l & 15;
+    // this lane's sample (row r0 + l%16): its place in the set
+    const bool real = r0 + col < nrow;
+    const int64_t i = b0 + r0 + col;
+    const int64_t src = !real ? 0 : bo.n ? batch_row(bo, bo.first + i) : i;
+    // All loads are issued before the first is waited for, the scattered ones
+    // (the sample's inputs, the targets of this lane's output fragment) first;
+    // waited for one group after the other they took 6 us of 10.
+    const float4 *xr = reinterpret_cast<const float4 *>(X) + src * (kMlpIn / 4);
+    const float4 x0 = xr[q == 1 ? 2 : 0], x1 = xr[1];
+    float t[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int64_t r = __shfl((long long)src, 4 * q + e, 64);
+        t[e] = Yt[r * kMlpOut + min(col, kMlpOut - 1)];
+    }
+    const float bi1 = bias[c0 + col], bi2 = bias[64 + c0 + col], bi3 = bias[128 + c0 + col], bi4 = bias[192 + col];
+    bf16x8 w1[1], w2[2], w3[2], w4[2], w2t[2], w3t[2], w4t[1];
+    w1[0] = load_rows(Wb + kW1b, 32, c0, 0);
+#pragma unroll
+    for (int k = 0; k < 2; k++) w2[k] = load_rows(Wb + kW2b, 64, c0, 32 * k);
+#pragma unroll
+    for (int k = 0; k < 2; k++) w3[k] = load_rows(Wb + kW3b, 64, c0, 32 * k);
+#pragma unroll
+    for (int k = 0; k < 2; k++) w4[k] = load_rows(Wb + kW4b, 64, 0, 32 * k);
+    w4t[0] = load_rows(Wb + kW4t, 32, c0, 0);
+#pragma unroll
+    for (int k = 0; k < 2; k++) w3t[k] = load_rows(Wb + kW3t, 64, c0, 32 * k);
+#pragma unroll
+    for (int k = 0; k < 2; k++) w2t[k] = load_rows(Wb + kW2t, 64, c0, 32 * k);
+    __builtin_amdgcn_sched_barrier(0);
+    // inputs 8 q .. 8 q + 7 of the sample: the first layer's A operand
+    bf16x8 xa[1];
+    {
+        const float f[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+        for (int e = 0; e < 8; e++) xa[0][e] = (bf16)(real && 8 * q + e < kMlpIn ? f[e] : 0.f);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        if (bo.n) t[e] = fminf(fmaxf(t[e] * (col < kMlpOutR ? bo.inv_yscale : bo.inv_jscale), -kClip), kClip);
+    if (c0 == 0 && q < 2)
+#pragma unroll
+        for (int e = 0; e < 8; e++) S.xT[(8 * q + e) * kLd + r0 + col] = xa[0][e];
+
+    // forward
+    bf16x8 A[2];
+    auto operand = [&](const bf16 *rows) {
+        __syncthreads();
+        A[0] = load_rows(rows, kLd, r0, 0);
+        A[1] = load_rows(rows, kLd, r0, 32);
+    };
+    const bf16x4 z1 = grad_layer<1>(xa, w1, bi1, r0, c0, S.rows[0], S.hT[0]);
+    operand(S.rows[0]);
+    const bf16x4 z2 = grad_layer<2>(A, w2, bi2, r0, c0, S.rows[1], S.hT[1]);
+    operand(S.rows[1]);
+    const bf16x4 z3 = grad_layer<2>(A, w3, bi3, r0, c0, S.rows[0], S.hT[2]);
+    operand(S.rows[0]);
+    if (c0 == 0) {
+        f32x4 y = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < 2; k++) y = mfma(A[k], w4[k], y);
+        // dY = 2 (y - t) / batch on the real rows and columns
+        bf16x4 d;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const int row = ti * 16 + 4 * (l >> 4) + e;
-            if (col < kMlpOut && row < nrow) {
-                const float d = y[ti][e] - Yt[(r0 + row) * kMlpOut + col];
-                lsum += d * d;
-                const bf16 gd = (bf16)(2.f * d * inv_batch);
-                sd[row * 64 + col] = gd;
-                b4s += (float)gd;
-            }
+            const int row = r0 + 4 * q + e;
+            const float v = y[e] + bi4 - t[e];
+            S.d4[row * 16 + col] = v;
+            d[e] = col < kMlpOut && row < nrow ? (bf16)(2.f * v * inv_batch) : (bf16)0.f;
+            S.rows[1][row * kLd + 16 + col] = (bf16)0.f;   // columns 16..31 of the operand
         }
-    wave_sync_lds();
-    // loss and db4
-    for (int d = 32; d >= 1; d >>= 1) lsum += __shfl_xor(lsum, d, 64);
-    if (l == 0) lpart[blockIdx.x] = lsum * inv_batch;
-    b4s += __shfl_xor(b4s, 16, 64);
-    b4s += __shfl_xor(b4s, 32, 64);
-    if (l < kMlpOut) g[kOffB4 + l] = b4s;
-    // layer 4 (W4 rows >= kMlpOut are zero, and so are dZ4's columns)
-    grad_w<1, 4>(sd, 64, sh[2], 64, g + kOffW4, 64, kMlpOut);
-    float dH[4][4][4];
-    grad_h<32>(sd, 64, Wb + kW4b, 64, dH);
-    // layer 3
-    backprop_act(dH, sz[2], sd, g + kOffB3);
-    grad_w<4, 4>(sd, 64, sh[1], 64, g + kOffW3, 64, 64);
-    grad_h<64>(sd, 64, Wb + kW3b, 64, dH);
-    // layer 2
-    backprop_act(dH, sz[1], sd, g + kOffB2);
-    grad_w<4, 4>(sd, 64, sh[0], 64, g + kOffW2, 64, 64);
-    grad_h<64>(sd, 64, Wb + kW2b, 64, dH);
-    // layer 1
-    backprop_act(dH, sz[0], sd, g + kOffB1);
-    grad_w<4, 1>(sd, 64, sx, 32, g + kOffW1, kMlpIn, 64);
+        put_tile(S.rows[1], S.d4T, r0, 0, d);
+    }
+    // backward (a buffer is written again two barriers after it was read)
+    operand(S.rows[1]);
+    grad_back<1>(A, w4t, z3, r0, c0, S.rows[0], S.dT[2]);
+    operand(S.rows[0]);
+    grad_back<2>(A, w3t, z2, r0, c0, S.rows[1], S.dT[1]);
+    operand(S.rows[1]);
+    grad_back<2>(A, w2t, z1, r0, c0, S.rows[0], S.dT[0]);
+    __syncthreads();
+
+    // weight gradients: a tile of W3 and of W2 per wave, W4 and W1 on the
+    // first eight; biases and loss on the others
+    float *g = gpart + (int64_t)blockIdx.x * kMlpParams;
+    const int ti = w & 3, tj = w >> 2;
+    grad_tile(S.dT[2], S.hT[1], ti, tj, g + kOffW3, 64, 64);
+    grad_tile(S.dT[1], S.hT[0], ti, tj, g + kOffW2, 64, 64);
+    if (tj == 0) {
+        grad_tile(S.d4T, S.hT[2], 0, ti, g + kOffW4, 64, kMlpOut);
+    } else if (tj == 1) {
+        grad_tile(S.dT[0], S.xT, ti, 0, g + kOffW1, kMlpIn, 64);
+    } else if (tj == 2) {
+        grad_bias(S.dT[2], ti, g + kOffB3);
+        grad_bias(S.dT[1], ti, g + kOffB2);
+    } else {
+        grad_bias(S.dT[0], ti, g + kOffB1);
+    }
+    if (w == 15) {
+        // loss and output biases, in the order of the fragments of all rows
+        float lsum = 0.f, b4s = 0.f;
+#pragma unroll
+        for (int tr = 0; tr < 4; tr++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int row = tr * 16 + 4 * q + e;
+                if (col < kMlpOut && row < nrow) {
+                    const float d = S.d4[row * 16 + col];
+                    lsum += d * d;
+                    b4s += (float)S.d4T[col * kLd + row];
+                }
+            }
+        for (int d = 32; d >= 1; d >>= 1) lsum += __shfl_xor(lsum, d, 64);
+        if (l == 0) lpart[blockIdx.x] = lsum * inv_batch;
+        b4s += __shfl_xor(b4s, 16, 64);
+        b4s += __shfl_xor(b4s, 32, 64);
+        if (l < kMlpOut) g[kOffB4 + l] = b4s;
+    }
 }
 
-// Sum of the per-wave partial gradients in wave order (deterministic).
-__global__ void k_mlp_reduce(const float *__restrict__ gpart, int nw, float *__restrict__ grad, const float *lpart,
-                             float *loss)
+// Sum of a column of the partial gradients in block order (deterministic), the
+// loads of kSumRun blocks in flight.
+constexpr int kSumRun = 32;
+__device__ __forceinline__ float sum_parts(const float *__restrict__ v, int64_t stride, int n)
 {
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < kMlpParams) {
-        float s = 0.f;
-        for (int w = 0; w < nw; w++) s += gpart[(int64_t)w * kMlpParams + p];
-        grad[p] = s;
+    float s = 0.f;
+    int w = 0;
+    for (; w + kSumRun <= n; w += kSumRun) {
+        float x[kSumRun];
+#pragma unroll
+        for (int k = 0; k < kSumRun; k++) x[k] = v[(w + k) * stride];
+#pragma unroll
+        for (int k = 0; k < kSumRun; k++) s += x[k];
     }
-    if (p == 0) {
-        float s = 0.f;
-        for (int w = 0; w < nw; w++) s += lpart[w];
-        *loss = s;
+    for (; w < n; w++) s += v[w * stride];
+    return s;
+}
+
+__global__ __launch_bounds__(64) void k_mlp_reduce(const float *__restrict__ gpart, int nw, float *__restrict__ grad,
+                                                   const float *lpart, float *loss)
+{
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < kMlpParams) grad[p] = sum_parts(gpart + p, kMlpParams, nw);
+    if (p == kMlpParams) *loss = sum_parts(lpart, 1, nw);
+}
+
+// ---- output scales of a training set --------------------------------------
+// Per block of outputs (residual, Jacobian): the value of a given rank among
+// |y| by three histogram passes over the bits of the floats (11, 11 and 10
+// bits; non-negative floats order as their bits), then the count and the FP64
+// sum of squares of the values up to it.  (On the host, a copy of the targets
+// and a partial sort of each block took 9 ms of every training call.)
+constexpr int kSelBins = 2048;
+struct ScaleSel {
+    unsigned prefix[2];              // bits fixed so far
+    unsigned pad[2];
+    unsigned long long rank[2];      // rank among the values with that prefix
+    double sum[2], cnt[2];
+};
+__device__ __forceinline__ int sel_shift(int pass) { return pass == 0 ? 21 : pass == 1 ? 10 : 0; }
+
+__global__ __launch_bounds__(256) void k_sel_hist(const float *__restrict__ Y, int64_t nval, int pass,
+                                                  const ScaleSel *__restrict__ sel, unsigned *hist)
+{
+    __shared__ unsigned h[2 * kSelBins];
+    for (int b = threadIdx.x; b < 2 * kSelBins; b += blockDim.x) h[b] = 0;
+    __syncthreads();
+    const int shift = sel_shift(pass), bits = pass == 2 ? 10 : 11;
+    const unsigned p0 = sel->prefix[0], p1 = sel->prefix[1];
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nval; i += (int64_t)gridDim.x * blockDim.x) {
+        const unsigned u = __float_as_uint(fabsf(Y[i]));
+        const int blk = (int)(i % kMlpOut) >= kMlpOutR;
+        if (pass == 0 || (u >> (shift + bits)) == (blk ? p1 : p0))
+            atomicAdd(&h[blk * kSelBins + ((u >> shift) & ((1u << bits) - 1))], 1u);
+    }
+    __syncthreads();
+    for (int b = threadIdx.x; b < 2 * kSelBins; b += blockDim.x)
+        if (h[b]) atomicAdd(&hist[b], h[b]);
+}
+
+// The bin holding the rank, one wave per block of outputs; clears the bins.
+__global__ __launch_bounds__(128) void k_sel_pick(int pass, ScaleSel *sel, unsigned *hist)
+{
+    const int blk = threadIdx.x >> 6, l = lane_id(), bits = pass == 2 ? 10 : 11, nbin = 1 << bits;
+    unsigned *h = hist + blk * kSelBins;
+    const unsigned long long rank = sel->rank[blk];
+    unsigned long long run = 0;
+    for (int b0 = 0; b0 < nbin; b0 += 64) {
+        const unsigned v = h[b0 + l];
+        h[b0 + l] = 0;
+        unsigned x = v;
+        for (int d = 1; d < 64; d <<= 1) {
+            const unsigned t = __shfl_up(x, d, 64);
+            if (l >= d) x += t;
+        }
+        const unsigned long long hi = run + x, lo = hi - v;
+        if (rank >= lo && rank < hi) {
+            sel->prefix[blk] = (sel->prefix[blk] << bits) | (unsigned)(b0 + l);
+            sel->rank[blk] = rank - lo;
+        }
+        run += __shfl(x, 63, 64);
     }
 }
 
-// Adam step on the FP32 master parameters, then refresh the BF16 copies.
-__global__ void k_adam(float *__restrict__ P, const float *__restrict__ G, float *__restrict__ m, float *__restrict__ v,
-                       float lr, float b1, float b2, float eps, float c1, float c2)
+constexpr int kSelBlocks = 256;
+__global__ __launch_bounds__(256) void k_sel_sum(const float *__restrict__ Y, int64_t nval, const ScaleSel *__restrict__ sel,
+                                                 double *part)
 {
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ double red[4][256];
+    double s[4] = {0.0, 0.0, 0.0, 0.0};   // sum, count of block 0, then of block 1
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nval; i += (int64_t)gridDim.x * blockDim.x) {
+        const float y = fabsf(Y[i]);
+        const int blk = (int)(i % kMlpOut) >= kMlpOutR;
+        if (__float_as_uint(y) <= sel->prefix[blk]) {
+            s[2 * blk] += (double)y * y;
+            s[2 * blk + 1] += 1.0;
+        }
+    }
+    for (int k = 0; k < 4; k++) red[k][threadIdx.x] = s[k];
+    __syncthreads();
+    for (int h = 128; h > 0; h >>= 1) {
+        if ((int)threadIdx.x < h)
+            for (int k = 0; k < 4; k++) red[k][threadIdx.x] += red[k][threadIdx.x + h];
+        __syncthreads();
+    }
+    if (threadIdx.x < 4) part[4 * blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
+}
+__global__ void k_sel_final(const double *part, int n, ScaleSel *sel)
+{
+    const int k = threadIdx.x;
+    if (k >= 4) return;
+    double s = 0.0;
+    for (int b = 0; b < n; b++) s += part[4 * b + k];
+    (k & 1 ? sel->cnt : sel->sum)[k >> 1] = s;
+}
+
+// The BF16 copies and the bias block's entry of parameter p (value v).
+__device__ __forceinline__ void pack_param(int p, float v, bf16 *Wb, float *bias)
+{
+    const bf16 b = (bf16)v;
+    if (p < kOffB1) {
+        Wb[kW1b + (p / kMlpIn) * 32 + p % kMlpIn] = b;
+    } else if (p < kOffW2) {
+        bias[p - kOffB1] = v;
+    } else if (p < kOffB2) {
+        const int k = p - kOffW2;
+        Wb[kW2b + k] = b;
+        Wb[kW2t + (k & 63) * 64 + (k >> 6)] = b;
+    } else if (p < kOffW3) {
+        bias[64 + p - kOffB2] = v;
+    } else if (p < kOffB3) {
+        const int k = p - kOffW3;
+        Wb[kW3b + k] = b;
+        Wb[kW3t + (k & 63) * 64 + (k >> 6)] = b;
+    } else if (p < kOffW4) {
+        bias[128 + p - kOffB3] = v;
+    } else if (p < kOffB4) {
+        const int k = p - kOffW4;
+        Wb[kW4b + k] = b;
+        Wb[kW4t + (k & 63) * 32 + (k >> 6)] = b;
+    } else {
+        bias[192 + p - kOffB4] = v;
+    }
+}
+
+// The rest of a training step in one launch: the reduction, the Adam step on
+// the FP32 master parameters and the refresh of the BF16 copies.  One wave per
+// 64 parameters over the whole device (the reduction alone, in 39 blocks with
+// one load in flight per thread, took 35 us).
+__global__ __launch_bounds__(64) void k_mlp_step(const float *__restrict__ gpart, int nw, const float *lpart, float *loss,
+                                                 float *__restrict__ P, float *__restrict__ m, float *__restrict__ v,
+                                                 float lr, float b1, float b2, float eps, float c1, float c2, bf16 *Wb,
+                                                 float *bias)
+{
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p == kMlpParams) *loss = sum_parts(lpart, 1, nw);
     if (p >= kMlpParams) return;
-    float g = G[p];
+    const float g = sum_parts(gpart + p, kMlpParams, nw);
     float mm = b1 * m[p] + (1.f - b1) * g;
     float vv = b2 * v[p] + (1.f - b2) * g * g;
     m[p] = mm;
     v[p] = vv;
-    P[p] -= lr * (mm / c1) / (sqrtf(vv / c2) + eps);
+    const float np = P[p] - lr * (mm / c1) / (sqrtf(vv / c2) + eps);
+    P[p] = np;
+    pack_param(p, np, Wb, bias);
 }
-
 
 // ---- features and the learned correction of the walk ---------------------------
 
@@ -811,6 +968,10 @@ __global__ void k_region_cells(const int *__restrict__ lrec, int lcap, int nreg,
     cnt[r] = c;
 }
 
+// Waves per record region in the kernels below (a team's walk leaves few,
+// longer regions).
+constexpr int kRecWaves = 8;
+
 // Exact residual (a_exact - a_multipole) of cell c at point t, FP64; the wave
 // shares the direct sum over the cell's bodies; valid in lane 0.
 __device__ void exact_residual(int c, double tx, double ty, double tz, const int2 *__restrict__ fnb,
@@ -859,14 +1020,19 @@ __device__ void exact_residual(int c, double tx, double ty, double tz, const int
 
 // Diagnostic: the correction a perfect model would give (exact residual at the
 // group centre for every recorded cell).
-__global__ __launch_bounds__(64) void k_exact_corr(const int *__restrict__ lrec, int lcap, const int2 *__restrict__ fnb,
+__global__ __launch_bounds__(64 * kRecWaves) void k_exact_corr(const int *__restrict__ lrec, int lcap, const int2 *__restrict__ fnb,
                                                    const double *__restrict__ mo, const double4 *__restrict__ bd,
                                                    double eps, int usequad, float4 *corr)
 {
     const int *reg = lrec + (int64_t)blockIdx.x * lcap;
     const int used = reg[0];
-    for (int p = 1; p < used;) {
+    const int w = threadIdx.x >> 6;   // record r goes to wave r mod kRecWaves
+    for (int p = 1, r = 0; p < used; r++) {
         const int g = reg[p], n = reg[p + 1];
+        if (r % kRecWaves != w) {
+            p += 5 + n;
+            continue;
+        }
         const double tx = __int_as_float(reg[p + 2]), ty = __int_as_float(reg[p + 3]), tz = __int_as_float(reg[p + 4]);
         double ax = 0.0, ay = 0.0, az = 0.0;
         for (int k = 0; k < n; k++) {
@@ -961,15 +1127,20 @@ __device__ void residual_field(int c, double tx, double ty, double tz, const int
 // field would give: per group the sums of the exact residuals and of their
 // Jacobians at the group centre over the recorded cells (12 floats: R, J row
 // major), and the centre.
-__global__ __launch_bounds__(64) void k_exact_corr1(const int *__restrict__ lrec, int lcap,
+__global__ __launch_bounds__(64 * kRecWaves) void k_exact_corr1(const int *__restrict__ lrec, int lcap,
                                                     const int2 *__restrict__ fnb, const double *__restrict__ mo,
                                                     const double4 *__restrict__ bd, double eps, int usequad,
                                                     float4 *corr)
 {
     const int *reg = lrec + (int64_t)blockIdx.x * lcap;
     const int used = reg[0];
-    for (int p = 1; p < used;) {
+    const int w = threadIdx.x >> 6;   // record r goes to wave r mod kRecWaves
+    for (int p = 1, r = 0; p < used; r++) {
         const int g = reg[p], n = reg[p + 1];
+        if (r % kRecWaves != w) {
+            p += 5 + n;
+            continue;
+        }
         const float cx = __int_as_float(reg[p + 2]), cy = __int_as_float(reg[p + 3]), cz = __int_as_float(reg[p + 4]);
         double s[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         for (int k = 0; k < n; k++) {
@@ -1020,8 +1191,9 @@ __global__ void k_apply_corr1(const int *__restrict__ gfirst, const int *__restr
 // the FP64 multipole force of the walk's formula) in units of M / r^2, and
 // its Jacobian in units of M / r^3.
 // Group g's samples go to goff[g] onwards, so the set is in group order
-// whichever wave walked which group (training is then reproducible).
-__global__ __launch_bounds__(64) void k_samples(const int *__restrict__ lrec, int lcap, const uint32_t *__restrict__ goff,
+// whichever wave walked which group (training is then reproducible).  One block
+// per record region, a wave per sample in turn.
+__global__ __launch_bounds__(64 * kRecWaves) void k_samples(const int *__restrict__ lrec, int lcap, const uint32_t *__restrict__ goff,
                                                 int ng,
                                                 const float4 *__restrict__ cA, const float4 *__restrict__ cB,
                                                 const float4 *__restrict__ cF0, const float4 *__restrict__ cF1,
@@ -1040,9 +1212,10 @@ __global__ __launch_bounds__(64) void k_samples(const int *__restrict__ lrec, in
             p += 5 + n;
             continue;
         }
-        int64_t j = goff[reg[p]];
+        const int64_t j0 = goff[reg[p]];
         const float cx = __int_as_float(reg[p + 2]), cy = __int_as_float(reg[p + 3]), cz = __int_as_float(reg[p + 4]);
-        for (int k = 0; k < n; k++, j++) {
+        for (int k = threadIdx.x >> 6; k < n; k += kRecWaves) {
+            const int64_t j = j0 + k;
             const int c = reg[p + 5 + k];
             double r[3], J[9];
             residual_field(c, cx, cy, cz, fnb, mo, bd, e2, usequad, r, J);
@@ -1075,47 +1248,19 @@ __global__ __launch_bounds__(64) void k_samples(const int *__restrict__ lrec, in
 
 }  // namespace
 
-// Training batch b of an epoch: rows (a*i + c) mod n (a coprime with n), targets
-// divided by their block's scale and clipped to +-kClip.
-constexpr float kClip = 10.f;
-__global__ void k_gather_batch(const float *__restrict__ X, const float *__restrict__ Y, int64_t n, uint64_t a,
-                               uint64_t c, int64_t first, int64_t cnt, float inv_yscale, float inv_jscale, float *bx,
-                               float *by)
+// Converts the FP32 master parameters to the padded BF16 MFMA layouts (the
+// padding stays zero from then on) and the FP32 bias block (b1 | b2 | b3 | b4
+// padded to 16).
+__global__ void k_mlp_zero(bf16 *__restrict__ Wb, float *__restrict__ bias)
 {
-    int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= cnt) return;
-    const uint64_t r = (uint64_t)((a * (uint64_t)(first + i) + c) % (uint64_t)n);
-    for (int k = 0; k < kMlpIn; k++) bx[i * kMlpIn + k] = X[r * kMlpIn + k];
-    for (int k = 0; k < kMlpOut; k++)
-        by[i * kMlpOut + k] = fminf(fmaxf(Y[r * kMlpOut + k] * (k < kMlpOutR ? inv_yscale : inv_jscale), -kClip), kClip);
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < kWbTotal) Wb[t] = (bf16)0.f;
+    if (t < 208) bias[t] = 0.f;
 }
-
-// Converts the FP32 master parameters to the padded BF16 MFMA layout and the
-// FP32 bias block (b1 | b2 | b3 | b4 padded to 16).
 __global__ void k_mlp_pack(const float *__restrict__ P, bf16 *__restrict__ Wb, float *__restrict__ bias)
 {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < kWbTotal) {
-        float v = 0.f;
-        if (t < kW2b) {
-            int o = t / 32, i = t % 32;
-            v = i < kMlpIn ? P[kOffW1 + o * kMlpIn + i] : 0.f;
-        } else if (t < kW3b) {
-            v = P[kOffW2 + (t - kW2b)];
-        } else if (t < kW4b) {
-            v = P[kOffW3 + (t - kW3b)];
-        } else {
-            int o = (t - kW4b) / 64, i = (t - kW4b) % 64;
-            v = o < kMlpOut ? P[kOffW4 + o * 64 + i] : 0.f;
-        }
-        Wb[t] = (bf16)v;
-    }
-    if (t < 64) {
-        bias[t] = P[kOffB1 + t];
-        bias[64 + t] = P[kOffB2 + t];
-        bias[128 + t] = P[kOffB3 + t];
-    }
-    if (t < 16) bias[192 + t] = t < kMlpOut ? P[kOffB4 + t] : 0.f;
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < kMlpParams) pack_param(p, P[p], Wb, bias);
 }
 
 // ---- host side ---------------------------------------------------------------
@@ -1123,7 +1268,8 @@ __global__ void k_mlp_pack(const float *__restrict__ P, bf16 *__restrict__ Wb, f
 void mlp_pack(bh_ctx *ctx)
 {
     Mlp &M = ctx->mlp;
-    k_mlp_pack<<<(kWbTotal + 255) / 256, 256, 0, ctx->stream>>>(ptr<float>(M.params), ptr<bf16>(M.wb), ptr<float>(M.bias));
+    k_mlp_zero<<<(kWbTotal + 255) / 256, 256, 0, ctx->stream>>>(ptr<bf16>(M.wb), ptr<float>(M.bias));
+    k_mlp_pack<<<(kMlpParams + 255) / 256, 256, 0, ctx->stream>>>(ptr<float>(M.params), ptr<bf16>(M.wb), ptr<float>(M.bias));
     BH_HIP(hipGetLastError());
 }
 
@@ -1159,7 +1305,7 @@ void mlp_correct(bh_ctx *ctx, const bh_params &p)
     if (exact1) {
         float4 *corr = ensure<float4>(M.corr, 4 * ngcap);
         k_zero_f4<<<(int)((4 * ngcap + 255) / 256), 256, 0, st>>>(corr, (int)(4 * ngcap));
-        k_exact_corr1<<<ctx->lnwave, 64, 0, st>>>(ptr<int>(ctx->lrec), (int)ctx->lcap, T.fnb, T.mo, T.bd, p.eps,
+        k_exact_corr1<<<ctx->lnwave, 64 * kRecWaves, 0, st>>>(ptr<int>(ctx->lrec), (int)ctx->lcap, T.fnb, T.mo, T.bd, p.eps,
                                                   p.usequad, corr);
         k_apply_corr1<<<gridg, 64, 0, st>>>(ptr<int>(ctx->gfirst), ptr<int>(ctx->gcount), stat, T.tperm, T.thi, T.tlo,
                                             corr, ptr<double4>(ctx->sacc), ptr<double>(ctx->phi),
@@ -1167,7 +1313,7 @@ void mlp_correct(bh_ctx *ctx, const bh_params &p)
     } else if (exact) {
         float4 *corr = ensure<float4>(M.corr, ngcap);
         k_zero_f4<<<(int)((ngcap + 255) / 256), 256, 0, st>>>(corr, (int)ngcap);
-        k_exact_corr<<<ctx->lnwave, 64, 0, st>>>(ptr<int>(ctx->lrec), (int)ctx->lcap, T.fnb, T.mo, T.bd, p.eps,
+        k_exact_corr<<<ctx->lnwave, 64 * kRecWaves, 0, st>>>(ptr<int>(ctx->lrec), (int)ctx->lcap, T.fnb, T.mo, T.bd, p.eps,
                                                  p.usequad, corr);
         k_apply_corr<<<gridg, 64, 0, st>>>(ptr<int>(ctx->gfirst), ptr<int>(ctx->gcount), stat, T.tperm, corr,
                                            ptr<double4>(ctx->sacc), ptr<double>(ctx->phi), ptr<double>(ctx->acc));
@@ -1220,7 +1366,7 @@ int64_t mlp_collect(bh_ctx *ctx, const bh_params &p)
     if (total == 0) return 0;
     float *nx = ensure<float>(M.snew_x, (size_t)total * kMlpIn), *ny = ensure<float>(M.snew_y, (size_t)total * kMlpOut);
     float4 *meta = ensure<float4>(M.smeta, total);
-    k_samples<<<nreg, 64, 0, st>>>(ptr<int>(ctx->lrec), (int)ctx->lcap, goff, ng, T.cA, T.cB, T.cF0, T.cF1, T.fnb, T.mo,
+    k_samples<<<nreg, 64 * kRecWaves, 0, st>>>(ptr<int>(ctx->lrec), (int)ctx->lcap, goff, ng, T.cA, T.cB, T.cF0, T.cF1, T.fnb, T.mo,
                                    T.bd, p.eps, p.usequad, nx, ny, meta);
     M.nlast = total;
     BH_HIP(hipGetLastError());
@@ -1253,30 +1399,63 @@ void mlp_forward(bh_ctx *ctx, const float *d_x, int64_t n, float *d_y)
     BH_HIP(hipGetLastError());
 }
 
-// Gradient of the mean squared error over the batch (x, y) at the current
-// parameters: grad[kMlpParams], loss.
-void mlp_grad(bh_ctx *ctx, const float *d_x, const float *d_y, int64_t n, float *d_grad, float *d_loss)
+// Partial gradients and losses of a batch of n rows (M.gpart, M.lpart);
+// returns their number.
+static int grad_parts(bh_ctx *ctx, const float *d_x, const float *d_y, int64_t n, const BatchOf &bo)
 {
     Mlp &M = ctx->mlp;
     const int nw = (int)((n + 63) / 64);
     float *gpart = ensure<float>(M.gpart, (size_t)nw * kMlpParams);
     float *lpart = ensure<float>(M.lpart, nw);
-    k_mlp_grad<<<nw, 64, 0, ctx->stream>>>(d_x, d_y, n, 1.f / (float)n, ptr<bf16>(M.wb), ptr<float>(M.bias), gpart,
-                                           lpart);
-    k_mlp_reduce<<<(kMlpParams + 255) / 256, 256, 0, ctx->stream>>>(gpart, nw, d_grad, lpart, d_loss);
-    BH_HIP(hipGetLastError());
+    k_mlp_grad<<<nw, 64 * kGradWaves, 0, ctx->stream>>>(d_x, d_y, n, bo, 1.f / (float)n, ptr<bf16>(M.wb),
+                                                        ptr<float>(M.bias), gpart, lpart);
+    return nw;
 }
 
-void mlp_gather(bh_ctx *ctx, uint64_t a, uint64_t c, int64_t first, int64_t cnt, float *bx, float *by)
+// Gradient of the mean squared error over the batch (x, y) at the current
+// parameters: grad[kMlpParams], loss.
+void mlp_grad(bh_ctx *ctx, const float *d_x, const float *d_y, int64_t n, float *d_grad, float *d_loss)
 {
     Mlp &M = ctx->mlp;
-    k_gather_batch<<<(int)((cnt + 255) / 256), 256, 0, ctx->stream>>>(ptr<float>(M.sx), ptr<float>(M.sy), M.nsamples, a, c,
-                                                                    first, cnt, 1.f / M.norm[0], 1.f / M.norm[3], bx,
-                                                                    by);
+    const int nw = grad_parts(ctx, d_x, d_y, n, BatchOf{});
+    k_mlp_reduce<<<kMlpParams / 64 + 1, 64, 0, ctx->stream>>>(ptr<float>(M.gpart), nw, d_grad, ptr<float>(M.lpart), d_loss);
     BH_HIP(hipGetLastError());
 }
 
-void mlp_adam(bh_ctx *ctx, const float *d_grad, float lr, int step)
+// Output scales of the residual and Jacobian blocks (M.norm): the rms of the
+// targets below the block's 99th percentile of |y| on the first 2^20 samples
+// (a few cells reach bodies close to the group centre, where the field is far
+// from linear; those targets are also clipped when the batches are gathered,
+// so they cannot dominate the loss).
+void mlp_scales(bh_ctx *ctx)
+{
+    Mlp &M = ctx->mlp;
+    hipStream_t st = ctx->stream;
+    const int64_t k = std::min<int64_t>(M.nsamples, 1 << 20), nval = kMlpOut * k;
+    const int64_t size[2] = {kMlpOutR * k, (kMlpOut - kMlpOutR) * k};
+    ScaleSel h{};
+    for (int b = 0; b < 2; b++) h.rank[b] = (unsigned long long)(0.99 * (double)(size[b] - 1));
+    ScaleSel *sel = ensure<ScaleSel>(M.sel, 1);
+    unsigned *hist = ensure<unsigned>(M.selhist, 2 * kSelBins);
+    double *part = ensure<double>(M.selpart, 4 * kSelBlocks);
+    BH_HIP(hipMemcpyAsync(sel, &h, sizeof h, hipMemcpyHostToDevice, st));
+    BH_HIP(hipMemsetAsync(hist, 0, 2 * kSelBins * sizeof(unsigned), st));
+    for (int pass = 0; pass < 3; pass++) {
+        k_sel_hist<<<kSelBlocks, 256, 0, st>>>(ptr<float>(M.sy), nval, pass, sel, hist);
+        k_sel_pick<<<1, 128, 0, st>>>(pass, sel, hist);
+    }
+    k_sel_sum<<<kSelBlocks, 256, 0, st>>>(ptr<float>(M.sy), nval, sel, part);
+    k_sel_final<<<1, 64, 0, st>>>(part, kSelBlocks, sel);
+    BH_HIP(hipGetLastError());
+    BH_HIP(hipMemcpyAsync(&h, sel, sizeof h, hipMemcpyDeviceToHost, st));
+    BH_HIP(hipStreamSynchronize(st));
+    for (int b = 0; b < 2; b++)
+        M.norm[b == 0 ? 0 : 3] = (float)std::max(1e-12, std::sqrt(h.sum[b] / std::max(h.cnt[b], 1.0)));
+}
+
+// One training step on rows (a (first + i) + c) mod nsamples, i < cnt, of the
+// sample set; its loss goes to d_loss.
+void mlp_train_step(bh_ctx *ctx, uint64_t a, uint64_t c, int64_t first, int64_t cnt, float lr, int step, float *d_loss)
 {
     Mlp &M = ctx->mlp;
     float *m = ensure<float>(M.adam_m, kMlpParams), *v = ensure<float>(M.adam_v, kMlpParams);
@@ -1284,11 +1463,13 @@ void mlp_adam(bh_ctx *ctx, const float *d_grad, float lr, int step)
         BH_HIP(hipMemsetAsync(m, 0, kMlpParams * sizeof(float), ctx->stream));
         BH_HIP(hipMemsetAsync(v, 0, kMlpParams * sizeof(float), ctx->stream));
     }
+    const int nw = grad_parts(ctx, ptr<float>(M.sx), ptr<float>(M.sy), cnt,
+                              BatchOf{a, c, first, M.nsamples, 1.f / M.norm[0], 1.f / M.norm[3]});
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
-    k_adam<<<(kMlpParams + 255) / 256, 256, 0, ctx->stream>>>(ptr<float>(M.params), d_grad, m, v, lr, b1, b2, 1e-8f, c1,
-                                                              c2);
-    mlp_pack(ctx);
+    k_mlp_step<<<kMlpParams / 64 + 1, 64, 0, ctx->stream>>>(ptr<float>(M.gpart), nw, ptr<float>(M.lpart), d_loss,
+                                                            ptr<float>(M.params), m, v, lr, b1, b2, 1e-8f, c1, c2,
+                                                            ptr<bf16>(M.wb), ptr<float>(M.bias));
     BH_HIP(hipGetLastError());
 }
 
