@@ -475,31 +475,40 @@ __global__ void k_scan_down(const uint32_t *in, uint32_t *out, int64_t n, const 
 
 // ---- radix sort (LSD, 8-bit digits, stable) -----------------------------------
 
-constexpr int kSortItems = 8;
-static_assert(kTpb == 256, "the radix kernels use one thread per 8-bit digit");
-constexpr int kSortTile = kTpb * kSortItems;
+constexpr int kSortTpb = 512, kSortWaves = kSortTpb / 64, kSortItems = 8;
+constexpr int kSortTile = kSortTpb * kSortItems;
+// Up to this many tiles a scatter block adds up the tiles' digit counts itself
+// (block-major histogram); beyond, k_hist_rows scans them (digit-major).  The
+// eight passes: 107 us at the line (131072 keys), 133 us with k_hist_rows at
+// 200000; the launches bound both.
+constexpr int kSortFewTiles = 32;
 
-// One sub-histogram per wave (skewed digits, e.g. the top byte of clustered
-// keys, would otherwise serialise the block on a few LDS counters).
-__global__ __launch_bounds__(kTpb) void k_radix_hist(const uint64_t *__restrict__ keys, int64_t n, int shift,
-                                                     uint32_t *hist, int nblk)
+// Digit counts of one tile, a sub-histogram per wave (skewed digits, e.g. the
+// top byte of clustered keys, would otherwise serialise the block on a few LDS
+// counters).
+__global__ __launch_bounds__(kSortTpb) void k_radix_hist(const uint64_t *__restrict__ keys, int64_t n, int shift,
+                                                         uint32_t *hist, int nblk)
 {
-    __shared__ uint32_t h[kTpb / 64][256];
+    __shared__ uint32_t h[kSortWaves][256];
+    for (int k = threadIdx.x; k < kSortWaves * 256; k += kSortTpb) (&h[0][0])[k] = 0;
+    uint64_t key[kSortItems];
+    const int64_t base = (int64_t)blockIdx.x * kSortTile + threadIdx.x;
 #pragma unroll
-    for (int w = 0; w < kTpb / 64; w++) h[w][threadIdx.x] = 0;
+    for (int r = 0; r < kSortItems; r++) key[r] = base + r * kSortTpb < n ? keys[base + r * kSortTpb] : 0;
     __syncthreads();
     uint32_t *hw = h[threadIdx.x >> 6];
-    const int64_t base = (int64_t)blockIdx.x * kSortTile;
 #pragma unroll
-    for (int r = 0; r < kSortItems; r++) {
-        int64_t i = base + (int64_t)r * kTpb + threadIdx.x;
-        if (i < n) atomicAdd(&hw[(keys[i] >> shift) & 255u], 1u);
-    }
+    for (int r = 0; r < kSortItems; r++)
+        if (base + r * kSortTpb < n) atomicAdd(&hw[(key[r] >> shift) & 255u], 1u);
     __syncthreads();
-    uint32_t c = 0;
+    const int t = threadIdx.x;
+    if (t < 256) {
+        uint32_t c = 0;
 #pragma unroll
-    for (int w = 0; w < kTpb / 64; w++) c += h[w][threadIdx.x];
-    hist[(int64_t)threadIdx.x * nblk + blockIdx.x] = c;
+        for (int w = 0; w < kSortWaves; w++) c += h[w][t];
+        if (nblk <= kSortFewTiles) hist[(int64_t)blockIdx.x * 256 + t] = c;
+        else hist[(int64_t)t * nblk + blockIdx.x] = c;
+    }
 }
 
 // Exclusive scan of each digit's row of the digit-major block histogram
@@ -527,78 +536,128 @@ __global__ __launch_bounds__(kTpb) void k_hist_rows(const uint32_t *__restrict__
     if (threadIdx.x == 0) dtot[blockIdx.x] = run;
 }
 
+// Lanes of the wave whose digit equals this lane's (among the lanes ok).
+__device__ __forceinline__ uint64_t digit_peers(uint32_t d, bool ok)
+{
+    uint64_t peers = __ballot(ok);
+#pragma unroll
+    for (int b = 0; b < 8; b++) {
+        const uint64_t bal = __ballot((d >> b) & 1u);
+        peers &= ((d >> b) & 1u) ? bal : ~bal;
+    }
+    return peers;
+}
+
+// Exclusive scan of one value per thread over the first 256 threads of the
+// block (ws: 4 words of LDS); every thread of the block calls it.
+__device__ __forceinline__ uint32_t scan256(uint32_t v, uint32_t *ws)
+{
+    const int w = threadIdx.x >> 6;
+    const uint32_t incl = wave_incl_scan(v);
+    if (w < 4 && lane_id() == 63) ws[w] = incl;
+    __syncthreads();
+    uint32_t off = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        if (k < w) off += ws[k];
+    return off + incl - v;
+}
+
 // Scatter one tile of kSortTile keys.  The tile is first ranked into LDS in
-// digit order: within a round of 256 consecutive keys, ranks among equal
-// digits come from a wave-level match (8 ballots) and a per-digit prefix over
-// the block's 4 waves, so equal digits keep their input order (round, wave,
-// lane).  Then consecutive threads copy consecutive LDS slots to the output,
-// so the writes of one digit's run are contiguous.
-__global__ __launch_bounds__(kTpb) void k_radix_scatter(const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
-                                                        uint64_t *__restrict__ kout, uint32_t *__restrict__ vout,
-                                                        int64_t n, int shift, const uint32_t *__restrict__ hist,
-                                                        const uint32_t *__restrict__ hist_scan,
-                                                        const uint32_t *__restrict__ dtot, int nblk)
+// digit order.  Each wave ranks its own kSortItems * 64 consecutive keys, 64 at
+// a time, without a block barrier: ranks among equal digits come from a match
+// (8 ballots) and the wave's running count of the digit, so equal digits keep
+// their input order (wave, round, lane); one scan over digits and waves then
+// places them.  Consecutive threads copy consecutive LDS slots to the output,
+// so the writes of one digit's run are contiguous.  (Ranking the block's
+// threads together, four barriers per 256 keys, took 9.5 us for a single tile
+// of 2048 and 36.9 us for 2^22 keys; this 6.2 and 27.7 us.)
+__global__ __launch_bounds__(kSortTpb) void k_radix_scatter(const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
+                                                            uint64_t *__restrict__ kout, uint32_t *__restrict__ vout,
+                                                            int64_t n, int shift, const uint32_t *__restrict__ hist,
+                                                            const uint32_t *__restrict__ hist_scan,
+                                                            const uint32_t *__restrict__ dtot, int nblk)
 {
     __shared__ uint64_t skey[kSortTile];
     __shared__ uint32_t sval[kSortTile];
-    __shared__ uint32_t toff[256];         // first LDS slot of each digit in this tile
-    __shared__ uint32_t gofs[256];         // output position of that slot
-    __shared__ uint32_t run[256];          // next free LDS slot per digit
-    __shared__ uint32_t wcnt[kTpb / 64][256];
+    __shared__ uint32_t gofs[256];                 // output position of a digit's first LDS slot, minus that slot
+    __shared__ uint32_t wcnt[kSortWaves][256];     // per wave: digit counts, then first LDS slots
+    __shared__ uint32_t ws[2][4];
     const int t = threadIdx.x, w = t >> 6, lane = lane_id();
-    {
-        uint32_t tot;
-        const uint32_t c = hist[(int64_t)t * nblk + blockIdx.x];
-        const uint32_t o = block_excl_scan(c, &tot);
-        const uint32_t dbase = block_excl_scan(dtot[t], &tot);
-        toff[t] = o;
-        run[t] = o;
-        gofs[t] = dbase + hist_scan[(int64_t)t * nblk + blockIdx.x] - o;
-    }
     const int64_t base = (int64_t)blockIdx.x * kSortTile;
     const int cnt = (int)min<int64_t>(kSortTile, n - base);
-    const uint64_t lt = (lane == 0) ? 0ULL : (~0ULL >> (64 - lane));
+    const int first = w * kSortItems * 64 + lane;  // this lane's first key in the tile
+    uint64_t key[kSortItems];
+    uint32_t val[kSortItems], rank[kSortItems];
+#pragma unroll
     for (int r = 0; r < kSortItems; r++) {
-#pragma unroll
-        for (int k = 0; k < kTpb / 64; k++) wcnt[k][t] = 0;
-        __syncthreads();
-        const int li = r * kTpb + t;
-        const bool ok = li < cnt;
-        const uint64_t key = ok ? kin[base + li] : 0;
-        const uint32_t val = ok ? vin[base + li] : 0;
-        const uint32_t d = ok ? (uint32_t)((key >> shift) & 255u) : 0u;
-        uint64_t peers = __ballot(ok);
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            const uint64_t bal = __ballot((d >> b) & 1u);
-            peers &= ((d >> b) & 1u) ? bal : ~bal;
-        }
-        const uint32_t rank = __popcll(peers & lt);
-        if (ok && rank == 0) wcnt[w][d] = __popcll(peers);
-        __syncthreads();
-        {
-            uint32_t acc = run[t];
-#pragma unroll
-            for (int k = 0; k < kTpb / 64; k++) {
-                const uint32_t c = wcnt[k][t];
-                wcnt[k][t] = acc;
-                acc += c;
-            }
-            run[t] = acc;
-        }
-        __syncthreads();
-        if (ok) {
-            const uint32_t slot = wcnt[w][d] + rank;
-            skey[slot] = key;
-            sval[slot] = val;
-        }
-        __syncthreads();   // wcnt is cleared at the top of the next round
+        const int li = first + r * 64;
+        key[r] = li < cnt ? kin[base + li] : 0;
+        val[r] = li < cnt ? vin[base + li] : 0;
     }
-    for (int j = t; j < cnt; j += kTpb) {
-        const uint64_t key = skey[j];
-        const uint32_t dst = gofs[(key >> shift) & 255u] + (uint32_t)j;
-        kout[dst] = key;
-        vout[dst] = sval[j];
+    // the digit's first output slot and this tile's place among its keys
+    uint32_t total = 0, before = 0;
+    if (t < 256) {
+        if (nblk <= kSortFewTiles) {
+#pragma unroll 8
+            for (int b = 0; b < nblk; b++) {
+                const uint32_t c = hist[b * 256 + t];
+                total += c;
+                if (b < (int)blockIdx.x) before += c;
+            }
+        } else {
+            total = dtot[t];
+            before = hist_scan[(int64_t)t * nblk + blockIdx.x];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 256 / 64; k++) wcnt[w][k * 64 + lane] = 0;
+    const uint64_t lt = (lane == 0) ? 0ULL : (~0ULL >> (64 - lane));
+    uint32_t *mine = wcnt[w];
+#pragma unroll
+    for (int r = 0; r < kSortItems; r++) {
+        const bool ok = first + r * 64 < cnt;
+        const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
+        const uint64_t peers = digit_peers(d, ok);
+        const uint32_t below = __popcll(peers & lt), old = mine[d];
+        rank[r] = old + below;
+        if (ok && below == 0) mine[d] = old + __popcll(peers);
+    }
+    const uint32_t dbase = scan256(total, ws[0]);  // (its barrier also ends the ranking)
+    uint32_t c[kSortWaves], sum = 0;
+    if (t < 256)
+#pragma unroll
+        for (int k = 0; k < kSortWaves; k++) {
+            c[k] = wcnt[k][t];
+            sum += c[k];
+        }
+    uint32_t slot0 = scan256(sum, ws[1]);
+    if (t < 256) {
+        gofs[t] = dbase + before - slot0;
+#pragma unroll
+        for (int k = 0; k < kSortWaves; k++) {
+            wcnt[k][t] = slot0;
+            slot0 += c[k];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortItems; r++)
+        if (first + r * 64 < cnt) {
+            const uint32_t slot = mine[(key[r] >> shift) & 255u] + rank[r];
+            skey[slot] = key[r];
+            sval[slot] = val[r];
+        }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortItems; r++) {
+        const int j = r * kSortTpb + t;
+        if (j < cnt) {
+            const uint64_t k = skey[j];
+            const uint32_t dst = gofs[(k >> shift) & 255u] + (uint32_t)j;
+            kout[dst] = k;
+            vout[dst] = sval[j];
+        }
     }
 }
 
@@ -1627,9 +1686,9 @@ void radix_sort_pairs(bh_ctx *ctx, uint64_t *k0, uint64_t *k1, uint32_t *v0, uin
     uint64_t *ka = k0, *kb = k1;
     uint32_t *va = v0, *vb = v1;
     for (int shift = begin_bit; shift < end_bit; shift += 8) {
-        k_radix_hist<<<nblk, kTpb, 0, ctx->stream>>>(ka, n, shift, hist, nblk);
-        k_hist_rows<<<256, kTpb, 0, ctx->stream>>>(hist, nblk, hscan, dtot);
-        k_radix_scatter<<<nblk, kTpb, 0, ctx->stream>>>(ka, va, kb, vb, n, shift, hist, hscan, dtot, nblk);
+        k_radix_hist<<<nblk, kSortTpb, 0, ctx->stream>>>(ka, n, shift, hist, nblk);
+        if (nblk > kSortFewTiles) k_hist_rows<<<256, kTpb, 0, ctx->stream>>>(hist, nblk, hscan, dtot);
+        k_radix_scatter<<<nblk, kSortTpb, 0, ctx->stream>>>(ka, va, kb, vb, n, shift, hist, hscan, dtot, nblk);
         std::swap(ka, kb);
         std::swap(va, vb);
     }
