@@ -416,16 +416,15 @@ void bh_destroy(bh_ctx *ctx)
     lf_drop_graph(ctx);
     bh::DevBuf *bufs[] = {&ctx->mass,   &ctx->pos,    &ctx->tpos,   &ctx->dbox,    &ctx->dboxi,  &ctx->keys0,
                           &ctx->keys1,  &ctx->vals0,  &ctx->vals1,  &ctx->hist,    &ctx->scan_tmp, &ctx->tkeys0,
-                          &ctx->tkeys1, &ctx->tvals0, &ctx->tvals1, &ctx->nmassive, &ctx->bd,    &ctx->bpk,   &ctx->bhi,
-                          &ctx->blo,    &ctx->thi,    &ctx->tlo,    &ctx->td,      &ctx->tperm,  &ctx->tself, &ctx->tinv, &ctx->tmap,
-                          &ctx->cpl,    &ctx->ccnt,   &ctx->cbase,  &ctx->cmin1,   &ctx->cmin2,  &ctx->cfirst,
+                          &ctx->tkeys1, &ctx->tvals0, &ctx->tvals1, &ctx->bd,    &ctx->bpk,   &ctx->bhi,
+                          &ctx->blo,    &ctx->thi,    &ctx->tlo,    &ctx->td,      &ctx->tself, &ctx->tinv, &ctx->tmap,
+                          &ctx->cpl,    &ctx->ccnt,   &ctx->cbase,  &ctx->cmin1,   &ctx->cfirst,
                           &ctx->clast,  &ctx->clevel, &ctx->csub,   &ctx->cnkids,  &ctx->crc2,
                           &ctx->cskip,  &ctx->pre,    &ctx->cmo,    &ctx->mpre,    &ctx->mpart,  &ctx->ptile, &ctx->pseg,
                           &ctx->cA,     &ctx->cB,     &ctx->cQ0,    &ctx->cQ1,     &ctx->counters, &ctx->frontier,
-                          &ctx->gctr,   &ctx->werr, &ctx->shlist, &ctx->shid,   &ctx->phi,    &ctx->acc,    &ctx->gfirst, &ctx->gcount,
+                          &ctx->gctr,   &ctx->shlist, &ctx->shid,   &ctx->phi,    &ctx->acc,    &ctx->gfirst, &ctx->gcount,
                           &ctx->gscan,  &ctx->goff,   &ctx->gcpl,   &ctx->gccnt,   &ctx->gcbase, &ctx->gm1,
-                          &ctx->gm2,    &ctx->gcf,    &ctx->gcl,    &ctx->gclv,   &ctx->lhist,  &ctx->llist,  &ctx->bcand,  &ctx->bcount, &ctx->lkeys0, &ctx->lkeys1,
-                          &ctx->lvals0, &ctx->lvals1, &ctx->cfnb, &ctx->cowner, &ctx->gowner,
+                          &ctx->gcf,    &ctx->gcl,    &ctx->gclv,   &ctx->lhist,  &ctx->llist,  &ctx->bcand,  &ctx->cfnb,
                           &ctx->vel,    &ctx->acc_old, &ctx->lfstep, &ctx->diag_partial, &ctx->diag_buf,
                           &ctx->n2b_buf, &ctx->nbc_buf, &ctx->lrec, &ctx->sacc,   &ctx->cF0,    &ctx->cF1,
                           &ctx->mlp.params, &ctx->mlp.wb, &ctx->mlp.bias, &ctx->mlp.gpart, &ctx->mlp.lpart,
@@ -573,6 +572,7 @@ bh_status bh_debug_cells(bh_ctx *ctx, int64_t cap, int *level, int *nbody, doubl
             if (level) level[i] = lv[i];
             if (nbody) nbody[i] = l[i] - f[i] + 1;
         }
+        bh::fill_moments(ctx);
         std::vector<double> mo(10 * k);
         BH_HIP(hipMemcpy(mo.data(), ctx->tree.mo, 10 * k * sizeof(double), hipMemcpyDeviceToHost));
         for (int64_t i = 0; i < k; i++) {

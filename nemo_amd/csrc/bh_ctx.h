@@ -32,7 +32,7 @@ struct bh_ctx {
     // second stream of the tree build (same priority): branches that no
     // kernel of the main stream needs until the matching join
     hipStream_t side = nullptr;
-    hipEvent_t fork_ev[6] = {};
+    hipEvent_t fork_ev[4] = {};
     std::string err;
     int inject = 0;
 
@@ -47,27 +47,26 @@ struct bh_ctx {
     // inputs (device, input order)
     bh::DevBuf mass, pos, tpos;
     // box state: double4 box, ints {first, start, changed, nonfinite}
-    bh::DevBuf dbox, dboxi, bcand, bcount;
+    bh::DevBuf dbox, dboxi, bcand;
     // sorting
     bh::DevBuf keys0, keys1, vals0, vals1, hist, scan_tmp;
     bh::DevBuf tkeys0, tkeys1, tvals0, tvals1;
-    bh::DevBuf nmassive;        // int
     // sorted bodies of the tree and of the test set
     bh::DevBuf bd, bhi, blo, bpk;   // bpk: (x, y, z, m) records in input order
-    bh::DevBuf thi, tlo, td, tperm, tself, tinv, tmap;
+    bh::DevBuf thi, tlo, td, tself, tinv, tmap;
     // topology
-    bh::DevBuf cpl, ccnt, cbase, cmin1, cmin2;
-    bh::DevBuf cfirst, clast, clevel, csub, cnkids, cskip, pre, cowner, gowner;
+    bh::DevBuf cpl, ccnt, cbase, cmin1;
+    bh::DevBuf cfirst, clast, clevel, csub, cnkids, cskip, pre;
     bh::DevBuf crc2;            // treecode1 Rcrit2 per cell (criterion != BH_CRIT_HACK)
-    bh::DevBuf cmo, cfnb, cA, cB, cQ0, cQ1, lhist, llist, lkeys0, lkeys1, lvals0, lvals1;
+    bh::DevBuf cmo, cfnb, cA, cB, cQ0, cQ1, lhist, llist;
     bh::DevBuf mpre, mpart;     // fast monopole trees: tile-local prefix sums of (m x, m y, m z, m), tile prefixes
     bh::DevBuf counters;        // u64: n2b, nbc, deep, n_mlp, err flags ...
     // groups of the test set (fast walk)
     bh::DevBuf gfirst, gcount, gscan, goff;
-    bh::DevBuf gcpl, gccnt, gcbase, gm1, gm2, gcf, gcl, gclv;
+    bh::DevBuf gcpl, gccnt, gcbase, gm1, gcf, gcl, gclv;
     int ngroups = 0;          // host copy after an evaluation
     // walk scratch
-    bh::DevBuf frontier, gctr, werr;
+    bh::DevBuf frontier, gctr;
     bh::DevBuf shlist, shid;    // super-group walk: shared lists per wave
     int64_t fcap = 0;
     // outputs (input order of the test set)
@@ -102,6 +101,7 @@ struct bh_ctx {
     bh::DevBuf ptile, pseg;     // prefix-sum moments of a batch: (first, end) body per tile, first tile per system
     int nptile = 0;
     bh::Tree tree;
+    bh::MomArgs mom;            // of the last fast build; its FP64 moments (tree.mo) are written on demand
     int64_t nb = 0;             // massive bodies (counted at upload)
     int cell_cap = 0;           // cell capacity of the tree arrays
     bool mlp_sampling = false;  // a sample-collection walk is running (the tree writes learned features)
@@ -146,6 +146,7 @@ T *ptr(DevBuf &b) { return static_cast<T *>(b.p); }
 
 // bh_tree.hip
 void build_tree(bh_ctx *ctx, const bh_params &p);
+void fill_moments(bh_ctx *ctx);   // tree.mo of the last build, if it was not written
 void exclusive_scan_u32(bh_ctx *ctx, const uint32_t *in, uint32_t *out, int64_t n,
                         const unsigned long long *dn = nullptr);
 void radix_sort_pairs(bh_ctx *ctx, uint64_t *k0, uint64_t *k1, uint32_t *v0, uint32_t *v1, int64_t n,

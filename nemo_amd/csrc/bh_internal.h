@@ -65,6 +65,25 @@ struct Tree {
     const float4 *cF1 = nullptr;       // Q_xx, Q_yy, Q_xy, Q_xz over M size^2
 };
 
+// The prefix-sum moments of a fast build: the bodies' tile sums, the cells, and
+// the records to write (bh_tree.hip k_moments_prefix).
+struct MomArgs {
+    bool quad = false;
+    int grid = 0;
+    const int *first = nullptr, *last = nullptr;
+    const uint8_t *level = nullptr;
+    const unsigned long long *ncellp = nullptr;
+    int nb = 0, ntile = 0;
+    const double4 *loc = nullptr, *part = nullptr;
+    const int *seg = nullptr;
+    const uint64_t *keys = nullptr;
+    float4 *cA = nullptr, *cB = nullptr, *cQ0 = nullptr, *cQ1 = nullptr, *cF0 = nullptr, *cF1 = nullptr;
+    const double4 *box = nullptr;
+    int lsys = 0, sysbits = 0;
+    const double4 *sysbox = nullptr;
+    const int64_t *boff = nullptr;
+};
+
 constexpr int kNoChild = INT32_MIN;  // empty octant in Tree::sub
 
 // Device status words (unsigned long long) written by the kernels and read

@@ -84,8 +84,8 @@ __device__ __forceinline__ BoxTest box_test(const double4 b)
 {
     const unsigned long long bits = (unsigned long long)__double_as_longlong(b.w);
     const unsigned e = (unsigned)((bits >> 52) & 0x7ff);
-    const bool p2 = (bits & 0x000FFFFFFFFFFFFFULL) == 0 && e - 1u < 0x7feu;
-    return {b, p2 ? 1.0 / b.w : 0.0, p2};
+    const bool p2 = (bits & 0x000FFFFFFFFFFFFFULL) == 0 && e - 1u < 0x7fdu;
+    return {b, p2 ? __longlong_as_double((long long)(0x7feu - e) << 52) : 0.0, p2};   // 2^-(e - 1023)
 }
 
 __device__ __forceinline__ bool fits(const double *x, const BoxTest &t)
@@ -102,9 +102,7 @@ __device__ __forceinline__ bool fits(const double4 c, const BoxTest &t)
 }
 
 // Massive bodies outside the starting box (the only ones that can ever make
-// expandbox grow it, since the box only grows), compacted in input order:
-// per-block counts, a scan, then per-block writes.  Block b owns the input
-// range [b*chunk, (b+1)*chunk).
+// expandbox grow it, since the box only grows).
 __device__ __forceinline__ bool outside_massive(const double *__restrict__ pos, const double *__restrict__ mass,
                                                 int64_t i, int64_t n, const BoxTest &b, int *bad)
 {
@@ -125,36 +123,10 @@ __device__ __forceinline__ bool outside_massive(const double *__restrict__ pos, 
 // so the rounds read it contiguously.
 constexpr int kBoxPer = 16, kBoxChunk = kTpb * kBoxPer;
 
-__global__ __launch_bounds__(kTpb) void k_box_compact(const double *__restrict__ pos, const double *__restrict__ mass,
-                                                      int64_t n, const double4 *__restrict__ box, double4 *cand,
-                                                      int *boxi, unsigned long long *stat)
-{
-    __shared__ uint32_t base;
-    const BoxTest b = box_test(*box);
-    const int64_t i0 = (int64_t)blockIdx.x * kBoxChunk + threadIdx.x;
-    int bad = 0;
-    uint32_t mask = 0;
-#pragma unroll
-    for (int k = 0; k < kBoxPer; k++)
-        if (outside_massive(pos, mass, i0 + k * kTpb, n, b, &bad)) mask |= 1u << k;
-    uint32_t tot;
-    uint32_t off = block_excl_scan((uint32_t)__popc(mask), &tot);
-    if (threadIdx.x == 0 && tot) base = atomicAdd(reinterpret_cast<uint32_t *>(&boxi[4]), tot);
-    __syncthreads();
-    while (mask) {
-        const int k = __ffs(mask) - 1;
-        mask &= mask - 1;
-        const int64_t i = i0 + k * kTpb;
-        const double *x = pos + 3 * i;
-        cand[base + off++] = make_double4(x[0], x[1], x[2], (double)i);
-    }
-    if (bad) atomicOr(&stat[S_FLAGS], (unsigned long long)F_NONFINITE);
-}
-
 // Doubling of expandbox (load.c:68-95) until body x fits.
 __device__ __forceinline__ double4 expand_for(const double *x, double4 b)
 {
-    for (int guard = 0; guard < 2000 && !fits(x, b); guard++) {
+    for (int guard = 0; guard < 2000 && !fits(x, box_test(b)); guard++) {
         double rmid0 = b.x + 0.5 * b.w, rmid1 = b.y + 0.5 * b.w, rmid2 = b.z + 0.5 * b.w;
         if (x[0] < rmid0) b.x -= b.w;
         if (x[1] < rmid1) b.y -= b.w;
@@ -164,71 +136,226 @@ __device__ __forceinline__ double4 expand_for(const double *x, double4 b)
     return b;
 }
 
-// One expansion round: every block reduces the lowest candidate index >=
-// start that lies outside the box (atomicMin into boxi[0]); the last block
-// to finish (ticket in boxi[3]) expands the box toward that body and moves
-// start past it, or, when no candidate is outside, sets boxi[5] (done), after
-// which the remaining rounds return at once.
-__global__ __launch_bounds__(kTpb) void k_box_round(const double *__restrict__ pos, const double4 *__restrict__ cand,
-                                                    double4 *box, int *boxi)
+// expandbox over I bodies per thread of one block, held in registers (body of
+// round r: first + r * 64, first - lane a multiple of 64; massive bit r of mask):
+// the first body in input order outside the box doubles it, then the next body
+// after that one, until none is outside.  At most `rounds` expansions; returns
+// whether the box closed (a non-finite body closes it and is flagged).
+// A wave looks through its bodies in input order, stops at the first 64 that
+// hold one outside and goes on from there after the expansion (what was inside
+// stays inside), so all rounds together test each body about once; testing all
+// of them in every round took 5 us per expansion at 12 bodies per thread.
+struct BoxPick {
+    int f[16];          // first body outside, per wave
+    double p[3];        // its position
+};
+
+template <int T, int I>
+__device__ __forceinline__ bool box_rounds(const double (&x)[I][3], unsigned mask, int first, double4 &b, int rounds,
+                                           BoxPick &pick, unsigned long long *stat)
 {
-    __shared__ int wbest[kTpb / 64];
-    if (boxi[5]) return;
-    const double4 b0 = *box;
-    const BoxTest b = box_test(b0);
-    const int start = boxi[1], nc = boxi[4];
-    int best = INT32_MAX;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nc; k += gridDim.x * blockDim.x) {
-        const double4 c = cand[k];
-        const int i = (int)c.w;
-        if (i >= start && i < best && !fits(c, b)) best = i;
-    }
+    static_assert(T / 64 <= 16, "BoxPick");
+    const int w = threadIdx.x >> 6, base = first - lane_id();
+    int start = 0, done = 0;
+    for (int round = 0;; round++) {
+        const BoxTest bt = box_test(b);
+        int mine = INT32_MAX;
+        double p[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) best = min(best, __shfl_xor(best, d, 64));
-    if (lane_id() == 0) wbest[threadIdx.x >> 6] = best;
+        for (int r = 0; r < I; r++)
+            if (r >= done && mine == INT32_MAX) {          // (the same in every lane)
+                const uint64_t m = __ballot((mask >> r & 1u) && first + r * 64 >= start && !fits(x[r], bt));
+                if (m) {
+                    const int at = __builtin_ctzll(m);
+                    mine = base + r * 64 + at;
+                    done = r;
+#pragma unroll
+                    for (int k = 0; k < 3; k++) p[k] = __shfl(x[r][k], at, 64);
+                } else {
+                    done = r + 1;
+                }
+            }
+        if (lane_id() == 0) pick.f[w] = mine;
+        __syncthreads();
+        int f = INT32_MAX;
+#pragma unroll
+        for (int k = 0; k < T / 64; k++) f = min(f, pick.f[k]);
+        if (f == mine && f != INT32_MAX && lane_id() == 0)
+#pragma unroll
+            for (int k = 0; k < 3; k++) pick.p[k] = p[k];
+        __syncthreads();
+        if (f == INT32_MAX) return true;
+        if (round == rounds) return false;
+#pragma unroll
+        for (int k = 0; k < 3; k++) p[k] = pick.p[k];
+        if (!(isfinite(p[0]) && isfinite(p[1]) && isfinite(p[2]))) {
+            if (threadIdx.x == 0) atomicOr(&stat[S_FLAGS], (unsigned long long)F_NONFINITE);
+            return true;
+        }
+        b = expand_for(p, b);
+        start = f + 1;
+    }
+}
+
+// One pass over the bodies from i0 on (boxi[1]: the first not yet expanded for).
+// Every block lists the bodies outside the box; the last one to finish (ticket
+// in boxi[6]) expands for the first of them and for the kBoxWindow bodies in
+// input order from there, which reach most of the extent, and, when the list is
+// short (few), looks it through for the next body outside until there is
+// none (boxi[5]: done, later passes return at once).  A longer list is left to
+// the next pass, against the grown box.  A launch per expansion instead (one for
+// each of 7 possible) took 14 us of 364 at 2^20 bodies inside the box.  One block
+// reads a list of 10^5 bodies (a halo that follows its disk) in ~50 us per look,
+// so from kBoxOne bodies on there is a second pass (3 us when nothing is left to
+// do), and only the last pass takes a list as long as kBoxFew.
+constexpr int kBoxOne = 1 << 15, kBoxShort = 1 << 12, kBoxFew = 1 << 17;
+constexpr int kBoxWinPer = 8, kBoxWindow = kTpb * kBoxWinPer, kBoxAhead = 4;
+
+__global__ __launch_bounds__(kTpb) void k_box_compact(const double *__restrict__ pos, const double *__restrict__ mass,
+                                                      int64_t i0, int64_t n, double4 *box, double4 *cand, int *boxi,
+                                                      int rounds, int few, unsigned long long *stat)
+{
+    __shared__ uint32_t base;
+    __shared__ int red[kTpb / 64];
+    __shared__ BoxPick pick;
+    __shared__ bool last;
+    if (boxi[5]) return;
+    const int begin = boxi[1];
+    double4 bx = *box;
+    BoxTest b = box_test(bx);
+    const int64_t j0 = i0 + (int64_t)blockIdx.x * kBoxChunk + threadIdx.x;
+    int bad = 0;
+    uint32_t mask = 0;
+#pragma unroll
+    for (int k = 0; k < kBoxPer; k++)
+        if (j0 + k * kTpb >= begin && outside_massive(pos, mass, j0 + k * kTpb, n, b, &bad)) mask |= 1u << k;
+    uint32_t tot;
+    uint32_t off = block_excl_scan((uint32_t)__popc(mask), &tot);
+    if (threadIdx.x == 0 && tot) base = atomicAdd(reinterpret_cast<uint32_t *>(&boxi[4]), tot);
+    if (tot) {
+        int f = mask ? (int)(j0 + (__ffs(mask) - 1) * kTpb) : INT32_MAX;
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) f = min(f, __shfl_xor(f, d, 64));
+        if (lane_id() == 0 && f != INT32_MAX) atomicMin(&boxi[0], f);
+    }
+    __syncthreads();
+    while (mask) {
+        const int k = __ffs(mask) - 1;
+        mask &= mask - 1;
+        const int64_t i = j0 + k * kTpb;
+        const double *x = pos + 3 * i;
+        cand[base + off++] = make_double4(x[0], x[1], x[2], (double)i);
+    }
+    if (bad) atomicOr(&stat[S_FLAGS], (unsigned long long)F_NONFINITE);
     __syncthreads();
     if (threadIdx.x == 0) {
-        int m = wbest[0];
+        if (tot) __threadfence();      // this block's candidates (the barrier ordered them before this thread)
+        last = atomicAdd(reinterpret_cast<unsigned *>(&boxi[6]), 1u) == gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    const int nc = atomicAdd(&boxi[4], 0);
+    int f = atomicAdd(&boxi[0], 0), start = begin;
+    for (int look = 0; f != INT32_MAX && look < rounds; look++) {
+        double x[kBoxWinPer][3];
+        unsigned massive = 0;
+        const int first = f + (int)(threadIdx.x >> 6) * kBoxWinPer * 64 + lane_id();
 #pragma unroll
-        for (int k = 1; k < kTpb / 64; k++) m = min(m, wbest[k]);
-        if (m != INT32_MAX) atomicMin(&boxi[0], m);
-        __threadfence();
-        const unsigned t = atomicAdd(reinterpret_cast<unsigned *>(&boxi[3]), 1u);
-        if (t == gridDim.x - 1) {
-            __threadfence();
-            const int first = atomicMin(&boxi[0], INT32_MAX);   // atomic read
-            boxi[3] = 0;
-            if (first != INT32_MAX) {
-                *box = expand_for(pos + 3 * (int64_t)first, b0);
-                boxi[2] += 1;
-                boxi[0] = INT32_MAX;
-                boxi[1] = first + 1;
-            } else {
-                boxi[5] = 1;
+        for (int r = 0; r < kBoxWinPer; r++) {
+            const int64_t i = min<int64_t>((int64_t)first + r * 64, n - 1);
+            if ((int64_t)first + r * 64 < n && mass[i] != 0.0) massive |= 1u << r;
+#pragma unroll
+            for (int k = 0; k < 3; k++) x[r][k] = pos[3 * i + k];
+        }
+        if (!box_rounds<kTpb, kBoxWinPer>(x, massive, first, bx, rounds, pick, stat)) break;
+        b = box_test(bx);
+        start = (int)min(n, (int64_t)f + kBoxWindow);
+        if (nc > few) break;
+        f = INT32_MAX;
+        for (int k0 = threadIdx.x; k0 < nc; k0 += kTpb * kBoxAhead) {
+            double4 c[kBoxAhead];
+#pragma unroll
+            for (int u = 0; u < kBoxAhead; u++) c[u] = cand[min(k0 + u * kTpb, nc - 1)];
+#pragma unroll
+            for (int u = 0; u < kBoxAhead; u++) {
+                const int i = (int)c[u].w;
+                if (i >= start && i < f && !fits(c[u], b)) f = i;
             }
         }
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) f = min(f, __shfl_xor(f, d, 64));
+        if (lane_id() == 0) red[threadIdx.x >> 6] = f;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kTpb / 64; k++) f = min(f, red[k]);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        *box = bx;
+        boxi[0] = INT32_MAX;
+        boxi[1] = start;
+        boxi[4] = boxi[6] = 0;
+        if (f == INT32_MAX) boxi[5] = 1;
     }
 }
 
 // Starting box: the caller's (rmin, rsize), or the previous box when keep.
-// boxi: [0] first outside candidate (min), [1] start index, [2] expansions,
-// [3] round ticket, [4] candidate count, [5] done.
-// Start of a build: clear the per-evaluation status words and, when box is
-// given, set the start box and the expansion bookkeeping (one launch).
-__global__ void k_build_start(unsigned long long *stat, int nzero, uint32_t *lwork, int nlwork, double4 *box,
-                              int *boxi, double rx, double ry, double rz, double rsize, int keep)
+// boxi: [0] first body outside of a pass (min), [1] first body not yet expanded
+// for, [4] bodies outside, [5] done, [6] ticket.
+struct BoxStart {
+    double rx, ry, rz, rsize;
+    int keep;
+};
+
+// Start of a build, by one block of at least 128 threads: clear the
+// per-evaluation status words and work counters.
+__device__ __forceinline__ void build_start(unsigned long long *stat, int nzero, uint32_t *lwork, int nlwork)
 {
     if ((int)threadIdx.x < nzero) stat[threadIdx.x] = 0;
     if (threadIdx.x == 0) stat[S_GCTR] = 0;
     if ((int)threadIdx.x < nlwork) lwork[threadIdx.x] = 0;
-    if (threadIdx.x != 0 || !box) return;
-    if (!keep) *box = make_double4(rx, ry, rz, rsize);
-    boxi[0] = INT32_MAX;
-    boxi[1] = 0;
-    boxi[2] = 0;
-    boxi[3] = 0;
-    boxi[4] = 0;
-    boxi[5] = 0;
+}
+
+__global__ void k_build_start(unsigned long long *stat, int nzero, uint32_t *lwork, int nlwork)
+{
+    build_start(stat, nzero, lwork, nlwork);
+}
+
+// Start of a build and, from a fresh box, expandbox over the first kBoxFirst
+// bodies by one block: in input order these already reach most of a system's
+// extent, so few of the others are candidates for k_box_compact.
+constexpr int kFirstTpb = 1024, kFirstPer = 8, kBoxFirst = kFirstTpb * kFirstPer;
+__global__ __launch_bounds__(kFirstTpb) void k_box_first(const double *__restrict__ pos, const double *__restrict__ mass,
+                                                         int64_t n, BoxStart st, int rounds, double4 *box, int *boxi,
+                                                         unsigned long long *stat, int nzero, uint32_t *lwork, int nlwork)
+{
+    __shared__ BoxPick pick;
+    build_start(stat, nzero, lwork, nlwork);
+    __syncthreads();
+    double4 b = st.keep ? *box : make_double4(st.rx, st.ry, st.rz, st.rsize);
+    if (!st.keep) {
+        double x[kFirstPer][3];
+        unsigned mask = 0;
+        const int first = (threadIdx.x >> 6) * kFirstPer * 64 + lane_id();
+#pragma unroll
+        for (int r = 0; r < kFirstPer; r++) {
+            const int64_t i = min<int64_t>(first + r * 64, n - 1);
+            if (first + r * 64 < n && mass[i] != 0.0) mask |= 1u << r;
+#pragma unroll
+            for (int k = 0; k < 3; k++) x[r][k] = pos[3 * i + k];
+        }
+        // (not closed within the rounds: the bodies left outside stay
+        // candidates only if k_box_compact starts over, so flag it)
+        if (!box_rounds<kFirstTpb, kFirstPer>(x, mask, first, b, rounds, pick, stat) && threadIdx.x == 0)
+            atomicOr(&stat[S_FLAGS], (unsigned long long)F_BOX_OPEN);
+    }
+    if (threadIdx.x == 0) {
+        if (!st.keep) *box = b;
+        boxi[0] = INT32_MAX;
+        boxi[1] = st.keep ? 0 : (int)min(n, (int64_t)kBoxFirst);
+        for (int k = 2; k < 7; k++) boxi[k] = 0;
+    }
 }
 
 // ---- batched ensembles: one box per system -----------------------------------
@@ -302,38 +429,49 @@ __global__ __launch_bounds__(kTpb) void k_sys_box(const double *__restrict__ pos
 
 // ---- keys ------------------------------------------------------------------
 
-__device__ __forceinline__ uint64_t spread3(uint64_t v)
+__device__ __forceinline__ uint32_t spread3(uint32_t v)   // of 10 bits
 {
-    v &= 0x1fffffULL;
-    v = (v | (v << 32)) & 0x1f00000000ffffULL;
-    v = (v | (v << 16)) & 0x1f0000ff0000ffULL;
-    v = (v | (v << 8)) & 0x100f00f00f00f00fULL;
-    v = (v | (v << 4)) & 0x10c30c30c30c30c3ULL;
-    v = (v | (v << 2)) & 0x1249249249249249ULL;
+    v = (v | v << 16) & 0x030000ffu;
+    v = (v | v << 8) & 0x0300f00fu;
+    v = (v | v << 4) & 0x030c30c3u;
+    v = (v | v << 2) & 0x09249249u;
     return v;
 }
 
-// Interleaved top `levels` bits of the three 30-bit integer coordinates.
+// Morton code of three 21-bit coordinates, x highest: bits 0..9, 10..19 and 20
+// by themselves, all in 32-bit operations.
+__device__ __forceinline__ uint64_t interleave(const uint32_t (&c)[3])
+{
+    auto part = [&](int sh) {
+        return spread3(c[0] >> sh & 0x3ffu) << 2 | spread3(c[1] >> sh & 0x3ffu) << 1 | spread3(c[2] >> sh & 0x3ffu);
+    };
+    const uint32_t top = (c[0] >> 20) << 2 | (c[1] >> 20) << 1 | c[2] >> 20, mid = part(10), low = part(0);
+    return (uint64_t)(top << 28 | mid >> 2) << 32 | (mid << 30 | low);
+}
+
+// Interleaved top `levels` bits of the three 30-bit integer coordinates
+// (box_test's multiplication in the place of the division where it is exact).
 __device__ __forceinline__ uint64_t morton_of(const double *x, const double4 b, int levels = kMaxLevel)
 {
-    uint64_t c[3];
+    const BoxTest t = box_test(b);
+    uint32_t c[3];
     const double rm[3] = {b.x, b.y, b.z};
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        double xsc = (x[k] - rm[k]) / b.w;
-        int64_t xi;
+        double xsc = t.p2 ? (x[k] - rm[k]) * t.inv : (x[k] - rm[k]) / b.w;
+        int32_t xi;
         if (!(xsc >= 0.0)) xi = 0;
         else if (!(xsc < 1.0)) xi = (1 << 30) - 1;
-        else xi = (int64_t)floor(1073741824.0 * xsc);
-        c[k] = (uint64_t)(xi >> (30 - levels));
+        else xi = (int32_t)(1073741824.0 * xsc);   // (the floor: xsc >= 0)
+        c[k] = (uint32_t)xi >> (30 - levels);
     }
-    return (spread3(c[0]) << 2) | (spread3(c[1]) << 1) | spread3(c[2]);
+    return interleave(c);
 }
 
 // Batch keys: [system id : sysbits][Morton code of kMaxLevel - sysbits/3
 // levels in the system's own box]; the system digits form the top levels.
 __global__ void k_keys_batch(const double *__restrict__ pos, int64_t n, const int64_t *__restrict__ off, int nsys,
-                             const double4 *__restrict__ sysbox, int sysbits, uint64_t *keys, uint32_t *vals)
+                             const double4 *__restrict__ sysbox, int sysbits, uint64_t *keys)
 {
     const int levels = kMaxLevel - sysbits / 3;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
@@ -345,7 +483,6 @@ __global__ void k_keys_batch(const double *__restrict__ pos, int64_t n, const in
         }
         const uint64_t m = morton_of(pos + 3 * i, sysbox[lo], levels);
         keys[i] = ((uint64_t)lo << (3 * levels)) | m;
-        vals[i] = (uint32_t)i;
     }
 }
 
@@ -356,7 +493,7 @@ __global__ void k_keys_batch(const double *__restrict__ pos, int64_t n, const in
 // done flag; a box that no round found closed (every candidate inside) is
 // flagged, and the host grows the number of rounds
 __global__ void k_keys(const double *__restrict__ pos, const double *__restrict__ mass, int64_t n,
-                       const double4 *__restrict__ box, uint64_t *keys, uint32_t *vals, double4 *pk,
+                       const double4 *__restrict__ box, uint64_t *keys, double4 *pk,
                        const int *__restrict__ boxi = nullptr, unsigned long long *stat = nullptr)
 {
     if (boxi && blockIdx.x == 0 && threadIdx.x == 0 && !boxi[5]) atomicOr(&stat[S_FLAGS], (unsigned long long)F_BOX_OPEN);
@@ -367,7 +504,6 @@ __global__ void k_keys(const double *__restrict__ pos, const double *__restrict_
         const double m = mass != nullptr ? mass[i] : 0.0;
         if (mass != nullptr && m == 0.0) k |= (1ULL << 63);
         keys[i] = k;
-        vals[i] = (uint32_t)i;
         if (pk) pk[i] = make_double4(x[0], x[1], x[2], m);
     }
 }
@@ -539,13 +675,16 @@ __global__ __launch_bounds__(kTpb) void k_hist_rows(const uint32_t *__restrict__
 // Lanes of the wave whose digit equals this lane's (among the lanes ok).
 __device__ __forceinline__ uint64_t digit_peers(uint32_t d, bool ok)
 {
-    uint64_t peers = __ballot(ok);
+    const uint64_t all = __ballot(ok);
+    uint32_t lo = (uint32_t)all, hi = (uint32_t)(all >> 32);
 #pragma unroll
     for (int b = 0; b < 8; b++) {
-        const uint64_t bal = __ballot((d >> b) & 1u);
-        peers &= ((d >> b) & 1u) ? bal : ~bal;
+        const uint32_t bit = (uint32_t)((int)(d << (31 - b)) >> 31);   // 0 or all ones
+        const uint64_t bal = __ballot(bit != 0);
+        lo &= ~((uint32_t)bal ^ bit);
+        hi &= ~((uint32_t)(bal >> 32) ^ bit);
     }
-    return peers;
+    return (uint64_t)hi << 32 | lo;
 }
 
 // Exclusive scan of one value per thread over the first 256 threads of the
@@ -569,10 +708,11 @@ __device__ __forceinline__ uint32_t scan256(uint32_t v, uint32_t *ws)
 // (8 ballots) and the wave's running count of the digit, so equal digits keep
 // their input order (wave, round, lane); one scan over digits and waves then
 // places them.  Consecutive threads copy consecutive LDS slots to the output,
-// so the writes of one digit's run are contiguous.  (Ranking the block's
+// so the writes of one digit's run are contiguous.  vin null: the values are
+// the indices.  (Ranking the block's
 // threads together, four barriers per 256 keys, took 9.5 us for a single tile
 // of 2048 and 36.9 us for 2^22 keys; this 6.2 and 27.7 us.)
-__global__ __launch_bounds__(kSortTpb) void k_radix_scatter(const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
+__global__ __launch_bounds__(kSortTpb) void k_radix_scatter(const uint64_t *__restrict__ kin, const uint32_t *vin,
                                                             uint64_t *__restrict__ kout, uint32_t *__restrict__ vout,
                                                             int64_t n, int shift, const uint32_t *__restrict__ hist,
                                                             const uint32_t *__restrict__ hist_scan,
@@ -593,7 +733,7 @@ __global__ __launch_bounds__(kSortTpb) void k_radix_scatter(const uint64_t *__re
     for (int r = 0; r < kSortItems; r++) {
         const int li = first + r * 64;
         key[r] = li < cnt ? kin[base + li] : 0;
-        val[r] = li < cnt ? vin[base + li] : 0;
+        val[r] = li >= cnt ? 0 : vin ? vin[base + li] : (uint32_t)(base + li);
     }
     // the digit's first output slot and this tile's place among its keys
     uint32_t total = 0, before = 0;
@@ -661,6 +801,282 @@ __global__ __launch_bounds__(kSortTpb) void k_radix_scatter(const uint64_t *__re
     }
 }
 
+// ---- sorting in one block's LDS, merge passes ------------------------------------
+
+// Sorts T * I keys of a block, stably, with their values (T threads, I keys each;
+// wave w's keys are [w * 64 I, (w + 1) * 64 I), lane l's every 64th from l: its
+// I registers in rounds).  LSD digits of 8 bits: each wave ranks its keys by
+// ballot match and running counts, one scan over digits and waves places them.
+// The upper 32 bits first (4 passes); keys that agree there (few, unless bodies
+// cluster at the thousandth of the box) form runs, whose starts are listed (one
+// listing pass and then a run per thread: sorting each run where it was met, 12
+// us of 41 at 12 keys per thread).  A run of up to kRunMax keys is sorted by
+// insertion by one thread, one of up to kRunWave by a wave that counts each key's
+// rank; longer runs, or too many of those, send the block through all eight
+// digits.  The sorted keys and values end in skey and sval.
+constexpr int kRunMax = 8, kRunWave = 512, kRunList = 256;
+
+template <int T, int I, class V>
+struct BlockSort {
+    static constexpr int kW = T / 64, kN = T * I;
+    uint64_t skey[kN];
+    V sval[kN];
+    uint32_t wcnt[kW][256];
+    uint32_t ws[4];
+    int nshort, nrun, toolong;       // runs listed for a thread and for a wave, and whether one was not
+    uint32_t runs[kRunList];         // start | length << 16
+    static_assert(kN <= 1 << 16, "run list");
+
+    __device__ __forceinline__ void pass(uint64_t (&key)[I], V (&val)[I], int shift)
+    {
+        const int t = threadIdx.x, w = t >> 6, lane = lane_id(), first = w * I * 64 + lane;
+        const uint64_t lt = (lane == 0) ? 0ULL : (~0ULL >> (64 - lane));
+        uint32_t *mine = wcnt[w];
+#pragma unroll
+        for (int k = 0; k < 4; k++) mine[k * 64 + lane] = 0;
+        uint32_t rank[I];
+#pragma unroll
+        for (int r = 0; r < I; r++) {
+            const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
+            const uint64_t peers = digit_peers(d, true);
+            const uint32_t below = __popcll(peers & lt), old = mine[d];
+            rank[r] = old + below;
+            if (below == 0) mine[d] = old + __popcll(peers);
+        }
+        __syncthreads();
+        uint32_t c[kW], sum = 0;
+        if (t < 256)
+#pragma unroll
+            for (int k = 0; k < kW; k++) {
+                c[k] = wcnt[k][t];
+                sum += c[k];
+            }
+        uint32_t slot = scan256(sum, ws);
+        if (t < 256)
+#pragma unroll
+            for (int k = 0; k < kW; k++) {
+                wcnt[k][t] = slot;
+                slot += c[k];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < I; r++) {
+            const uint32_t at = mine[(key[r] >> shift) & 255u] + rank[r];
+            skey[at] = key[r];
+            sval[at] = val[r];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < I; r++) {
+            key[r] = skey[first + r * 64];
+            val[r] = sval[first + r * 64];
+        }
+    }
+
+    // n: real keys; the padding past them (all ones) sorts behind them.
+    __device__ __forceinline__ void sort(uint64_t (&key)[I], V (&val)[I], int n)
+    {
+        if (threadIdx.x == 0) nshort = nrun = toolong = 0;
+#pragma unroll 1
+        for (int shift = 32; shift < 64; shift += 8) pass(key, val, shift);
+        // (the counters' memory takes the list; a run has two keys or more)
+        uint16_t *starts = reinterpret_cast<uint16_t *>(&wcnt[0][0]);
+        static_assert(kN / 2 <= 2 * 256 * kW, "list of runs");
+        auto hi = [&](int i) { return (uint32_t)(skey[i] >> 32); };
+        for (int i = threadIdx.x; i < n - 1; i += T) {
+            const uint32_t h = hi(i), next = hi(i + 1), prev = i > 0 ? hi(i - 1) : ~h;
+            if (next == h && prev != h) starts[atomicAdd(&nshort, 1)] = (uint16_t)i;
+        }
+        __syncthreads();
+        // (the upper halves stay as they are while runs are being sorted)
+        const int nlist = nshort;
+        for (int q = threadIdx.x; q < nlist; q += T) {
+            const int i = starts[q];
+            const uint32_t h = hi(i);
+            int e = i + 2;
+            while (e < n && e - i <= kRunMax && hi(e) == h) e++;
+            if (e - i > kRunMax) {
+                int top = min(n, i + kRunWave + 1) + 1;    // (the keys are sorted by their upper halves)
+                while (top - e > 1) {
+                    const int mid = (e + top) >> 1;
+                    if (hi(mid - 1) == h) e = mid;
+                    else top = mid;
+                }
+                const int at = e - i > kRunWave ? kRunList : atomicAdd(&nrun, 1);
+                if (at < kRunList) runs[at] = (uint32_t)i | (uint32_t)(e - i) << 16;
+                else toolong = 1;
+                continue;
+            }
+            for (int k = i + 1; k < e; k++) {
+                const uint64_t x = skey[k];
+                const V v = sval[k];
+                int j = k;
+                for (; j > i && skey[j - 1] > x; j--) {
+                    skey[j] = skey[j - 1];
+                    sval[j] = sval[j - 1];
+                }
+                skey[j] = x;
+                sval[j] = v;
+            }
+        }
+        __syncthreads();
+        if (!toolong) {
+            constexpr int kPer = kRunWave / 64;
+            for (int q = threadIdx.x >> 6; q < nrun; q += kW) {
+                const int i = (int)(runs[q] & 0xffff), len = (int)(runs[q] >> 16);
+                uint64_t x[kPer];
+                V v[kPer];
+                int rank[kPer];
+#pragma unroll
+                for (int u = 0; u < kPer; u++) {
+                    const int at = u * 64 + lane_id();
+                    x[u] = at < len ? skey[i + at] : 0;
+                    v[u] = at < len ? sval[i + at] : 0;
+                    rank[u] = 0;
+                }
+                for (int j0 = 0; j0 < len; j0 += 8) {      // (eight loads in flight)
+                    uint64_t y[8];
+#pragma unroll
+                    for (int k = 0; k < 8; k++) y[k] = skey[i + min(j0 + k, len - 1)];
+#pragma unroll
+                    for (int u = 0; u < kPer; u++)
+                        if (64 * u < len)
+#pragma unroll
+                            for (int k = 0; k < 8; k++)
+                                rank[u] += j0 + k < len && (y[k] < x[u] || (y[k] == x[u] && j0 + k < u * 64 + lane_id()));
+                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+                for (int u = 0; u < kPer; u++)
+                    if (u * 64 + lane_id() < len) {
+                        skey[i + rank[u]] = x[u];
+                        sval[i + rank[u]] = v[u];
+                    }
+            }
+        } else {
+            const int first = (threadIdx.x >> 6) * I * 64 + lane_id();
+#pragma unroll
+            for (int r = 0; r < I; r++) {
+                key[r] = skey[first + r * 64];
+                val[r] = sval[first + r * 64];
+            }
+#pragma unroll 1
+            for (int shift = 0; shift < 64; shift += 8) pass(key, val, shift);
+        }
+        __syncthreads();
+    }
+};
+
+// Key of body i of a set of n (the padding past it sorts last): the Morton key
+// in the box b, with bit 63 for a massless body when mass is given.
+__device__ __forceinline__ uint64_t key_of(const double *__restrict__ pos, const double *__restrict__ mass, int64_t i,
+                                           int64_t n, const double4 &b, double4 *pk)
+{
+    if (i >= n) return ~0ULL;
+    const double x[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
+    const double m = mass ? mass[i] : 0.0;
+    if (pk) pk[i] = make_double4(x[0], x[1], x[2], m);
+    return morton_of(x, b) | (mass && m == 0.0 ? 1ULL << 63 : 0);
+}
+
+// Sorted tiles of kSortTile bodies: keys computed from the positions (and the
+// packed records pk written) or, pos null, read from keys.  boxi as in k_keys.
+__global__ __launch_bounds__(kSortTpb) void k_tile_sort(const double *__restrict__ pos, const double *__restrict__ mass,
+                                                        int64_t n, const double4 *__restrict__ box,
+                                                        const uint64_t *__restrict__ keys, uint64_t *kout, uint32_t *vout,
+                                                        double4 *pk, const int *__restrict__ boxi, unsigned long long *stat)
+{
+    __shared__ BlockSort<kSortTpb, kSortItems, uint32_t> S;
+    if (boxi && blockIdx.x == 0 && threadIdx.x == 0 && !boxi[5]) atomicOr(&stat[S_FLAGS], (unsigned long long)F_BOX_OPEN);
+    const int64_t base = (int64_t)blockIdx.x * kSortTile;
+    const int first = (threadIdx.x >> 6) * kSortItems * 64 + lane_id();
+    const double4 b = pos ? *box : make_double4(0, 0, 0, 1);
+    uint64_t key[kSortItems];
+    uint32_t val[kSortItems];
+#pragma unroll
+    for (int r = 0; r < kSortItems; r++) {
+        const int64_t i = base + first + r * 64;
+        val[r] = (uint32_t)i;
+        if (pos) key[r] = key_of(pos, mass, i, n, b, pk);
+        else key[r] = i < n ? keys[i] : ~0ULL;
+    }
+    S.sort(key, val, (int)min<int64_t>(kSortTile, n - base));
+    for (int j = threadIdx.x; j < kSortTile && base + j < n; j += kSortTpb) {
+        kout[base + j] = S.skey[j];
+        vout[base + j] = S.sval[j];
+    }
+}
+
+// One merge pass: pairs of sorted runs of `run` keys (the first run's key first
+// when equal) into runs of twice that.  A block writes kMergeTile outputs of
+// one pair; two waves find where they begin and end in the two runs by 64-way
+// searches, the block stages its keys in LDS and each thread merges
+// kMergeItems of them.
+constexpr int kMergeItems = 8, kMergeTile = kTpb * kMergeItems;
+static_assert(kSortTile % kMergeTile == 0, "an output tile lies in one pair of runs");
+
+__global__ __launch_bounds__(kTpb) void k_merge(const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
+                                                uint64_t *__restrict__ kout, uint32_t *__restrict__ vout, int64_t n,
+                                                int64_t run)
+{
+    __shared__ uint64_t sk[kMergeTile];
+    __shared__ uint32_t sv[kMergeTile];
+    __shared__ int cut[2];
+    const int64_t o0 = (int64_t)blockIdx.x * kMergeTile, base = o0 / (2 * run) * (2 * run);
+    const uint64_t *A = kin + base, *B = A + run;
+    const int na = (int)min(run, n - base), nb = (int)max<int64_t>(0, min(run, n - base - run));
+    const int d0 = (int)(o0 - base), d1 = min(d0 + kMergeTile, na + nb);
+    const int w = threadIdx.x >> 6, lane = lane_id();
+    if (w < 2) {
+        // keys of A among the first d of the merged pair
+        const int d = w ? d1 : d0;
+        int lo = max(0, d - nb), hi = min(d, na);
+        while (lo < hi) {
+            const int step = (hi - lo + 63) >> 6, mid = lo + lane * step;
+            const unsigned long long m = __ballot(mid < hi && A[min(mid, hi - 1)] <= B[d - 1 - min(mid, hi - 1)]);
+            const int c = __popcll(m);         // the first c probes hold
+            const int l = c ? lo + (c - 1) * step + 1 : lo;
+            hi = min(hi, lo + c * step);
+            lo = min(l, hi);
+        }
+        if (lane == 0) cut[w] = lo;
+    }
+    __syncthreads();
+    const int a0 = cut[0], a1 = cut[1], b0 = d0 - a0, ca = a1 - a0, tot = d1 - d0;
+    for (int j = threadIdx.x; j < tot; j += kTpb) {
+        const int64_t src = base + (j < ca ? a0 + j : run + b0 + (j - ca));
+        sk[j] = kin[src];
+        sv[j] = vin[src];
+    }
+    __syncthreads();
+    const int cb = tot - ca, d = min((int)threadIdx.x * kMergeItems, tot);
+    int lo = max(0, d - cb), hi = min(d, ca);
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (sk[mid] <= sk[ca + d - 1 - mid]) lo = mid + 1;
+        else hi = mid;
+    }
+    int ia = lo, ib = ca + d - lo;
+    uint64_t ka = ia < ca ? sk[ia] : 0, kb = ib < tot ? sk[ib] : 0;
+#pragma unroll
+    for (int k = 0; k < kMergeItems; k++) {
+        if (d + k >= tot) break;
+        const bool fromA = ib >= tot || (ia < ca && ka <= kb);
+        const int at = fromA ? ia : ib;
+        kout[o0 + d + k] = fromA ? ka : kb;
+        vout[o0 + d + k] = sv[at];
+        if (fromA) {
+            ia++;
+            ka = ia < ca ? sk[ia] : 0;
+        } else {
+            ib++;
+            kb = ib < tot ? sk[ib] : 0;
+        }
+    }
+}
+
 // ---- gather sorted bodies ----------------------------------------------------
 
 __device__ __forceinline__ void split2(double x, float &hi, float &lo)
@@ -688,7 +1104,7 @@ __global__ void k_gather_test(const uint32_t *__restrict__ perm, int64_t nt, con
     l.w = 0.f;
     thi[s] = h;
     tlo[s] = l;
-    td[s] = make_double4(x, y, z, 0.0);
+    if (td) td[s] = make_double4(x, y, z, 0.0);
     const int b = tmap ? tmap[o] : -1;
     tself[s] = b;
     if (b >= 0) tinv[b] = (int)s;
@@ -704,64 +1120,141 @@ __global__ void k_tree_index(const uint32_t *__restrict__ vs, int64_t n, int nb,
 
 // ---- topology ----------------------------------------------------------------
 
-// cpl and its copy cq = cpl + 1 (0..22, for the 8-entry range scans).
-__global__ void k_cpl(const uint64_t *__restrict__ keys, int nb, int8_t *cpl, uint8_t *cq, uint32_t *ccnt)
-{
-    for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < nb; s += gridDim.x * blockDim.x) {
-        int c = -1, cp = -1;
-        if (s + 1 < nb) c = min(kMaxLevel, (__clzll(keys[s] ^ keys[s + 1]) - 1) / 3);
-        if (s > 0) cp = min(kMaxLevel, (__clzll(keys[s - 1] ^ keys[s]) - 1) / 3);
-        cpl[s] = (int8_t)c;
-        cq[s] = (uint8_t)(c + 1);
-        ccnt[s] = (uint32_t)max(0, c - cp);
-    }
-}
-
-// Cells needed = cbase[n]; the count used is clamped to the capacity and an
+// Cells needed (raw); the count used is clamped to the capacity and an
 // overflow is flagged (the host then grows the arrays and evaluates again).
 struct CellClamp {
-    const uint32_t *cbase;
-    int n;
     unsigned long long cap;
     unsigned long long *stat;
     int slot, slot_raw;
     unsigned long long flag;
 };
 
-__device__ __forceinline__ void clamp_cells(const CellClamp &c)
+__device__ __forceinline__ void clamp_cells(const CellClamp &c, unsigned long long raw)
 {
-    const unsigned long long raw = c.n >= 2 ? c.cbase[c.n] : 0;
     c.stat[c.slot_raw] = raw;
     c.stat[c.slot] = raw < c.cap ? raw : c.cap;
     if (raw > c.cap) atomicOr(&c.stat[S_FLAGS], c.flag);
 }
 
-// Block minima over 64 entries of a byte array in the cq domain (cpl + 1,
-// values 0..22): level 1 over cq, levels 2 and 3 over the level below, for
-// the range-end search.
-// out[b] = min of in[64 b .. 64 b + 63] (entries past nin ignored): eight
-// lanes per output, one 8-byte load each (in is 8-byte aligned), then a min
-// across the eight.  Launch with 8 * nout threads.  cc (first pyramid level
-// only): thread 0 also sets the cell count.
-__global__ void k_cmin(const uint8_t *__restrict__ in, int nin, uint8_t *out, int nout, CellClamp cc = CellClamp{})
+// Per body: cpl, its copy cq = cpl + 1 (0..22, for the 8-entry range scans),
+// the count of cells that start there, and the sums and minima above them:
+// part[b] the cells of block b's kScanChunk bodies, m1 and m2 the minima of cq
+// over 64 and 4096 entries (a wave's round and the block; the range-end search
+// reads them).  One pass over the keys in the place of four launches.
+static_assert(kScanChunk == 4096, "a block's bodies are one m2 entry");
+__global__ __launch_bounds__(kTpb) void k_cpl(const uint64_t *__restrict__ keys, int nb, int8_t *cpl, uint8_t *cq,
+                                              uint32_t *ccnt, uint32_t *part, uint8_t *m1, uint8_t *m2)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (cc.stat && t == 0) clamp_cells(cc);
-    const int b = t >> 3, lo = b * 64 + 8 * (t & 7);
-    int m = 255;
-    if (b < nout) {
-        if (lo + 8 <= nin) {
-            const uint64_t w = *reinterpret_cast<const uint64_t *>(in + lo);
+    __shared__ int wmin[kTpb / 64];
+    const int lane = lane_id(), w = threadIdx.x >> 6;
+    const int base = blockIdx.x * kScanChunk + (int)threadIdx.x;
+    uint64_t key[kScanItems], edge[kScanItems];
 #pragma unroll
-            for (int j = 0; j < 8; j++) m = min(m, (int)((w >> (8 * j)) & 255));
-        } else {
-            for (int j = lo; j < nin; j++) m = min(m, (int)in[j]);
-        }
+    for (int r = 0; r < kScanItems; r++) {
+        const int i = base + r * kTpb;
+        key[r] = i < nb ? keys[i] : 0;
+        // lane 0 also needs the key before the wave's, lane 63 the one after
+        const int j = lane == 0 ? i - 1 : i + 1;
+        edge[r] = (lane == 0 || lane == 63) && j >= 0 && j < nb ? keys[j] : 0;
     }
-    m = min(m, __shfl_xor(m, 1, 64));
-    m = min(m, __shfl_xor(m, 2, 64));
-    m = min(m, __shfl_xor(m, 4, 64));
-    if (b < nout && (t & 7) == 0) out[b] = (uint8_t)m;
+    uint32_t sum = 0;
+    int low = 255;
+#pragma unroll
+    for (int r = 0; r < kScanItems; r++) {
+        const int i = base + r * kTpb;
+        const uint64_t after = __shfl_down(key[r], 1, 64);
+        int c = -1;
+        if (i + 1 < nb) c = min(kMaxLevel, (__clzll(key[r] ^ (lane == 63 ? edge[r] : after)) - 1) / 3);
+        int cp = __shfl_up(c, 1, 64);
+        if (lane == 0) cp = i > 0 ? min(kMaxLevel, (__clzll(edge[r] ^ key[r]) - 1) / 3) : -1;
+        const uint32_t n = (uint32_t)max(0, c - cp);
+        int m = i < nb ? c + 1 : 255;
+        if (i < nb) {
+            cpl[i] = (int8_t)c;
+            cq[i] = (uint8_t)(c + 1);
+            ccnt[i] = n;
+            sum += n;
+        }
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) m = min(m, __shfl_xor(m, d, 64));
+        if (lane == 0 && i < nb) m1[i >> 6] = (uint8_t)m;
+        low = min(low, m);
+    }
+    if (lane == 0) wmin[w] = low;
+    uint32_t tot;
+    block_excl_scan(sum, &tot);
+    if (threadIdx.x == 0) {
+        part[blockIdx.x] = tot;
+#pragma unroll
+        for (int k = 1; k < kTpb / 64; k++) low = min(low, wmin[k]);
+        m2[blockIdx.x] = (uint8_t)low;
+    }
+}
+
+// Sum of v[0 .. n) over the block (every thread gets it).
+__device__ __forceinline__ uint32_t block_sum(const uint32_t *__restrict__ v, int n)
+{
+    uint32_t x = 0;
+    for (int i = threadIdx.x; i < n; i += kTpb) x += v[i];
+    uint32_t tot;
+    block_excl_scan(x, &tot);
+    return tot;
+}
+
+// cbase: exclusive scan of ccnt from the blocks' sums (scanned: part holds
+// their exclusive scan already, else each block adds up those before it).  The
+// last block stores the total and sets the cell count; block 0 forms the
+// third minima level (m3, 262144 bodies per entry).
+__global__ __launch_bounds__(kTpb) void k_cbase(const uint32_t *__restrict__ ccnt, uint32_t *__restrict__ cbase, int n,
+                                                const uint32_t *__restrict__ part, bool scanned,
+                                                const uint8_t *__restrict__ m2, int n2, uint8_t *m3, CellClamp cc)
+{
+    const uint32_t before = scanned ? part[blockIdx.x] : block_sum(part, blockIdx.x);
+    const int64_t mine = (int64_t)blockIdx.x * kScanChunk + (int64_t)threadIdx.x * kScanItems;
+    const bool full = mine + kScanItems <= n;      // (ccnt and cbase are 16-byte aligned)
+    uint32_t v[kScanItems], s = 0;
+    if (full) {
+#pragma unroll
+        for (int r = 0; r < kScanItems / 4; r++) {
+            const uint4 q = reinterpret_cast<const uint4 *>(ccnt + mine)[r];
+            v[4 * r] = q.x;
+            v[4 * r + 1] = q.y;
+            v[4 * r + 2] = q.z;
+            v[4 * r + 3] = q.w;
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < kScanItems; r++) v[r] = mine + r < n ? ccnt[mine + r] : 0;
+    }
+#pragma unroll
+    for (int r = 0; r < kScanItems; r++) s += v[r];
+    uint32_t tot;
+    uint32_t ex = before + block_excl_scan(s, &tot);
+    uint32_t o[kScanItems];
+#pragma unroll
+    for (int r = 0; r < kScanItems; r++) {
+        o[r] = ex;
+        ex += v[r];
+    }
+    if (full) {
+#pragma unroll
+        for (int r = 0; r < kScanItems / 4; r++)
+            reinterpret_cast<uint4 *>(cbase + mine)[r] = make_uint4(o[4 * r], o[4 * r + 1], o[4 * r + 2], o[4 * r + 3]);
+    } else {
+#pragma unroll
+        for (int r = 0; r < kScanItems; r++)
+            if (mine + r < n) cbase[mine + r] = o[r];
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        cbase[n] = before + tot;
+        clamp_cells(cc, before + tot);
+    }
+    if (blockIdx.x == 0)
+        for (int j = threadIdx.x; 64 * j < n2; j += kTpb) {
+            int m = 255;
+            for (int k = 64 * j; k < min(n2, 64 * j + 64); k++) m = min(m, (int)m2[k]);
+            m3[j] = (uint8_t)m;
+        }
 }
 
 // Flags (the high bit of a byte) of the entries k, k+1, .. of the aligned
@@ -816,60 +1309,236 @@ __device__ int range_end(const uint8_t *__restrict__ cq, const uint8_t *__restri
     }
 }
 
-// Owner body of every cell: body s starts the cells cbase[s] .. cbase[s+1]-1.
-__global__ void k_owner(const uint32_t *__restrict__ cbase, int nb, const unsigned long long *ncellp, int *owner)
-{
-    const int ncell = (int)*ncellp;
-    for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < nb; s += gridDim.x * blockDim.x) {
-        const int id1 = min((int)cbase[s + 1], ncell);
-        for (int id = (int)cbase[s]; id < id1; id++) owner[id] = s;
-    }
-}
+// The whole front of a small build in one block (n <= T * I): BOX: the start of
+// the build and expandbox; then keys, sort and, for nb >= 2 bodies in the tree,
+// the cells (what k_cpl, k_cbase and k_cells compute).  At these sizes every
+// step of the general path is a launch of ~3 us of work (35 launches with the
+// radix passes, 0.2 ms).
+constexpr int kSmallTpb = 1024;
+template <int I>
+struct SmallFront {
+    BlockSort<kSmallTpb, I, uint16_t> S;
+    // cpl + 1 and its minima, read eight entries at a time (range_end)
+    __attribute__((aligned(8))) uint8_t cq[kSmallTpb * I + 64];
+    __attribute__((aligned(8))) uint8_t m1[kSmallTpb * I / 64 + 8];
+    __attribute__((aligned(8))) uint8_t m2[16], m3[16];
+    uint32_t wsum[kSmallTpb / 64];
+    BoxPick pick;
+};
 
-// One thread per cell (grid-stride over the device cell count).  The cells
-// that start at body s are the levels cpl[s-1]+1 .. cpl[s] with ids from
-// cbase[s]; the range of a cell of level L ends before the first j >= s with
-// cpl[j] < L.
-__global__ void k_cells(const int8_t *__restrict__ cpl, const uint8_t *__restrict__ cq, const uint32_t *__restrict__ cbase,
-                        const int *__restrict__ owner,
-                        const uint8_t *__restrict__ m1, const uint8_t *__restrict__ m2, const uint8_t *__restrict__ m3,
-                        const unsigned long long *ncellp, int *cfirst, int *clast, uint8_t *clevel, int *cskip,
-                        int *pre, int2 *fnb, unsigned long long *deep)
+struct FrontOut {
+    uint64_t *keys;
+    uint32_t *vals;
+    int8_t *cpl;
+    uint32_t *cbase;
+    int *first, *last;
+    uint8_t *level;
+    int *skip, *pre;        // null for a separate test set, as in k_cells
+    int2 *fnb;
+    unsigned long long *deep;
+};
+
+template <int I, bool BOX>
+__global__ __launch_bounds__(kSmallTpb) void k_front(const double *__restrict__ pos, const double *__restrict__ mass, int n,
+                                                     int nb, BoxStart st, int rounds, double4 *box,
+                                                     unsigned long long *stat, int nzero, uint32_t *lwork, int nlwork,
+                                                     FrontOut out, CellClamp cc)
 {
-    const int ncell = (int)*ncellp;
-    const int stride = gridDim.x * blockDim.x;
-    for (int base = blockIdx.x * blockDim.x; base < ncell; base += stride) {
-        const int id = base + threadIdx.x;
+    __shared__ SmallFront<I> M;
+    const int t = threadIdx.x, w = t >> 6, lane = lane_id(), first = w * I * 64 + lane;
+    uint64_t key[I];
+    uint16_t val[I];
+    if (BOX) {
+        build_start(stat, nzero, lwork, nlwork);
+        __syncthreads();
+        double x[I][3];
+        unsigned mask = 0;
+#pragma unroll
+        for (int r = 0; r < I; r++) {
+            const int i = min(first + r * 64, n - 1);
+            if (first + r * 64 < n && mass[i] != 0.0) mask |= 1u << r;
+#pragma unroll
+            for (int k = 0; k < 3; k++) x[r][k] = pos[3 * i + k];
+        }
+        double4 b = st.keep ? *box : make_double4(st.rx, st.ry, st.rz, st.rsize);
+        const bool closed = box_rounds<kSmallTpb, I>(x, mask, first, b, rounds, M.pick, stat);
+        if (t == 0) {
+            *box = b;
+            if (!closed) atomicOr(&stat[S_FLAGS], (unsigned long long)F_BOX_OPEN);
+        }
+#pragma unroll
+        for (int r = 0; r < I; r++) {
+            val[r] = (uint16_t)(first + r * 64);
+            key[r] = first + r * 64 < n ? morton_of(x[r], b) | (mask >> r & 1u ? 0 : 1ULL << 63) : ~0ULL;
+        }
+    } else {
+        const double4 b = *box;
+#pragma unroll
+        for (int r = 0; r < I; r++) {
+            val[r] = (uint16_t)(first + r * 64);
+            key[r] = key_of(pos, mass, first + r * 64, n, b, nullptr);
+        }
+    }
+    M.S.sort(key, val, n);
+    for (int j = t; j < n; j += kSmallTpb) {
+        out.keys[j] = M.S.skey[j];
+        out.vals[j] = M.S.sval[j];
+    }
+    if (nb < 2) return;
+    // thread t: the bodies t I .. t I + I - 1
+    uint32_t cnt[I], sum = 0;
+    int cp = -1;
+    if (t * I > 0 && t * I < nb)
+        cp = min(kMaxLevel, (__clzll(M.S.skey[t * I - 1] ^ M.S.skey[t * I]) - 1) / 3);
+#pragma unroll
+    for (int r = 0; r < I; r++) {
+        const int j = t * I + r;
+        int c = -1;
+        if (j + 1 < nb) c = min(kMaxLevel, (__clzll(M.S.skey[j] ^ M.S.skey[j + 1]) - 1) / 3);
+        cnt[r] = j < nb ? (uint32_t)max(0, c - cp) : 0;
+        sum += cnt[r];
+        M.cq[j] = j < nb ? (uint8_t)(c + 1) : 255;
+        if (j < nb) out.cpl[j] = (int8_t)c;
+        cp = c;
+    }
+    const uint32_t incl = wave_incl_scan(sum);
+    if (lane == 63) M.wsum[w] = incl;
+    __syncthreads();
+    uint32_t base = incl - sum, tot = 0;
+#pragma unroll
+    for (int k = 0; k < kSmallTpb / 64; k++) {
+        if (k < w) base += M.wsum[k];
+        tot += M.wsum[k];
+    }
+    // the keys are written: their LDS takes the cell numbers and, behind them,
+    // the body of each cell (kOwn of them; sets with more cells find it by a
+    // search)
+    constexpr int kAll = kSmallTpb * I, kOwn = 2 * kAll - 8;
+    uint32_t *cb = reinterpret_cast<uint32_t *>(M.S.skey);
+    uint16_t *own = reinterpret_cast<uint16_t *>(cb + kAll + 4);
+#pragma unroll
+    for (int r = 0; r < I; r++) {
+        const int j = t * I + r;
+        if (j < nb) {
+            out.cbase[j] = base;
+            cb[j] = base;
+            for (uint32_t k = base; k < min(base + cnt[r], (uint32_t)kOwn); k++) own[k] = (uint16_t)j;
+        }
+        base += cnt[r];
+    }
+    // minima over 64, 4096 and all (at most 262144) entries; those past nb are 255
+    constexpr int kM1 = kAll / 64, kM2 = (kAll + 4095) / 4096;
+    for (int k = t; k < 8 * kM1; k += kSmallTpb) {      // eight lanes per entry
+        const uint64_t q = *reinterpret_cast<const uint64_t *>(M.cq + 8 * k);
+        int m = 255;
+#pragma unroll
+        for (int u = 0; u < 8; u++) m = min(m, (int)(q >> (8 * u) & 255));
+#pragma unroll
+        for (int d = 4; d >= 1; d >>= 1) m = min(m, __shfl_xor(m, d, 64));
+        if ((k & 7) == 0) M.m1[k >> 3] = (uint8_t)m;
+    }
+    __syncthreads();
+    if (t < kM2) {
+        int m = 255;
+        for (int k = 64 * t; k < min(64 * t + 64, kM1); k++) m = min(m, (int)M.m1[k]);
+        M.m2[t] = (uint8_t)m;
+    }
+    if (t == 0) {
+        out.cbase[nb] = tot;
+        cb[nb] = tot;
+        M.m3[0] = 0;               // (one entry: the search below it always looks closer)
+        clamp_cells(cc, tot);
+    }
+    __syncthreads();
+    const int ncell = (int)min((unsigned long long)tot, cc.cap);
+    if (out.pre)
+        for (int s = t; s < nb; s += kSmallTpb)
+            if ((int)cb[s + 1] <= ncell) out.pre[s + cb[s + 1]] = s;
+    for (int id0 = 0; id0 < ncell; id0 += kSmallTpb) {
+        const int id = id0 + t;
         bool isdeep = false;
         if (id < ncell) {
-            const int s = owner[id];
-            const int l0 = (s > 0 ? cpl[s - 1] : -1) + 1;
-            const int L = l0 + (id - (int)cbase[s]);
-            const int e = range_end(cq, m1, m2, m3, s, L);
-            cfirst[id] = s;
-            clast[id] = e;
-            clevel[id] = (uint8_t)L;
-            if (cskip) cskip[id] = (e + 1) + (int)cbase[e + 1];
-            if (fnb) fnb[id] = make_int2(s, e - s + 1);
-            if (pre) pre[s + id] = ~id;
+            int s;
+            if (id < kOwn) {
+                s = own[id];
+            } else {
+                int lo = 0, hi = nb;               // last body with cb <= id
+                while (hi - lo > 1) {
+                    const int mid = (lo + hi) >> 1;
+                    if ((int)cb[mid] <= id) lo = mid;
+                    else hi = mid;
+                }
+                s = lo;
+            }
+            // (cq = cpl + 1)
+            const int L = (s > 0 ? (int)M.cq[s - 1] : 0) + (id - (int)cb[s]);
+            const int e = range_end(M.cq, M.m1, M.m2, M.m3, s, L);
+            out.first[id] = s;
+            out.last[id] = e;
+            out.level[id] = (uint8_t)L;
+            if (out.skip) out.skip[id] = (e + 1) + (int)cb[e + 1];
+            if (out.fnb) out.fnb[id] = make_int2(s, e - s + 1);
+            if (out.pre) out.pre[s + id] = ~id;
             isdeep = L == kMaxLevel;
         }
         const unsigned long long m = __ballot(isdeep);
-        if (deep && m && lane_id() == 0) atomicAdd(deep, (unsigned long long)__popcll(m));
+        if (out.deep && m && lane == 0) atomicAdd(out.deep, (unsigned long long)__popcll(m));
     }
 }
 
-// Pre-order position of body s: after the cells that start at s.
-__global__ void k_body_pre(const uint32_t *__restrict__ cbase, int nb, const unsigned long long *ncellp, int *pre)
+// Every cell and the pre-order places of the bodies.  A block takes kCellBodies
+// bodies (grid-stride); the cells that start at body s are the levels cpl[s-1]+1
+// .. cpl[s] with ids from cbase[s], so the block's cells are consecutive: each
+// body writes its place at its first cell in LDS, a cell's body is the last
+// such place before it, and the cells are then taken one per thread (about half
+// as many as bodies).  The range of a cell of level L ends before the first j >=
+// s with cpl[j] < L.  A body's pre-order position follows the cells that start
+// at it.
+constexpr int kCellPer = 2, kCellBodies = kTpb * kCellPer;
+
+__global__ __launch_bounds__(kTpb) void k_cells(const int8_t *__restrict__ cpl, const uint8_t *__restrict__ cq,
+                                                const uint32_t *__restrict__ cbase, int nb, const uint8_t *__restrict__ m1,
+                                                const uint8_t *__restrict__ m2, const uint8_t *__restrict__ m3,
+                                                const unsigned long long *ncellp, int *cfirst, int *clast,
+                                                uint8_t *clevel, int *cskip, int *pre, int2 *fnb, unsigned long long *deep)
 {
-    const uint32_t ncell = (uint32_t)*ncellp;
-    for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < nb; s += gridDim.x * blockDim.x)
-        if (cbase[s + 1] <= ncell) pre[s + cbase[s + 1]] = s;
+    __shared__ unsigned short own[kCellBodies * (kMaxLevel + 1)];   // body of each cell of the block
+    const int ncell = (int)*ncellp;
+    for (int s0 = blockIdx.x * kCellBodies; s0 < nb; s0 += gridDim.x * kCellBodies) {
+        const int first = (int)cbase[s0], end = min(ncell, (int)cbase[min(nb, s0 + kCellBodies)]);
+#pragma unroll
+        for (int k = 0; k < kCellPer; k++) {
+            const int j = k * kTpb + (int)threadIdx.x, s = s0 + j;
+            if (s < nb) {
+                const int c0 = (int)cbase[s], c1 = (int)cbase[s + 1];
+                if (pre && c1 <= ncell) pre[s + c1] = s;
+                for (int c = c0; c < c1; c++) own[c - first] = (unsigned short)j;
+            }
+        }
+        __syncthreads();
+        for (int id0 = first; id0 < end; id0 += kTpb) {
+            const int id = id0 + (int)threadIdx.x;
+            bool isdeep = false;
+            if (id < end) {
+                const int s = s0 + own[id - first];
+                const int L = (s > 0 ? cpl[s - 1] : -1) + 1 + (id - (int)cbase[s]);
+                const int e = range_end(cq, m1, m2, m3, s, L);
+                cfirst[id] = s;
+                clast[id] = e;
+                clevel[id] = (uint8_t)L;
+                if (cskip) cskip[id] = (e + 1) + (int)cbase[e + 1];
+                if (fnb) fnb[id] = make_int2(s, e - s + 1);
+                if (pre) pre[s + id] = ~id;
+                isdeep = L == kMaxLevel;
+            }
+            const unsigned long long m = __ballot(isdeep);
+            if (deep && m && lane_id() == 0) atomicAdd(deep, (unsigned long long)__popcll(m));
+        }
+        __syncthreads();
+    }
 }
 
 __global__ void k_set_int(int *p, int v) { *p = v; }
-
-__global__ void k_copy_count(const uint32_t *src, unsigned long long *dst) { *dst = *src; }
 
 // Fixed-size groups of consecutive points (sets too small to need a topology).
 __global__ void k_groups_trivial(int64_t n, int G, int *gfirst, int *gcount, unsigned long long *stat)
@@ -933,7 +1602,7 @@ template <bool WRITE>
 __device__ uint32_t pack_groups(int c, const uint64_t *__restrict__ keys, const int8_t *__restrict__ cpl,
                                 const uint32_t *__restrict__ cbase, const int *__restrict__ cfirst,
                                 const int *__restrict__ clast, const uint8_t *__restrict__ clevel, int G, int lsys,
-                                int ncell, const int *__restrict__ csub, const int2 *__restrict__ fnb, int *gfirst,
+                                int ncell, const int *kids, const int2 *__restrict__ fnb, int *gfirst,
                                 int *gcount, uint32_t off)
 {
     int s, e;
@@ -1005,15 +1674,12 @@ __device__ uint32_t pack_groups(int c, const uint64_t *__restrict__ keys, const 
             }
         }
     };
-    if (csub) {
-        // children from the tree's child slots: (first point, count) per octant
-        const int4 s0 = reinterpret_cast<const int4 *>(csub)[2 * (int64_t)c];
-        const int4 s1 = reinterpret_cast<const int4 *>(csub)[2 * (int64_t)c + 1];
-        const int r[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+    if (fnb) {
+        // children from the tree's child slots (kids): (first point, count) per octant
         int2 f[8];
 #pragma unroll
         for (int o = 0; o < 8; o++)
-            f[o] = r[o] == kNoChild ? make_int2(0, 0) : (r[o] >= 0 ? make_int2(r[o], 1) : fnb[~r[o]]);
+            f[o] = kids[o] == kNoChild ? make_int2(0, 0) : (kids[o] >= 0 ? make_int2(kids[o], 1) : fnb[~kids[o]]);
 #pragma unroll
         for (int o = 0; o < 8; o++)
             if (f[o].y > G) big |= 1u << o;
@@ -1038,31 +1704,6 @@ __device__ uint32_t pack_groups(int c, const uint64_t *__restrict__ keys, const 
     return k;
 }
 
-__global__ void k_group_count(const uint64_t *__restrict__ keys, const int8_t *__restrict__ cpl,
-                              const uint32_t *__restrict__ cbase,
-                              const int *__restrict__ cfirst, const int *__restrict__ clast,
-                              const uint8_t *__restrict__ clevel, const unsigned long long *ncellp, int G,
-                              int lsys, const int *__restrict__ csub, const int2 *__restrict__ fnb, uint32_t *gcnt)
-{
-    const int ncell = (int)*ncellp;
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncell; c += gridDim.x * blockDim.x)
-        gcnt[c] = pack_groups<false>(c, keys, cpl, cbase, cfirst, clast, clevel, G, lsys, ncell, csub, fnb, nullptr,
-                                     nullptr, 0);
-}
-
-__global__ void k_group_write(const uint64_t *__restrict__ keys, const int8_t *__restrict__ cpl,
-                              const uint32_t *__restrict__ cbase,
-                              const int *__restrict__ cfirst, const int *__restrict__ clast,
-                              const uint8_t *__restrict__ clevel, const unsigned long long *ncellp, int G, int lsys,
-                              const int *__restrict__ csub, const int2 *__restrict__ fnb,
-                              const uint32_t *__restrict__ goff, int *gfirst, int *gcount)
-{
-    const int ncell = (int)*ncellp;
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncell; c += gridDim.x * blockDim.x)
-        pack_groups<true>(c, keys, cpl, cbase, cfirst, clast, clevel, G, lsys, ncell, csub, fnb, gfirst, gcount,
-                          goff[c]);
-}
-
 // Walk roots of a batch: the system's root cell (the cell at the first
 // spatial level, lsys) or, for a one-body system, that body.
 __global__ void k_sysroot_init(const int64_t *__restrict__ off, int nsys, int *root)
@@ -1080,53 +1721,105 @@ __global__ void k_sysroot_cells(const uint8_t *__restrict__ clevel, const int *_
     root[s] = ~c;
 }
 
-// Children of each cell in octant order; parent links; child-cell counts.
-__device__ void children_of(int c, const uint64_t *__restrict__ keys, const int8_t *__restrict__ cpl,
-                            const uint32_t *__restrict__ cbase, const int *__restrict__ cfirst,
-                            const int *__restrict__ clast, const uint8_t *__restrict__ clevel, int ncell, int *csub,
-                            int *cnkids);
-
-__global__ void k_children(const uint64_t *__restrict__ keys, const int8_t *__restrict__ cpl,
-                           const uint32_t *__restrict__ cbase, const int *__restrict__ cfirst,
-                           const int *__restrict__ clast, const uint8_t *__restrict__ clevel,
-                           const unsigned long long *ncellp, int *csub, int *cnkids)
+// Children of cell c in octant order (r[8]); returns the entries pushed when it
+// is opened.
+__device__ __forceinline__ int children_of(int c, int s, int e, int L, const uint64_t *__restrict__ keys,
+                                           const int8_t *__restrict__ cpl, const uint32_t *__restrict__ cbase,
+                                           const int *__restrict__ clast, int ncell, int *r)
 {
-    const int ncell = (int)*ncellp;
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncell; c += gridDim.x * blockDim.x)
-        children_of(c, keys, cpl, cbase, cfirst, clast, clevel, ncell, csub, cnkids);
-}
-
-__device__ void children_of(int c, const uint64_t *__restrict__ keys, const int8_t *__restrict__ cpl,
-                            const uint32_t *__restrict__ cbase, const int *__restrict__ cfirst,
-                            const int *__restrict__ clast, const uint8_t *__restrict__ clevel, int ncell, int *csub,
-                            int *cnkids)
-{
-    int s = cfirst[c], e = clast[c], L = clevel[c];
-    int r[8];
 #pragma unroll
     for (int o = 0; o < 8; o++) r[o] = kNoChild;
+    if (L == kMaxLevel) return e - s + 1;        // bucket: bodies s..e are the children
+    const int shift = 60 - 3 * L;                // octant digit of level L+1
     int nk = 0;
-    if (L == kMaxLevel) {            // bucket: bodies s..e are the children
-        nk = e - s + 1;
-    } else {
-        const int shift = 60 - 3 * L;    // octant digit of level L+1
-        int t = s;
-        while (t <= e) {
-            const int o = (int)((keys[t] >> shift) & 7);
-            int cc;
-            const int tn = child_end(c, s, e, t, L, cpl, cbase, clast, ncell, &cc);
-            const int ref = cc >= 0 ? ~cc : t;
+    for (int t = s; t <= e;) {
+        const int o = (int)((keys[t] >> shift) & 7);
+        int cc;
+        const int tn = child_end(c, s, e, t, L, cpl, cbase, clast, ncell, &cc);
+        const int ref = cc >= 0 ? ~cc : t;
 #pragma unroll
-            for (int k = 0; k < 8; k++)
-                if (k == o) r[k] = ref;
-            t = tn;
-            nk++;
+        for (int k = 0; k < 8; k++)
+            if (k == o) r[k] = ref;
+        t = tn;
+        nk++;
+    }
+    return nk;
+}
+
+// Child slots of every cell (KIDS) and the number of groups it emits (gcnt,
+// when not null: groups of at most G points), with the sums of gcnt over
+// kGroupChunk cells (gpart) for k_group_write's offsets.  fnb: the tree's body
+// ranges when the groups are cut from its child slots, else null.
+constexpr int kGroupChunk = kTpb;
+
+template <bool KIDS>
+__global__ __launch_bounds__(kTpb) void k_children(const uint64_t *__restrict__ keys, const int8_t *__restrict__ cpl,
+                                                   const uint32_t *__restrict__ cbase, const int *__restrict__ cfirst,
+                                                   const int *__restrict__ clast, const uint8_t *__restrict__ clevel,
+                                                   const unsigned long long *ncellp, int *csub, int *cnkids, int G,
+                                                   int lsys, const int2 *__restrict__ fnb, uint32_t *gcnt,
+                                                   uint32_t *gpart)
+{
+    const int ncell = (int)*ncellp;
+    for (int chunk = blockIdx.x; chunk * kGroupChunk < ncell; chunk += gridDim.x) {
+        uint32_t mine = 0;
+        const int c = chunk * kGroupChunk + (int)threadIdx.x;
+        if (c < ncell) {
+            int r[8];
+            if (KIDS) {
+                const int s = cfirst[c], e = clast[c], L = clevel[c];
+                const int nk = children_of(c, s, e, L, keys, cpl, cbase, clast, ncell, r);
+                int4 *sub = reinterpret_cast<int4 *>(csub + 8 * (int64_t)c);
+                sub[0] = make_int4(r[0], r[1], r[2], r[3]);
+                sub[1] = make_int4(r[4], r[5], r[6], r[7]);
+                cnkids[c] = nk;
+            }
+            if (gcnt) {
+                mine = pack_groups<false>(c, keys, cpl, cbase, cfirst, clast, clevel, G, lsys, ncell, r, fnb, nullptr,
+                                          nullptr, 0);
+                gcnt[c] = mine;
+            }
+        }
+        if (gcnt) {
+            uint32_t tot;
+            block_excl_scan(mine, &tot);
+            if (threadIdx.x == 0) gpart[chunk] = tot;
         }
     }
-    int4 *sub = reinterpret_cast<int4 *>(csub + 8 * (int64_t)c);
-    sub[0] = make_int4(r[0], r[1], r[2], r[3]);
-    sub[1] = make_int4(r[4], r[5], r[6], r[7]);
-    cnkids[c] = nk;
+}
+
+// Writes the groups in cell order: a chunk's offset is the sum of the chunks
+// before it (each block adds them up), a cell's the scan inside the chunk.
+__global__ __launch_bounds__(kTpb) void k_group_write(const uint64_t *__restrict__ keys, const int8_t *__restrict__ cpl,
+                                                      const uint32_t *__restrict__ cbase, const int *__restrict__ cfirst,
+                                                      const int *__restrict__ clast, const uint8_t *__restrict__ clevel,
+                                                      const unsigned long long *ncellp, int G, int lsys,
+                                                      const int *__restrict__ csub, const int2 *__restrict__ fnb,
+                                                      const uint32_t *__restrict__ gcnt, const uint32_t *__restrict__ gpart,
+                                                      int *gfirst, int *gcount, unsigned long long *stat)
+{
+    const int ncell = (int)*ncellp;
+    for (int chunk = blockIdx.x; chunk * kGroupChunk < ncell; chunk += gridDim.x) {
+        const bool last = (chunk + 1) * kGroupChunk >= ncell;
+        const uint32_t here = gpart[chunk];
+        if (!here && !last) continue;
+        uint32_t off = block_sum(gpart, chunk);
+        if (last && threadIdx.x == 0) stat[S_NGROUPS] = off + here;
+        if (!here) continue;
+        const int c = chunk * kGroupChunk + (int)threadIdx.x;
+        const uint32_t n = c < ncell ? gcnt[c] : 0;
+        uint32_t tot;
+        off += block_excl_scan(n, &tot);
+        if (!n) continue;
+        int r[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (csub) {
+            const int4 s0 = reinterpret_cast<const int4 *>(csub)[2 * (int64_t)c];
+            const int4 s1 = reinterpret_cast<const int4 *>(csub)[2 * (int64_t)c + 1];
+            r[0] = s0.x; r[1] = s0.y; r[2] = s0.z; r[3] = s0.w;
+            r[4] = s1.x; r[5] = s1.y; r[6] = s1.z; r[7] = s1.w;
+        }
+        pack_groups<true>(c, keys, cpl, cbase, cfirst, clast, clevel, G, lsys, ncell, r, fnb, gfirst, gcount, off);
+    }
 }
 
 // Moments of cell c from its children's (computed before it: the levels
@@ -1145,14 +1838,16 @@ __device__ __forceinline__ void cell_records(int c, double M, double px, double 
                                              const int *__restrict__ cfirst, double *mo, float4 *cA, float4 *cB,
                                              float4 *cQ0, float4 *cQ1, float4 *cF0, float4 *cF1)
 {
-    double *me = mo + 10 * (int64_t)c;
-    me[0] = M;
-    me[1] = px;
-    me[2] = py;
-    me[3] = pz;
-    if (QUAD) {
+    if (mo) {
+        double *me = mo + 10 * (int64_t)c;
+        me[0] = M;
+        me[1] = px;
+        me[2] = py;
+        me[3] = pz;
+        if (QUAD) {
 #pragma unroll
-        for (int u = 0; u < 6; u++) me[4 + u] = q[u];
+            for (int u = 0; u < 6; u++) me[4 + u] = q[u];
+        }
     }
     float4 A, B;
     split2(px, A.x, B.x);
@@ -1317,6 +2012,7 @@ __device__ void cell_moments(int c, const int *__restrict__ csub, const int *__r
 constexpr int kPreThr = 256, kPrePer = 8;
 static_assert(kPreThr * kPrePer == kPreTile, "prefix tile");
 
+__device__ __forceinline__ double4 d4sub(double4 a, double4 b) { return make_double4(a.x - b.x, a.y - b.y, a.z - b.z, a.w - b.w); }
 __device__ __forceinline__ double4 d4add(double4 a, double4 b) { return make_double4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
 
 __device__ __forceinline__ double4 body_mom(const double4 b) { return make_double4(b.x * b.w, b.y * b.w, b.z * b.w, b.w); }
@@ -1398,7 +2094,7 @@ __global__ __launch_bounds__(kPreThr) void k_gather_tree(const uint32_t *__restr
             const int i = r.x + k * kPreThr + (int)threadIdx.x;
             const double4 b = v[k];
             if (i < r.y) {
-                bd[i] = b;
+                if (bd) bd[i] = b;
                 float4 h, l;
                 split2(b.x, h.x, l.x);
                 split2(b.y, h.y, l.y);
@@ -1437,6 +2133,87 @@ __global__ __launch_bounds__(kPreThr) void k_gather_tree(const uint32_t *__restr
     }
 }
 
+// The same by 1024 threads per tile and vector of sums (blockIdx.y), for few
+// tiles (one tile's eight rounds of scans, 24 with the second moments, took 19
+// to 30 us): four groups of kPreThr threads take two rounds each, all wave scans
+// first, then every round's carry from the totals before it, in
+// k_gather_tree's order of additions.
+constexpr int kFewThr = 1024, kFewPer = kPreTile / kFewThr, kFewTiles = 8;
+__global__ __launch_bounds__(kFewThr) void k_gather_few(const uint32_t *__restrict__ perm, int nb,
+                                                        const double *__restrict__ pos, const double *__restrict__ mass,
+                                                        const double4 *__restrict__ pk, double4 *bd, float4 *bhi,
+                                                        float4 *blo, int ntile, double4 *loc, double4 *part)
+{
+    constexpr int kW = kPreThr / 64;   // waves per round
+    __shared__ double4 wtot[kPrePer][kW];
+    const int t = blockIdx.x, lo = t * kPreTile, hi = min(nb, lo + kPreTile), vec = blockIdx.y;
+    const int lane = lane_id(), w = (threadIdx.x & (kPreThr - 1)) >> 6, g = threadIdx.x / kPreThr;
+    double4 v[kFewPer], x[kFewPer];
+    int at[kFewPer];
+#pragma unroll
+    for (int u = 0; u < kFewPer; u++) {
+        const int k = g * kFewPer + u;
+        at[u] = lo + k * kPreThr + (int)(threadIdx.x & (kPreThr - 1));
+        v[u] = make_double4(0, 0, 0, 0);
+        if (at[u] < hi) {
+            const int64_t o = perm[at[u]];
+            v[u] = pk ? pk[o] : make_double4(pos[3 * o], pos[3 * o + 1], pos[3 * o + 2], mass[o]);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kFewPer; u++) {
+        const double4 b = v[u];
+        if (vec == 0 && at[u] < hi) {
+            if (bd) bd[at[u]] = b;
+            float4 h, l;
+            split2(b.x, h.x, l.x);
+            split2(b.y, h.y, l.y);
+            split2(b.z, h.z, l.z);
+            h.w = (float)b.w;
+            l.w = 0.f;
+            bhi[at[u]] = h;
+            blo[at[u]] = l;
+        }
+        // m x, m y, m z, m; xx, xy, xz, yy; yz, zz
+        const double4 mm = body_mom(b);
+        v[u] = vec == 0 ? mm : vec == 1 ? make_double4(mm.x * b.x, mm.x * b.y, mm.x * b.z, mm.y * b.y)
+                                        : make_double4(mm.y * b.z, mm.z * b.z, 0.0, 0.0);
+        double4 s = v[u];
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const double4 y = make_double4(__shfl_up(s.x, d, 64), __shfl_up(s.y, d, 64), __shfl_up(s.z, d, 64),
+                                           __shfl_up(s.w, d, 64));
+            if (lane >= d) s = d4add(s, y);
+        }
+        x[u] = s;
+        if (lane == 63) wtot[g * kFewPer + u][w] = s;
+    }
+    if (!loc) return;
+    __syncthreads();
+    // carry: the totals of the rounds before, each the sum of its waves
+    double4 carry = make_double4(0, 0, 0, 0);
+    auto waves = [&](int k, int to) {
+        double4 a = make_double4(0, 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < kW; q++)
+            if (q < to) a = d4add(a, wtot[k][q]);
+        return a;
+    };
+    for (int k = 0; k < g * kFewPer; k++) carry = d4add(carry, waves(k, kW));
+#pragma unroll
+    for (int u = 0; u < kFewPer; u++) {
+        const int k = g * kFewPer + u;
+        const double4 ex = d4add(waves(k, w), d4sub(x[u], v[u]));
+        const double4 sum = d4add(d4add(carry, ex), v[u]);
+        if (at[u] < hi) {
+            if (vec < 2) loc[vec * (int64_t)nb + at[u]] = sum;
+            else reinterpret_cast<double2 *>(loc + 2 * (int64_t)nb)[at[u]] = make_double2(sum.x, sum.y);
+        }
+        carry = d4add(carry, waves(k, kW));
+    }
+    if (threadIdx.x == kFewThr - 1) part[vec * (int64_t)ntile + t] = carry;
+}
+
 // Exclusive scan of the tile sums of one system per block.
 // (vector blockIdx.y of the tile sums, part[v ntile + t])
 __global__ __launch_bounds__(kPreThr) void k_pre_top(double4 *part, const int *__restrict__ seg, int ntile)
@@ -1454,8 +2231,6 @@ __global__ __launch_bounds__(kPreThr) void k_pre_top(double4 *part, const int *_
     }
 }
 
-__device__ __forceinline__ double4 d4sub(double4 a, double4 b) { return make_double4(a.x - b.x, a.y - b.y, a.z - b.z, a.w - b.w); }
-
 // Mass, c.o.m. and the FP32 walk records of every cell from the prefixes
 // (the records cell_moments writes for a monopole build).  The sums over the
 // cell's bodies [s, e] are loc[e] - loc[s-1] inside one tile, else the
@@ -1463,37 +2238,32 @@ __device__ __forceinline__ double4 d4sub(double4 a, double4 b) { return make_dou
 // tile-local sums.  Tile of body i: seg[sys] + (i - s0) / kPreTile, s0 the
 // system's first body (one system: i / kPreTile).  In a batch, the cells
 // above the systems' roots are never walked and get no moments.
+// mo (may be null): the FP64 moments.
 template <bool QUAD>
-__global__ __launch_bounds__(kTpb) void k_moments_prefix(const int *__restrict__ cfirst, const int *__restrict__ clast,
-                                                         const uint8_t *__restrict__ clevel,
-                                                         const unsigned long long *ncellp, int nb, int ntile,
-                                                         const double4 *__restrict__ loc, const double4 *__restrict__ part,
-                                                         const int *__restrict__ seg, const uint64_t *__restrict__ keys,
-                                                         double *mo, float4 *cA, float4 *cB, float4 *cQ0, float4 *cQ1,
-                                                         float4 *cF0, float4 *cF1, const double4 *__restrict__ box,
-                                                         int lsys, int sysbits, const double4 *__restrict__ sysbox,
-                                                         const int64_t *__restrict__ boff)
+__global__ __launch_bounds__(kTpb) void k_moments_prefix(MomArgs m, double *mo)
 {
-    const int ncell = (int)*ncellp;
+    const int ncell = (int)*m.ncellp;
+    const int nb = m.nb, ntile = m.ntile;
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncell; c += gridDim.x * blockDim.x) {
-        const int s = cfirst[c], e = clast[c];
-        const int L = clevel[c];
+        const int s = m.first[c], e = m.last[c];
+        const int L = m.level[c];
         int Lg = L, s0 = 0, t0 = 0;
-        double4 bx = *box;
-        if (sysbox) {
-            const int sys = sysbits ? (int)(keys[s] >> (63 - sysbits)) : 0;
-            bx = sysbox[sys];
-            Lg = L - lsys;
-            s0 = (int)boff[sys];
-            t0 = seg[sys];
+        double4 bx = *m.box;
+        if (m.sysbox) {
+            const int sys = m.sysbits ? (int)(m.keys[s] >> (63 - m.sysbits)) : 0;
+            bx = m.sysbox[sys];
+            Lg = L - m.lsys;
+            s0 = (int)m.boff[sys];
+            t0 = m.seg[sys];
         }
-        double *me = mo + 10 * (int64_t)c;
         if (Lg < 0) {
+            if (mo) {
 #pragma unroll
-            for (int u = 0; u < (QUAD ? 10 : 4); u++) me[u] = 0.0;
-            cA[c] = make_float4(0.f, 0.f, 0.f, 0.f);
-            cB[c] = make_float4(0.f, 0.f, 0.f, 3.0e38f);
-            if (QUAD && cQ0) cQ0[c] = cQ1[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+                for (int u = 0; u < (QUAD ? 10 : 4); u++) mo[10 * (int64_t)c + u] = 0.0;
+            }
+            m.cA[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+            m.cB[c] = make_float4(0.f, 0.f, 0.f, 3.0e38f);
+            if (QUAD && m.cQ0) m.cQ0[c] = m.cQ1[c] = make_float4(0.f, 0.f, 0.f, 0.f);
             continue;
         }
         const int tb = t0 + (e - s0) / kPreTile;
@@ -1505,12 +2275,12 @@ __global__ __launch_bounds__(kTpb) void k_moments_prefix(const int *__restrict__
         // keep the precision of their own magnitudes); across more, the
         // difference of the tiles' prefixes (cells of over kPreTile bodies)
         auto at = [&](int v, int i) {
-            if (v < 2) return loc[(int64_t)v * nb + i];
-            const double2 q2 = reinterpret_cast<const double2 *>(loc + 2 * (int64_t)nb)[i];
+            if (v < 2) return m.loc[(int64_t)v * nb + i];
+            const double2 q2 = reinterpret_cast<const double2 *>(m.loc + 2 * (int64_t)nb)[i];
             return make_double4(q2.x, q2.y, 0.0, 0.0);
         };
         auto span = [&](int v) {
-            const double4 *pv = part + (int64_t)v * ntile;
+            const double4 *pv = m.part + (int64_t)v * ntile;
             double4 d = at(v, e);
             if (s > s0) {
                 const double4 la = at(v, s - 1);
@@ -1540,7 +2310,8 @@ __global__ __launch_bounds__(kTpb) void k_moments_prefix(const int *__restrict__
             q[4] = 3.0 * t[4];
             q[5] = 3.0 * t[5] - tr;
         }
-        cell_records<QUAD>(c, M, px, py, pz, q, L, Lg, bx.w, bx, keys, cfirst, mo, cA, cB, cQ0, cQ1, cF0, cF1);
+        cell_records<QUAD>(c, M, px, py, pz, q, L, Lg, bx.w, bx, m.keys, m.first, mo, m.cA, m.cB, m.cQ0, m.cQ1, m.cF0,
+                           m.cF1);
     }
 }
 
@@ -1655,6 +2426,7 @@ inline int nblocks(int64_t n, int tpb = kTpb) { return (int)std::max<int64_t>(1,
 // Grid of the kernels that stride over a device-side count bounded by cap.
 constexpr int kGatherBlocksPerCU = 8;   // grid of the tree build's gather (tiles of kPreTile bodies), per CU
 constexpr int kBodyBlocksPerCU = 16;    // grid of the per-body topology kernels (grid-stride), per CU
+constexpr int kScanFewParts = 2048;     // up to this many chunk sums (2^23 bodies) k_cbase's blocks add up those before them
 constexpr int kCapBlocksPerCU = 8;      // grid of the per-cell kernels (grid-stride over the device count), per CU
 inline int capgrid(const bh_ctx *ctx, int64_t cap)
 {
@@ -1679,6 +2451,7 @@ void exclusive_scan_u32(bh_ctx *ctx, const uint32_t *in, uint32_t *out, int64_t 
 void radix_sort_pairs(bh_ctx *ctx, uint64_t *k0, uint64_t *k1, uint32_t *v0, uint32_t *v1, int64_t n,
                       int begin_bit, int end_bit, uint64_t **kout, uint32_t **vout)
 {
+    // (the values are the indices: v0 is written by the second pass)
     int nblk = (int)std::max<int64_t>(1, (n + kSortTile - 1) / kSortTile);
     uint32_t *hist = ensure<uint32_t>(ctx->hist, 2 * (256 * (size_t)nblk + 1) + 256);
     uint32_t *hscan = hist + 256 * (size_t)nblk + 1;
@@ -1688,7 +2461,7 @@ void radix_sort_pairs(bh_ctx *ctx, uint64_t *k0, uint64_t *k1, uint32_t *v0, uin
     for (int shift = begin_bit; shift < end_bit; shift += 8) {
         k_radix_hist<<<nblk, kSortTpb, 0, ctx->stream>>>(ka, n, shift, hist, nblk);
         if (nblk > kSortFewTiles) k_hist_rows<<<256, kTpb, 0, ctx->stream>>>(hist, nblk, hscan, dtot);
-        k_radix_scatter<<<nblk, kSortTpb, 0, ctx->stream>>>(ka, va, kb, vb, n, shift, hist, hscan, dtot, nblk);
+        k_radix_scatter<<<nblk, kSortTpb, 0, ctx->stream>>>(ka, shift == begin_bit ? nullptr : va, kb, vb, n, shift, hist, hscan, dtot, nblk);
         std::swap(ka, kb);
         std::swap(va, vb);
     }
@@ -1697,9 +2470,44 @@ void radix_sort_pairs(bh_ctx *ctx, uint64_t *k0, uint64_t *k1, uint32_t *v0, uin
     *vout = va;
 }
 
-// Cell ranges of the sorted key array keys[0..n): cpl, cbase (n+1 entries),
-// block minima, and first/last/level of every cell, launched over the cell
-// capacity with the cell count kept on the device (stat[slot]).  n >= 2.
+// Merge passes over sorted tiles up to this many keys, radix passes beyond: 75
+// against 102 us at 10^5, 103 against 129 at 3 10^5, 174 against 166 at 2^20, 303
+// against 236 at 2^21 (keys and sort; a merge pass more per doubling, where the
+// radix passes stream).
+constexpr int64_t kMergeMax = 1 << 20;
+
+// Sorts n Morton keys with their indices: of the bodies at pos (mass and pk as
+// in k_tile_sort) in the box, or (pos null) the keys in k0.  k0/k1, v0/v1: two
+// buffers each; the sorted arrays are one of each.
+static void sort_keys(bh_ctx *ctx, const double *pos, const double *mass, int64_t n, const double4 *box, double4 *pk,
+                      const int *boxi, uint64_t *k0, uint64_t *k1, uint32_t *v0, uint32_t *v1, uint64_t **kout,
+                      uint32_t **vout)
+{
+    hipStream_t st = ctx->stream;
+    unsigned long long *stat = ptr<unsigned long long>(ctx->counters);
+    if (n <= kMergeMax) {
+        const int tiles = (int)((n + kSortTile - 1) / kSortTile);
+        uint64_t *ka = k1, *kb = k0;
+        uint32_t *va = v1, *vb = v0;
+        k_tile_sort<<<tiles, kSortTpb, 0, st>>>(pos, mass, n, box, k0, ka, va, pk, boxi, stat);
+        for (int64_t run = kSortTile; run < n; run *= 2) {
+            k_merge<<<(int)((n + kMergeTile - 1) / kMergeTile), kTpb, 0, st>>>(ka, va, kb, vb, n, run);
+            std::swap(ka, kb);
+            std::swap(va, vb);
+        }
+        *kout = ka;
+        *vout = va;
+    } else {
+        if (pos)
+            k_keys<<<(int)std::min<int64_t>(nblocks(n), (int64_t)ctx->ncu * 16), kTpb, 0, st>>>(pos, mass, n, box, k0,
+                                                                                               pk, boxi, stat);
+        radix_sort_pairs(ctx, k0, k1, v0, v1, n, 0, 64, kout, vout);
+    }
+    BH_HIP(hipGetLastError());
+}
+
+// Cell ranges of the sorted key array keys[0..n): cpl, cbase (n+1 entries), and
+// first/last/level of every cell.
 struct Topo {
     int8_t *cpl;
     uint32_t *cbase;
@@ -1709,70 +2517,135 @@ struct Topo {
     const unsigned long long *ncellp;
 };
 
-static Topo topology(bh_ctx *ctx, const uint64_t *keys, int n, int cap, DevBuf &bcpl, DevBuf &bcnt, DevBuf &bbase,
-                     DevBuf &bm1, DevBuf &bfirst, DevBuf &blast, DevBuf &blevel, DevBuf *bskip, DevBuf *bpre,
-                     DevBuf *bfnb, DevBuf &bowner, int slot, int slot_raw, unsigned long long flag)
+// The buffers of a topology of n >= 2 points and at most cap cells; tset: of a
+// separate test set.
+struct TopoBufs {
+    Topo t;
+    int n;
+    uint8_t *cq, *m1, *m2, *m3;
+    uint32_t *ccnt, *part;
+    int *skip, *pre;
+    int2 *fnb;
+    CellClamp clamp;
+};
+
+static TopoBufs topo_alloc(bh_ctx *ctx, int n, int cap, bool tset)
 {
-    hipStream_t st = ctx->stream;
     unsigned long long *stat = ptr<unsigned long long>(ctx->counters);
-    Topo t{};
-    t.cap = cap;
-    t.ncellp = stat + slot;
-    t.cpl = ensure<int8_t>(bcpl, 2 * (size_t)n + 32);
-    uint8_t *cq = reinterpret_cast<uint8_t *>(t.cpl) + ((n + 15) & ~7);   // 8-aligned, n + 8 bytes
-    uint32_t *ccnt = ensure<uint32_t>(bcnt, n + 1);
-    t.cbase = ensure<uint32_t>(bbase, n + 1);
-    const int bgrid = (int)std::min<int64_t>(nblocks(n), (int64_t)ctx->ncu * kBodyBlocksPerCU);
-    k_cpl<<<bgrid, kTpb, 0, st>>>(keys, n, t.cpl, cq, ccnt);
-    exclusive_scan_u32(ctx, ccnt, t.cbase, n);
-    int n1 = (n + 63) / 64, n2 = (n1 + 63) / 64, n3 = (n2 + 63) / 64;
+    TopoBufs b{};
+    b.n = n;
+    b.t.cap = cap;
+    b.t.ncellp = stat + (tset ? S_TNCELL : S_NCELL);
+    b.t.cpl = ensure<int8_t>(tset ? ctx->gcpl : ctx->cpl, 2 * (size_t)n + 32);
+    b.cq = reinterpret_cast<uint8_t *>(b.t.cpl) + ((n + 15) & ~7);   // 8-aligned, n + 8 bytes
+    b.ccnt = ensure<uint32_t>(tset ? ctx->gccnt : ctx->ccnt, n + 1);
+    b.t.cbase = ensure<uint32_t>(tset ? ctx->gcbase : ctx->cbase, n + 1);
+    const int n1 = (n + 63) / 64, n2 = (n1 + 63) / 64, n3 = (n2 + 63) / 64;
     // each level 8-byte aligned with at least one word of padding (the
     // search reads whole words; it stops at the entry holding cpl[n-1] = -1)
     auto words = [](int v) { return (v + 15) & ~7; };
-    uint8_t *m1 = reinterpret_cast<uint8_t *>(ensure<int8_t>(bm1, words(n1) + words(n2) + words(n3)));
-    uint8_t *m2 = m1 + words(n1), *m3 = m2 + words(n2);
-    const CellClamp cc{t.cbase, n, (unsigned long long)cap, stat, slot, slot_raw, flag};
-    k_cmin<<<nblocks(8 * (int64_t)n1), kTpb, 0, st>>>(cq, n, m1, n1, cc);
-    k_cmin<<<nblocks(8 * (int64_t)n2), kTpb, 0, st>>>(m1, n1, m2, n2);
-    k_cmin<<<nblocks(8 * (int64_t)n3), kTpb, 0, st>>>(m2, n2, m3, n3);
-    t.first = ensure<int>(bfirst, cap);
-    t.last = ensure<int>(blast, cap);
-    t.level = ensure<uint8_t>(blevel, cap);
-    int *cskip = bskip ? ensure<int>(*bskip, cap) : nullptr;
-    int *pre = bpre ? ensure<int>(*bpre, (size_t)n + cap) : nullptr;
-    int2 *fnb = bfnb ? ensure<int2>(*bfnb, cap) : nullptr;
-    int *owner = ensure<int>(bowner, cap);
-    k_owner<<<bgrid, kTpb, 0, st>>>(t.cbase, n, t.ncellp, owner);
-    k_cells<<<capgrid(ctx, cap), kTpb, 0, st>>>(t.cpl, cq, t.cbase, owner, m1, m2, m3, t.ncellp, t.first, t.last, t.level,
-                                                cskip, pre, fnb, bskip ? stat + S_DEEP : nullptr);
-    if (pre) k_body_pre<<<bgrid, kTpb, 0, st>>>(t.cbase, n, t.ncellp, pre);
-    BH_HIP(hipGetLastError());
-    return t;
+    b.m1 = reinterpret_cast<uint8_t *>(ensure<int8_t>(tset ? ctx->gm1 : ctx->cmin1, words(n1) + words(n2) + words(n3)));
+    b.m2 = b.m1 + words(n1);
+    b.m3 = b.m2 + words(n2);
+    b.part = ensure<uint32_t>(ctx->scan_tmp, n2 + 2);
+    b.t.first = ensure<int>(tset ? ctx->gcf : ctx->cfirst, cap);
+    b.t.last = ensure<int>(tset ? ctx->gcl : ctx->clast, cap);
+    b.t.level = ensure<uint8_t>(tset ? ctx->gclv : ctx->clevel, cap);
+    if (!tset) {
+        b.skip = ensure<int>(ctx->cskip, cap);
+        b.pre = ensure<int>(ctx->pre, (size_t)n + cap);
+        b.fnb = ensure<int2>(ctx->cfnb, cap);
+    }
+    b.clamp = CellClamp{(unsigned long long)cap, stat, tset ? S_TNCELL : S_NCELL, tset ? S_TNCELL_RAW : S_NCELL_RAW,
+                        tset ? F_TCELL_OVF : F_CELL_OVF};
+    return b;
 }
 
-// Groups of the sorted test set for the fast walk (ctx->gfirst/gcount, count
-// in stat[S_NGROUPS]).
-// csub/fnb: the tree's child slots and (first, count) per cell, when the
-// groups are cut from the tree's own topology.
-static void make_groups(bh_ctx *ctx, const Topo *t, const uint64_t *keys, int64_t n, int G, int lsys = 0,
-                        const int *csub = nullptr, const int2 *fnb = nullptr)
+// Prefix lengths, minima and cell numbers of the sorted keys (k_front computes
+// them for small sets).
+static void topo_scan(bh_ctx *ctx, const TopoBufs &b, const uint64_t *keys)
+{
+    hipStream_t st = ctx->stream;
+    const int n2 = (b.n + kScanChunk - 1) / kScanChunk;
+    k_cpl<<<n2, kTpb, 0, st>>>(keys, b.n, b.t.cpl, b.cq, b.ccnt, b.part, b.m1, b.m2);
+    const bool scanned = n2 > kScanFewParts;
+    if (scanned) k_scan_top<<<1, kTpb, 0, st>>>(b.part, n2, b.part + n2 + 1, 0);
+    k_cbase<<<n2, kTpb, 0, st>>>(b.ccnt, b.t.cbase, b.n, b.part, scanned, b.m2, n2, b.m3, b.clamp);
+}
+
+// Every cell, launched over the cell capacity with the cell count kept on the
+// device.
+static void topo_cells(bh_ctx *ctx, const TopoBufs &b)
+{
+    const int grid = std::min((b.n + kCellBodies - 1) / kCellBodies, ctx->ncu * kBodyBlocksPerCU);
+    k_cells<<<grid, kTpb, 0, ctx->stream>>>(b.t.cpl, b.cq, b.t.cbase, b.n, b.m1, b.m2, b.m3, b.t.ncellp, b.t.first,
+                                            b.t.last, b.t.level, b.skip, b.pre, b.fnb,
+                                            b.skip ? ptr<unsigned long long>(ctx->counters) + S_DEEP : nullptr);
+    BH_HIP(hipGetLastError());
+}
+
+// k_front for a set of n <= kSmallMax points: nb of them get a topology (b).
+// (measured: 119 against 129 us for the build at 6144 bodies, but 149 against 132
+// at 9000 with 12 bodies per thread)
+constexpr int kSmallMax = kSmallTpb * 6;
+
+template <bool BOX>
+static void small_front(bh_ctx *ctx, const double *pos, const double *mass, int n, int nb, const BoxStart &start, int rounds,
+                        double4 *box, uint32_t *lwork, int nlwork, uint64_t *keys, uint32_t *vals, const TopoBufs *b)
+{
+    unsigned long long *stat = ptr<unsigned long long>(ctx->counters);
+    FrontOut out{};
+    out.keys = keys;
+    out.vals = vals;
+    CellClamp cc{};
+    if (b) {
+        out = FrontOut{keys,   vals,  b->t.cpl, b->t.cbase, b->t.first, b->t.last, b->t.level, b->skip,
+                       b->pre, b->fnb, b->skip ? stat + S_DEEP : nullptr};
+        cc = b->clamp;
+    }
+    auto go = [&](auto kernel) {
+        kernel<<<1, kSmallTpb, 0, ctx->stream>>>(pos, mass, n, b ? nb : 0, start, rounds, box, stat, S_ZERO, lwork, nlwork,
+                                                 out, cc);
+    };
+    if (n <= 2 * kSmallTpb) go(k_front<2, BOX>);
+    else go(k_front<6, BOX>);
+    BH_HIP(hipGetLastError());
+}
+
+// Child slots (kids: the tree's cells) and, for the fast walk, the groups of
+// the sorted test set cut from the cells of t (ctx->gfirst/gcount, count in
+// stat[S_NGROUPS]): G > 0, of at most G points; own: from the tree's own child
+// slots.
+static void make_cells(bh_ctx *ctx, const Topo &t, const uint64_t *keys, int64_t n, bool kids, int G, bool own, int lsys)
 {
     hipStream_t st = ctx->stream;
     unsigned long long *stat = ptr<unsigned long long>(ctx->counters);
-    int *gf = ensure<int>(ctx->gfirst, n), *gc = ensure<int>(ctx->gcount, n);
-    if (t == nullptr) {
-        int64_t ng = (n + G - 1) / G;
-        k_groups_trivial<<<nblocks(ng), kTpb, 0, st>>>(n, G, gf, gc, stat);
-        return;
+    const int chunks = (t.cap + kGroupChunk - 1) / kGroupChunk;
+    const int grid = std::max(1, std::min(chunks, ctx->ncu * kCapBlocksPerCU));
+    uint32_t *gcnt = G ? ensure<uint32_t>(ctx->gscan, t.cap) : nullptr;
+    uint32_t *gpart = G ? ensure<uint32_t>(ctx->goff, chunks) : nullptr;
+    int *csub = kids ? ptr<int>(ctx->csub) : nullptr, *cnkids = kids ? ptr<int>(ctx->cnkids) : nullptr;
+    const int2 *fnb = own ? ptr<int2>(ctx->cfnb) : nullptr;
+    if (kids)
+        k_children<true><<<grid, kTpb, 0, st>>>(keys, t.cpl, t.cbase, t.first, t.last, t.level, t.ncellp, csub, cnkids, G,
+                                                lsys, fnb, gcnt, gpart);
+    else
+        k_children<false><<<grid, kTpb, 0, st>>>(keys, t.cpl, t.cbase, t.first, t.last, t.level, t.ncellp, nullptr,
+                                                 nullptr, G, lsys, nullptr, gcnt, gpart);
+    if (G) {
+        int *gf = ensure<int>(ctx->gfirst, n), *gc = ensure<int>(ctx->gcount, n);
+        k_group_write<<<grid, kTpb, 0, st>>>(keys, t.cpl, t.cbase, t.first, t.last, t.level, t.ncellp, G, lsys,
+                                             own ? csub : nullptr, fnb, gcnt, gpart, gf, gc, stat);
     }
-    uint32_t *gcnt = ensure<uint32_t>(ctx->gscan, (size_t)t->cap + 1);
-    uint32_t *goff = ensure<uint32_t>(ctx->goff, (size_t)t->cap + 1);
-    k_group_count<<<capgrid(ctx, t->cap), kTpb, 0, st>>>(keys, t->cpl, t->cbase, t->first, t->last, t->level,
-                                                         t->ncellp, G, lsys, csub, fnb, gcnt);
-    exclusive_scan_u32(ctx, gcnt, goff, t->cap, t->ncellp);
-    k_group_write<<<capgrid(ctx, t->cap), kTpb, 0, st>>>(keys, t->cpl, t->cbase, t->first, t->last, t->level,
-                                                         t->ncellp, G, lsys, csub, fnb, goff, gf, gc);
-    k_copy_count<<<1, 1, 0, st>>>(goff + t->cap, stat + S_NGROUPS);
+    BH_HIP(hipGetLastError());
+}
+
+// Groups of consecutive points, for a set of at most one group.
+static void one_group(bh_ctx *ctx, int64_t n, int G)
+{
+    k_groups_trivial<<<nblocks((n + G - 1) / G), kTpb, 0, ctx->stream>>>(n, G, ensure<int>(ctx->gfirst, n),
+                                                                         ensure<int>(ctx->gcount, n),
+                                                                         ptr<unsigned long long>(ctx->counters));
     BH_HIP(hipGetLastError());
 }
 
@@ -1780,41 +2653,22 @@ static void make_groups(bh_ctx *ctx, const Topo *t, const uint64_t *keys, int64_
 void debug_keys(bh_ctx *ctx, uint64_t *d_out)
 {
     double4 *d_box = ensure<double4>(ctx->dbox, 1);
-    uint32_t *tmp;
-    BH_HIP(hipMalloc(&tmp, ctx->nmass * sizeof(uint32_t)));
     k_keys<<<nblocks(ctx->nmass), kTpb, 0, ctx->stream>>>(ptr<double>(ctx->pos), ptr<double>(ctx->mass), ctx->nmass,
-                                                          d_box, d_out, tmp, nullptr);
+                                                          d_box, d_out, nullptr);
     BH_HIP(hipStreamSynchronize(ctx->stream));
-    BH_HIP(hipFree(tmp));
 }
 
-// Groups of the sorted test set.  When the test set is exactly the tree's
-// body set the tree topology is reused; otherwise the test keys get their own.
-static void build_groups(bh_ctx *ctx, const bh_params &p, const Topo *tree_topo, const uint64_t *ks,
-                         const uint64_t *tks)
+void fill_moments(bh_ctx *ctx)
 {
-    const int G = p.group_size > 0 ? p.group_size : 64;
-    const int64_t nt = ctx->ntest;
-    const Tree &T = ctx->tree;
-    // at most G points: one group (a cell only cuts groups for children of a
-    // cell holding more than G points); batches keep one group per system
-    if (ctx->nsys == 0 && nt <= G) {
-        make_groups(ctx, nullptr, nullptr, nt, G);
-        return;
-    }
-    if (ctx->self_test && nt == T.nb && tree_topo) {
-        make_groups(ctx, tree_topo, ks, nt, G, ctx->sysbits / 3, T.sub, T.fnb);
-        return;
-    }
-    if (ctx->nsys > 1) throw ApiFail(BH_ERR_STATE, "batch groups need the system-aware topology");
-    if (nt <= G || nt < 2) {
-        make_groups(ctx, nullptr, nullptr, nt, G);
-        return;
-    }
-    if (ctx->tcell_cap == 0) ctx->tcell_cap = (int)std::min<int64_t>(2 * nt + 64, INT32_MAX / 2);
-    Topo t = topology(ctx, tks, (int)nt, ctx->tcell_cap, ctx->gcpl, ctx->gccnt, ctx->gcbase, ctx->gm1, ctx->gcf,
-                      ctx->gcl, ctx->gclv, nullptr, nullptr, nullptr, ctx->gowner, S_TNCELL, S_TNCELL_RAW, F_TCELL_OVF);
-    make_groups(ctx, &t, tks, nt, G);
+    Tree &T = ctx->tree;
+    if (T.mo || T.cap == 0) return;
+    const MomArgs &m = ctx->mom;
+    double *mo = ensure<double>(ctx->cmo, 10 * (size_t)T.cap);
+    if (m.quad) k_moments_prefix<true><<<m.grid, kTpb, 0, ctx->stream>>>(m, mo);
+    else k_moments_prefix<false><<<m.grid, kTpb, 0, ctx->stream>>>(m, mo);
+    BH_HIP(hipGetLastError());
+    BH_HIP(hipStreamSynchronize(ctx->stream));
+    T.mo = mo;
 }
 
 // The build's second stream.  side_fork(k): ctx->side waits for the work
@@ -1822,7 +2676,7 @@ static void build_groups(bh_ctx *ctx, const bh_params &p, const Topo *tree_topo,
 // far on ctx->side; main_wait(k): the main stream waits for that mark.
 // Under graph capture the side stream joins the capture through the forked
 // event and every branch is joined back before the build returns.
-enum { kForkSort = 0, kMarkGather = 1, kForkTopo = 2, kMarkLevels = 3, kForkKids = 4, kMarkGroups = 5 };
+enum { kForkSort = 0, kMarkGather = 1, kForkTopo = 2, kMarkLevels = 3 };
 
 static void side_fork(bh_ctx *ctx, int k)
 {
@@ -1833,21 +2687,6 @@ static void side_fork(bh_ctx *ctx, int k)
 static void side_mark(bh_ctx *ctx, int k) { BH_HIP(hipEventRecord(ctx->fork_ev[k], ctx->side)); }
 
 static void main_wait(bh_ctx *ctx, int k) { BH_HIP(hipStreamWaitEvent(ctx->stream, ctx->fork_ev[k], 0)); }
-
-// build_groups on the side stream (its launches and scans use ctx->stream).
-static void build_groups_side(bh_ctx *ctx, const bh_params &p, const Topo *tree_topo, const uint64_t *ks,
-                              const uint64_t *tks)
-{
-    hipStream_t main = ctx->stream;
-    ctx->stream = ctx->side;
-    try {
-        build_groups(ctx, p, tree_topo, ks, tks);
-    } catch (...) {
-        ctx->stream = main;
-        throw;
-    }
-    ctx->stream = main;
-}
 
 // Builds the tree of the uploaded mass set and the sorted test set.  No host
 // synchronisation: every count stays on the device and capacities come from
@@ -1862,8 +2701,6 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
     int *d_boxi = ensure<int>(ctx->dboxi, 8);
     unsigned long long *stat = ensure<unsigned long long>(ctx->counters, S_NSLOTS);
     const bool timing = !ctx->capturing;
-    static_assert(S_ZERO <= 128, "k_build_start clears the status words with one 128-thread block");
-
     // -- box: start from the caller's box (or the previous one) and expand in
     //    input order; a fixed number of rounds, checked afterwards
     const bool keep = p.keep_box && ctx->box_valid;
@@ -1875,43 +2712,56 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
     double4 *sysbox = nsys ? ensure<double4>(ctx->sysbox, nsys) : nullptr;
     // level-list counters and cursors (k_level_count / k_level_place)
     uint32_t *lwork = ensure<uint32_t>(ctx->lhist, 3 * (kLevels + 1));
-    static_assert(3 * (kLevels + 1) <= 128, "k_build_start clears the level counters with one 128-thread block");
-    if (nsys) {
-        k_build_start<<<1, 128, 0, st>>>(stat, S_ZERO, lwork, 3 * (kLevels + 1), nullptr, nullptr, 0.0, 0.0, 0.0, 0.0,
-                                        0);
-        k_sys_box<<<nsys, kTpb, 0, st>>>(d_pos, sysoff, sysbox, d_box, r0, r1, r2, p.rsize, keep ? 1 : 0,
-                                         16 * ctx->box_rounds, stat);
-    } else {
-    k_build_start<<<1, 128, 0, st>>>(stat, S_ZERO, lwork, 3 * (kLevels + 1), d_box, d_boxi, r0, r1, r2, p.rsize,
-                                    keep ? 1 : 0);
-    double4 *cand = ensure<double4>(ctx->bcand, n);
-    k_box_compact<<<(int)((n + kBoxChunk - 1) / kBoxChunk), kTpb, 0, st>>>(d_pos, d_mass, n, d_box, cand, d_boxi,
-                                                                            stat);
+    constexpr int nlwork = 3 * (kLevels + 1);
+    static_assert(nlwork <= 128 && S_ZERO <= 128, "build_start clears them with one block of at least 128 threads");
+    const BoxStart start{r0, r1, r2, p.rsize, keep ? 1 : 0};
     const int rounds = std::max(1, keep ? ctx->box_rounds_keep : ctx->box_rounds);
-    for (int r = 0; r <= rounds; r++) k_box_round<<<ctx->ncu, kTpb, 0, st>>>(d_pos, cand, d_box, d_boxi);
-    }
 
-    // -- keys and sort of the mass set (massless bodies sort last)
+    // -- box, keys and sort of the mass set (massless bodies sort last); small
+    //    sets in one launch, with the scans of the topology
     uint64_t *k0 = ensure<uint64_t>(ctx->keys0, n), *k1 = ensure<uint64_t>(ctx->keys1, n);
     uint32_t *v0 = ensure<uint32_t>(ctx->vals0, n), *v1 = ensure<uint32_t>(ctx->vals1, n);
-    const int grid_n = (int)std::min<int64_t>(nblocks(n), (int64_t)ctx->ncu * 16);
+    const bool small = nsys == 0 && n <= kSmallMax;
+    const int cap = ctx->cell_cap;
+    TopoBufs tb{};
+    if (nb > 1) tb = topo_alloc(ctx, nb, cap, false);
     double4 *pk = nullptr;
-    if (nsys) {
-        k_keys_batch<<<grid_n, kTpb, 0, st>>>(d_pos, n, sysoff, nsys, sysbox, ctx->sysbits, k0, v0);
-        k_sysroot_init<<<nblocks(nsys), kTpb, 0, st>>>(sysoff, nsys, ensure<int>(ctx->sysroot, nsys));
-    } else {
-        pk = ensure<double4>(ctx->bpk, n);
-        k_keys<<<grid_n, kTpb, 0, st>>>(d_pos, d_mass, n, d_box, k0, v0, pk, d_boxi, stat);
-    }
     uint64_t *ks;
     uint32_t *vs;
-    if (timing) BH_HIP(hipEventRecord(ctx->ev[6], st));
-    radix_sort_pairs(ctx, k0, k1, v0, v1, n, 0, 64, &ks, &vs);
+    if (small) {
+        if (timing) BH_HIP(hipEventRecord(ctx->ev[6], st));
+        small_front<true>(ctx, d_pos, d_mass, (int)n, nb, start, 16 * rounds, d_box, lwork, nlwork, k0, v0,
+                          nb > 1 ? &tb : nullptr);
+        ks = k0;
+        vs = v0;
+    } else if (nsys) {
+        k_build_start<<<1, 128, 0, st>>>(stat, S_ZERO, lwork, nlwork);
+        k_sys_box<<<nsys, kTpb, 0, st>>>(d_pos, sysoff, sysbox, d_box, r0, r1, r2, p.rsize, keep ? 1 : 0,
+                                         16 * ctx->box_rounds, stat);
+        const int grid_n = (int)std::min<int64_t>(nblocks(n), (int64_t)ctx->ncu * 16);
+        k_keys_batch<<<grid_n, kTpb, 0, st>>>(d_pos, n, sysoff, nsys, sysbox, ctx->sysbits, k0);
+        k_sysroot_init<<<nblocks(nsys), kTpb, 0, st>>>(sysoff, nsys, ensure<int>(ctx->sysroot, nsys));
+        if (timing) BH_HIP(hipEventRecord(ctx->ev[6], st));
+        sort_keys(ctx, nullptr, nullptr, n, d_box, nullptr, nullptr, k0, k1, v0, v1, &ks, &vs);
+    } else {
+        // from a fresh box the first bodies are expanded for by one block, the
+        // others by passes over all
+        k_box_first<<<1, kFirstTpb, 0, st>>>(d_pos, d_mass, n, start, 16 * rounds, d_box, d_boxi, stat, S_ZERO, lwork,
+                                             nlwork);
+        const int64_t i0 = keep ? 0 : std::min<int64_t>(n, kBoxFirst);
+        double4 *cand = ensure<double4>(ctx->bcand, n);
+        const int grid = std::max(1, (int)((n - i0 + kBoxChunk - 1) / kBoxChunk));
+        for (int pass = n - i0 > kBoxOne ? std::max(2, rounds / 4) : 1; pass > 0; pass--)
+            k_box_compact<<<grid, kTpb, 0, st>>>(d_pos, d_mass, i0, n, d_box, cand, d_boxi, 16 * rounds,
+                                                 pass == 1 ? kBoxFew : kBoxShort, stat);
+        pk = ensure<double4>(ctx->bpk, n);
+        if (timing) BH_HIP(hipEventRecord(ctx->ev[6], st));
+        sort_keys(ctx, d_pos, d_mass, n, d_box, pk, d_boxi, k0, k1, v0, v1, &ks, &vs);
+    }
     if (timing) BH_HIP(hipEventRecord(ctx->ev[7], st));
 
     Tree &T = ctx->tree;
     T.nb = nb;
-    double4 *bd = ensure<double4>(ctx->bd, std::max(nb, 1));
     float4 *bhi = ensure<float4>(ctx->bhi, std::max(nb, 1));
     float4 *blo = ensure<float4>(ctx->blo, std::max(nb, 1));
     // fast builds take the moments from prefix sums of the gathered bodies
@@ -1922,6 +2772,12 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
     const bool prefix_moments = p.mode == BH_MODE_FAST && nb > 1;
     const bool prefix_quad = prefix_moments && (p.usequad || feat_b);
     const int nvec = prefix_quad ? 3 : 1;
+    // the FP64 bodies and moments are read by the strict walk, the sampling
+    // and exact-field passes and treecode1's radii; a plain fast build leaves
+    // them out (at 2^22 bodies 0.13 + 0.16 GB of stores beside the topology)
+    // and bh_debug_cells has the moments written when it asks for them
+    const bool need64 = !prefix_moments || ctx->mlp_sampling || p.learned > 1 || p.criterion != BH_CRIT_HACK;
+    double4 *bd = need64 ? ensure<double4>(ctx->bd, std::max(nb, 1)) : nullptr;
     double4 *mpre = prefix_moments ? ensure<double4>(ctx->mpre, (size_t)nvec * nb) : nullptr;
     // the gather (HBM-bound; with, for prefix-moment builds, the tile-local
     // sums) on the second stream beside the topology (latency-bound); only
@@ -1934,14 +2790,22 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
     side_fork(ctx, kForkSort);
     if (nb > 0) {
         const int ggrid = std::min(ntile, ctx->ncu * kGatherBlocksPerCU);
-        if (nvec == 3)
+        // (builds of 1000 and 2048 bodies with second moments 83 against 96 and 101
+        // us; the same from 9000 bodies on, where the topology hides it, and slower
+        // from 10^5 on: 189 against 181, 271 against 257 at 5.2 10^5)
+        const bool few = !tiles && ntile <= kFewTiles;
+        if (few)
+            k_gather_few<<<dim3(ntile, mpre ? nvec : 1), kFewThr, 0, ctx->side>>>(vs, nb, d_pos, d_mass, pk, bd, bhi, blo,
+                                                                                  ntile, mpre, part);
+        else if (nvec == 3)
             k_gather_tree<3><<<ggrid, kPreThr, 0, ctx->side>>>(vs, nb, d_pos, d_mass, pk, bd, bhi, blo, tiles, ntile,
                                                                mpre, part);
         else
             k_gather_tree<1><<<ggrid, kPreThr, 0, ctx->side>>>(vs, nb, d_pos, d_mass, pk, bd, bhi, blo, tiles, ntile,
                                                                mpre, part);
     }
-    if (prefix_moments)
+    // (the cells of a single tile never ask for its prefix)
+    if (prefix_moments && ntile > 1)
         k_pre_top<<<dim3(nsys ? nsys : 1, nvec), kPreThr, 0, ctx->side>>>(part, nsys ? ptr<int>(ctx->pseg) : nullptr,
                                                                          ntile);
     side_mark(ctx, kMarkGather);
@@ -1955,17 +2819,23 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
     const int64_t nt = ctx->ntest;
     const bool alias = ctx->self_test && nt == nb;
     float4 *thi = alias ? nullptr : ensure<float4>(ctx->thi, nt), *tlo = alias ? nullptr : ensure<float4>(ctx->tlo, nt);
-    double4 *td = alias ? nullptr : ensure<double4>(ctx->td, nt);
+    double4 *td = alias || p.mode == BH_MODE_FAST ? nullptr : ensure<double4>(ctx->td, nt);   // (the strict walk's)
     int *tself = alias ? nullptr : ensure<int>(ctx->tself, nt);
-    uint32_t *tperm = alias ? nullptr : ensure<uint32_t>(ctx->tperm, nt);
     const uint64_t *tks_for_groups = ks;
     T.thi = thi;
     T.tlo = tlo;
     T.td = td;
-    T.tperm = tperm;
     T.tself = tself;
     T.tinv = nullptr;
     T.selfmode = ctx->self_test ? 2 : 0;
+    // groups of a test set with its own order (fast mode): at most G points
+    // are one group (a cell only cuts groups for children of a cell holding
+    // more than G points; batches, whose test set is the tree's, keep one
+    // group per system); more are cut from the topology of their own keys
+    const int G = p.mode == BH_MODE_FAST ? (p.group_size > 0 ? p.group_size : 64) : 0;
+    const bool tset_topo = !alias && G > 0 && nt > G && nt >= 2;
+    TopoBufs ttb{};
+    if (tset_topo && ctx->tcell_cap == 0) ctx->tcell_cap = (int)std::min<int64_t>(2 * nt + 64, INT32_MAX / 2);
     if (alias) {
         // the test set is the tree's body set in the same order
         T.thi = bhi;
@@ -1984,22 +2854,42 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
         uint64_t *tk0 = ensure<uint64_t>(ctx->tkeys0, nt), *tk1 = ensure<uint64_t>(ctx->tkeys1, nt);
         uint32_t *tv0 = ensure<uint32_t>(ctx->tvals0, nt), *tv1 = ensure<uint32_t>(ctx->tvals1, nt);
         const double *d_tpos = ctx->self_test ? d_pos : ptr<double>(ctx->tpos);
-        k_keys<<<(int)std::min<int64_t>(nblocks(nt), (int64_t)ctx->ncu * 16), kTpb, 0, st>>>(d_tpos, nullptr, nt, d_box,
-                                                                                            tk0, tv0, nullptr);
         uint64_t *tks;
         uint32_t *tvs;
-        radix_sort_pairs(ctx, tk0, tk1, tv0, tv1, nt, 0, 64, &tks, &tvs);
+        if (nt <= kSmallMax) {
+            if (tset_topo) ttb = topo_alloc(ctx, (int)nt, ctx->tcell_cap, true);
+            small_front<false>(ctx, d_tpos, nullptr, (int)nt, (int)nt, start, 0, d_box, nullptr, 0, tk0, tv0,
+                               tset_topo ? &ttb : nullptr);
+            tks = tk0;
+            tvs = tv0;
+        } else {
+            sort_keys(ctx, d_tpos, nullptr, nt, d_box, nullptr, nullptr, tk0, tk1, tv0, tv1, &tks, &tvs);
+        }
         tks_for_groups = tks;
-        BH_HIP(hipMemcpyAsync(tperm, tvs, nt * sizeof(uint32_t), hipMemcpyDeviceToDevice, st));
+        T.tperm = tvs;
         int *tmap = nullptr, *tinv = nullptr;
         if (ctx->self_test) {
             tmap = ensure<int>(ctx->tmap, nt);
             tinv = ensure<int>(ctx->tinv, std::max(nb, 1));
             k_tree_index<<<nblocks(nt), kTpb, 0, st>>>(vs, nt, nb, tmap);
         }
-        k_gather_test<<<nblocks(nt), kTpb, 0, st>>>(tperm, nt, d_tpos, thi, tlo, td, tself, tmap, tinv);
+        k_gather_test<<<nblocks(nt), kTpb, 0, st>>>(T.tperm, nt, d_tpos, thi, tlo, td, tself, tmap, tinv);
         T.tinv = tinv;
     }
+
+    auto test_groups = [&]() {
+        if (nsys > 1) throw ApiFail(BH_ERR_STATE, "batch groups need the system-aware topology");
+        if (!tset_topo) {
+            one_group(ctx, nt, G);
+            return;
+        }
+        if (nt > kSmallMax) {
+            ttb = topo_alloc(ctx, (int)nt, ctx->tcell_cap, true);
+            topo_scan(ctx, ttb, tks_for_groups);
+            topo_cells(ctx, ttb);
+        }
+        make_cells(ctx, ttb.t, tks_for_groups, nt, false, G, false, 0);
+    };
 
     // -- topology over the cell capacity
     int *pre = ensure<int>(ctx->pre, std::max(nb, 1) + (size_t)std::max(ctx->cell_cap, 1));
@@ -2009,21 +2899,21 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
     if (nb <= 1) {
         main_wait(ctx, kMarkGather);
         if (nb == 1) k_set_int<<<1, 1, 0, st>>>(pre, 0);
-        if (p.mode == BH_MODE_FAST) build_groups(ctx, p, nullptr, ks, tks_for_groups);
+        if (p.mode == BH_MODE_FAST) test_groups();
         return;
     }
-    const int cap = ctx->cell_cap;
-    Topo tt = topology(ctx, ks, nb, cap, ctx->cpl, ctx->ccnt, ctx->cbase, ctx->cmin1, ctx->cfirst, ctx->clast,
-                       ctx->clevel, &ctx->cskip, &ctx->pre, &ctx->cfnb, ctx->cowner, S_NCELL, S_NCELL_RAW, F_CELL_OVF);
+    const Topo tt = tb.t;
+    if (!small) {
+        topo_scan(ctx, tb, ks);
+        topo_cells(ctx, tb);
+    }
     T.cap = cap;
-    int8_t *cpl = tt.cpl;
-    uint32_t *cbase = tt.cbase;
     int *cfirst = tt.first, *clast = tt.last;
     uint8_t *clevel = tt.level;
     T.pre = ptr<int>(ctx->pre);
     int *csub = ensure<int>(ctx->csub, 8 * (size_t)cap);
     int *cnkids = ensure<int>(ctx->cnkids, cap);
-    double *mo = ensure<double>(ctx->cmo, 10 * (size_t)cap);
+    double *mo = need64 ? ensure<double>(ctx->cmo, 10 * (size_t)cap) : nullptr;
     float4 *cA = ensure<float4>(ctx->cA, cap), *cB = ensure<float4>(ctx->cB, cap);
     float4 *cQ0 = ensure<float4>(ctx->cQ0, cap), *cQ1 = ensure<float4>(ctx->cQ1, cap);
     float4 *cF0 = ensure<float4>(ctx->cF0, cap), *cF1 = ensure<float4>(ctx->cF1, cap);
@@ -2036,22 +2926,44 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
     if (prefix_moments) {
         // the moments on the second stream (after its prefix scan), beside
         // the child slots and the groups on the main stream
-        const int *pseg = nsys ? ptr<int>(ctx->pseg) : nullptr;
-        const int64_t *boff = nsys ? ptr<int64_t>(ctx->boff) : nullptr;
-        if (prefix_quad)
-            k_moments_prefix<true><<<capgrid(ctx, cap), kTpb, 0, sd>>>(
-                cfirst, clast, clevel, tt.ncellp, nb, ntile, mpre, part, pseg, ks, mo, cA, cB,
-                p.usequad ? cQ0 : nullptr, cQ1, feat_b ? cF0 : nullptr, cF1, d_box, lsys, ctx->sysbits, sysbox, boff);
-        else
-            k_moments_prefix<false><<<capgrid(ctx, cap), kTpb, 0, sd>>>(
-                cfirst, clast, clevel, tt.ncellp, nb, ntile, mpre, part, pseg, ks, mo, cA, cB, nullptr, nullptr,
-                nullptr, nullptr, d_box, lsys, ctx->sysbits, sysbox, boff);
+        MomArgs m;
+        m.quad = prefix_quad;
+        m.grid = capgrid(ctx, cap);
+        m.first = cfirst;
+        m.last = clast;
+        m.level = clevel;
+        m.ncellp = tt.ncellp;
+        m.nb = nb;
+        m.ntile = ntile;
+        m.loc = mpre;
+        m.part = part;
+        m.seg = nsys ? ptr<int>(ctx->pseg) : nullptr;
+        m.keys = ks;
+        m.cA = cA;
+        m.cB = cB;
+        m.cQ0 = p.usequad ? cQ0 : nullptr;
+        m.cQ1 = cQ1;
+        m.cF0 = feat_b ? cF0 : nullptr;
+        m.cF1 = cF1;
+        m.box = d_box;
+        m.lsys = lsys;
+        m.sysbits = ctx->sysbits;
+        m.sysbox = sysbox;
+        m.boff = nsys ? ptr<int64_t>(ctx->boff) : nullptr;
+        ctx->mom = m;
+        if (prefix_quad) k_moments_prefix<true><<<m.grid, kTpb, 0, sd>>>(m, mo);
+        else k_moments_prefix<false><<<m.grid, kTpb, 0, sd>>>(m, mo);
     } else {
         k_level_count<<<capgrid(ctx, cap), kTpb, 0, sd>>>(clevel, tt.ncellp, lcount);
         k_level_place<<<capgrid(ctx, cap), kTpb, 0, sd>>>(clevel, tt.ncellp, lcount, loffd, lcursor, llist);
     }
     side_mark(ctx, kMarkLevels);
-    k_children<<<capgrid(ctx, cap), kTpb, 0, st>>>(ks, cpl, cbase, cfirst, clast, clevel, tt.ncellp, csub, cnkids);
+    // the child slots and the groups on the main stream beside the moments
+    const bool few = nsys == 0 && nt <= G;
+    const bool own = alias && !few && G > 0;
+    make_cells(ctx, tt, ks, nt, true, own ? G : 0, own, lsys);
+    if (G && few) one_group(ctx, nt, G);
+    else if (G && !own) test_groups();
     T.first = cfirst;
     T.last = clast;
     T.fnb = ptr<int2>(ctx->cfnb);
@@ -2059,19 +2971,6 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
     T.skip = ptr<int>(ctx->cskip);
     T.sub = csub;
     T.nkids = cnkids;
-    // the groups need the child slots and the topology only: on the second
-    // stream (after the level lists there) beside the level-by-level
-    // moments, or on the main stream while the second computes the moments
-    // from the prefix sums
-    const bool groups = p.mode == BH_MODE_FAST;
-    const bool groups_side = groups && !prefix_moments;
-    if (groups_side) {
-        side_fork(ctx, kForkKids);
-        build_groups_side(ctx, p, &tt, ks, tks_for_groups);
-        side_mark(ctx, kMarkGroups);
-    } else if (groups) {
-        build_groups(ctx, p, &tt, ks, tks_for_groups);
-    }
     main_wait(ctx, kMarkGather);
     main_wait(ctx, kMarkLevels);
     const int mgrid = ctx->ncu * 4;
@@ -2106,7 +3005,6 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
     T.cQ1 = cQ1;
     T.cF0 = cF0;
     T.cF1 = cF1;
-    if (groups_side) main_wait(ctx, kMarkGroups);
 }
 
 }  // namespace bh
