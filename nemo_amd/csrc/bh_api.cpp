@@ -637,7 +637,7 @@ bh_status bh_lf_force(bh_ctx *ctx, double *diag, int64_t *n2b, int64_t *nbc)
         const int nd = 36 * std::max(1, ctx->nsys);
         double *dd = bh::ensure<double>(ctx->diag_buf, nd);
         long long *d2 = bh::ensure<long long>(ctx->n2b_buf, 1), *dc = bh::ensure<long long>(ctx->nbc_buf, 1);
-        bh::lf_after_force(ctx, dd, d2, dc);
+        bh::lf_after_force(ctx, dd, d2, dc, false);
         std::vector<double> h(nd);
         long long c[2];
         BH_HIP(hipMemcpyAsync(h.data(), dd, nd * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
@@ -678,8 +678,7 @@ bh_status bh_lf_run(bh_ctx *ctx, int64_t nsteps, int use_graph, double *diag, in
         if (!ctx->box_valid || !use_graph) {
             bh_params q = lf_params(ctx);
             eval(ctx, &q, nullptr);
-            bh::lf_after_force(ctx, dd, d2, dc);
-            bh::lf_drift(ctx);
+            bh::lf_after_force(ctx, dd, d2, dc, true);
             done = 1;
         }
         bh_params q = lf_params(ctx);
@@ -696,8 +695,7 @@ bh_status bh_lf_run(bh_ctx *ctx, int64_t nsteps, int use_graph, double *diag, in
                     bh::build_tree(ctx, q);
                     if (q.mode == BH_MODE_STRICT) bh::walk_strict(ctx, q);
                     else bh::walk_fast(ctx, q);
-                    bh::lf_after_force(ctx, dd, d2, dc);
-                    bh::lf_drift(ctx);
+                    bh::lf_after_force(ctx, dd, d2, dc, true);
                 } catch (...) {
                     ctx->capturing = false;
                     hipGraph_t g = nullptr;
@@ -717,8 +715,7 @@ bh_status bh_lf_run(bh_ctx *ctx, int64_t nsteps, int use_graph, double *diag, in
                 bh::build_tree(ctx, q);
                 if (q.mode == BH_MODE_STRICT) bh::walk_strict(ctx, q);
                 else bh::walk_fast(ctx, q);
-                bh::lf_after_force(ctx, dd, d2, dc);
-                bh::lf_drift(ctx);
+                bh::lf_after_force(ctx, dd, d2, dc, true);
             }
         }
         unsigned long long h[bh::S_NSLOTS];

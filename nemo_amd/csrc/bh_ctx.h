@@ -170,7 +170,7 @@ int64_t mlp_collect(bh_ctx *ctx, const bh_params &p);
 // bh_lf.hip
 void lf_reset(bh_ctx *ctx);
 void lf_reset_record(bh_ctx *ctx);
-void lf_after_force(bh_ctx *ctx, double *diag_out, long long *n2b_out, long long *nbc_out);
+void lf_after_force(bh_ctx *ctx, double *diag_out, long long *n2b_out, long long *nbc_out, bool drift);
 void lf_drift(bh_ctx *ctx);
 
 }  // namespace bh
