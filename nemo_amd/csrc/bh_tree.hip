@@ -101,27 +101,14 @@ __device__ __forceinline__ bool fits(const double4 c, const BoxTest &t)
     return fits(x, t);
 }
 
-// Massive bodies outside the starting box (the only ones that can ever make
-// expandbox grow it, since the box only grows).
-__device__ __forceinline__ bool outside_massive(const double *__restrict__ pos, const double *__restrict__ mass,
-                                                int64_t i, int64_t n, const BoxTest &b, int *bad)
-{
-    if (i >= n) return false;
-    // mass and position loads issued together (one memory round trip)
-    const double m = mass[i];
-    const double x[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
-    if (m == 0.0 || fits(x, b)) return false;
-    if (!(isfinite(x[0]) && isfinite(x[1]) && isfinite(x[2]))) *bad = 1;
-    return true;
-}
-
-// Compaction in any order (the rounds take the lowest index).  Block b owns
+// Massive bodies outside the box (the only ones that can ever make expandbox
+// grow it, since the box only grows) are listed in any order.  Block b owns
 // bodies [b*kBoxChunk, (b+1)*kBoxChunk); in step k thread t tests body
-// b*kBoxChunk + k*kTpb + t (coalesced) into bit k of a mask, a block scan of
-// the counts gives the slots and one atomic per block (boxi[4]) reserves the
-// block's range.  A candidate is stored with its position (x, y, z, index),
-// so the rounds read it contiguously.
-constexpr int kBoxPer = 16, kBoxChunk = kTpb * kBoxPer;
+// b*kBoxChunk + k*kTpb + t (coalesced) into bit k of a mask (kBoxLoad steps'
+// loads in flight), a block scan of the counts gives the slots and one atomic
+// per block (boxi[4]) reserves the block's range.  A candidate is stored with
+// its position (x, y, z, index), so the looks read it contiguously.
+constexpr int kBoxPer = 16, kBoxChunk = kTpb * kBoxPer, kBoxLoad = 8;
 
 // Doubling of expandbox (load.c:68-95) until body x fits.
 __device__ __forceinline__ double4 expand_for(const double *x, double4 b)
@@ -227,8 +214,23 @@ __global__ __launch_bounds__(kTpb) void k_box_compact(const double *__restrict__
     int bad = 0;
     uint32_t mask = 0;
 #pragma unroll
-    for (int k = 0; k < kBoxPer; k++)
-        if (j0 + k * kTpb >= begin && outside_massive(pos, mass, j0 + k * kTpb, n, b, &bad)) mask |= 1u << k;
+    for (int k0 = 0; k0 < kBoxPer; k0 += kBoxLoad) {
+        double m[kBoxLoad], x[kBoxLoad][3];
+#pragma unroll
+        for (int k = 0; k < kBoxLoad; k++) {
+            const int64_t i = min(j0 + (k0 + k) * kTpb, n - 1);
+            m[k] = mass[i];
+#pragma unroll
+            for (int c = 0; c < 3; c++) x[k][c] = pos[3 * i + c];
+        }
+#pragma unroll
+        for (int k = 0; k < kBoxLoad; k++) {
+            const int64_t i = j0 + (k0 + k) * kTpb;
+            if (i < begin || i >= n || m[k] == 0.0 || fits(x[k], b)) continue;
+            if (!(isfinite(x[k][0]) && isfinite(x[k][1]) && isfinite(x[k][2]))) bad = 1;
+            mask |= 1u << (k0 + k);
+        }
+    }
     uint32_t tot;
     uint32_t off = block_excl_scan((uint32_t)__popc(mask), &tot);
     if (threadIdx.x == 0 && tot) base = atomicAdd(reinterpret_cast<uint32_t *>(&boxi[4]), tot);
