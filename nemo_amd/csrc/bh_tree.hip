@@ -983,31 +983,37 @@ __device__ __forceinline__ uint64_t key_of(const double *__restrict__ pos, const
     return morton_of(x, b) | (mass && m == 0.0 ? 1ULL << 63 : 0);
 }
 
-// Sorted tiles of kSortTile bodies: keys computed from the positions (and the
+// Sorted tiles of kMergeRun bodies: keys computed from the positions (and the
 // packed records pk written) or, pos null, read from keys.  boxi as in k_keys.
-__global__ __launch_bounds__(kSortTpb) void k_tile_sort(const double *__restrict__ pos, const double *__restrict__ mass,
+// Few blocks with a chain of LDS round trips each: 16 waves of 4 keys per lane,
+// not 8 waves of 8 (24 us for 10^4 bodies, 50 for 2^20).
+constexpr int kTileTpb = 1024, kTileItems = 4, kMergeRun = kTileTpb * kTileItems;
+constexpr int kLogRun = 12;
+static_assert(1 << kLogRun == kMergeRun, "runs of the first pass");
+
+__global__ __launch_bounds__(kTileTpb) void k_tile_sort(const double *__restrict__ pos, const double *__restrict__ mass,
                                                         int64_t n, const double4 *__restrict__ box,
                                                         const uint64_t *__restrict__ keys, uint64_t *kout, uint32_t *vout,
                                                         double4 *pk, const int *__restrict__ boxi, unsigned long long *stat)
 {
-    __shared__ BlockSort<kSortTpb, kSortItems, uint32_t> S;
+    __shared__ BlockSort<kTileTpb, kTileItems, uint16_t> S;
     if (boxi && blockIdx.x == 0 && threadIdx.x == 0 && !boxi[5]) atomicOr(&stat[S_FLAGS], (unsigned long long)F_BOX_OPEN);
-    const int64_t base = (int64_t)blockIdx.x * kSortTile;
-    const int first = (threadIdx.x >> 6) * kSortItems * 64 + lane_id();
+    const int64_t base = (int64_t)blockIdx.x * kMergeRun;
+    const int first = (threadIdx.x >> 6) * kTileItems * 64 + lane_id();
     const double4 b = pos ? *box : make_double4(0, 0, 0, 1);
-    uint64_t key[kSortItems];
-    uint32_t val[kSortItems];
+    uint64_t key[kTileItems];
+    uint16_t val[kTileItems];
 #pragma unroll
-    for (int r = 0; r < kSortItems; r++) {
+    for (int r = 0; r < kTileItems; r++) {
         const int64_t i = base + first + r * 64;
-        val[r] = (uint32_t)i;
+        val[r] = (uint16_t)(first + r * 64);
         if (pos) key[r] = key_of(pos, mass, i, n, b, pk);
         else key[r] = i < n ? keys[i] : ~0ULL;
     }
-    S.sort(key, val, (int)min<int64_t>(kSortTile, n - base));
-    for (int j = threadIdx.x; j < kSortTile && base + j < n; j += kSortTpb) {
+    S.sort(key, val, (int)min<int64_t>(kMergeRun, n - base));
+    for (int j = threadIdx.x; j < kMergeRun && base + j < n; j += kTileTpb) {
         kout[base + j] = S.skey[j];
-        vout[base + j] = S.sval[j];
+        vout[base + j] = (uint32_t)(base + S.sval[j]);
     }
 }
 
@@ -1017,7 +1023,7 @@ __global__ __launch_bounds__(kSortTpb) void k_tile_sort(const double *__restrict
 // searches, the block stages its keys in LDS and each thread merges
 // kMergeItems of them.
 constexpr int kMergeItems = 8, kMergeTile = kTpb * kMergeItems;
-static_assert(kSortTile % kMergeTile == 0, "an output tile lies in one pair of runs");
+static_assert(kMergeRun % kMergeTile == 0, "an output tile lies in one pair of runs");
 
 __global__ __launch_bounds__(kTpb) void k_merge(const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
                                                 uint64_t *__restrict__ kout, uint32_t *__restrict__ vout, int64_t n,
@@ -1061,14 +1067,13 @@ __global__ __launch_bounds__(kTpb) void k_merge(const uint64_t *__restrict__ kin
         else hi = mid;
     }
     int ia = lo, ib = ca + d - lo;
-    uint64_t ka = ia < ca ? sk[ia] : 0, kb = ib < tot ? sk[ib] : 0;
+    uint64_t ka = ia < ca ? sk[ia] : 0, kb = ib < tot ? sk[ib] : 0, key[kMergeItems];
+    uint32_t val[kMergeItems];
 #pragma unroll
     for (int k = 0; k < kMergeItems; k++) {
-        if (d + k >= tot) break;
         const bool fromA = ib >= tot || (ia < ca && ka <= kb);
-        const int at = fromA ? ia : ib;
-        kout[o0 + d + k] = fromA ? ka : kb;
-        vout[o0 + d + k] = sv[at];
+        key[k] = fromA ? ka : kb;
+        val[k] = sv[min(fromA ? ia : ib, tot - 1)];
         if (fromA) {
             ia++;
             ka = ia < ca ? sk[ia] : 0;
@@ -1077,6 +1082,56 @@ __global__ __launch_bounds__(kTpb) void k_merge(const uint64_t *__restrict__ kin
             kb = ib < tot ? sk[ib] : 0;
         }
     }
+    // through LDS, so that neighbours write neighbouring keys
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kMergeItems; k++)
+        if (d + k < tot) {
+            sk[d + k] = key[k];
+            sv[d + k] = val[k];
+        }
+    __syncthreads();
+    for (int j = threadIdx.x; j < tot; j += kTpb) {
+        kout[o0 + j] = sk[j];
+        vout[o0 + j] = sv[j];
+    }
+}
+
+// One pass merging four sorted runs of 2^lrun keys at a time by ranks: a key's
+// place is its place in its own run plus, per other run, the keys before it
+// there (an earlier run's equal keys come first), found by binary searches side
+// by side.  Neighbouring keys probe neighbouring places, so a wave's loads are
+// few lines, mostly in cache, and a pass of four runs takes what k_merge's of
+// two does (8 us) until the loads bound it (kRankMax).
+constexpr int kWays = 4;
+__global__ __launch_bounds__(kTpb) void k_rank_merge(const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
+                                                     uint64_t *__restrict__ kout, uint32_t *__restrict__ vout, int n,
+                                                     int lrun)
+{
+    const int i = blockIdx.x * kTpb + (int)threadIdx.x;
+    if (i >= n) return;
+    const uint64_t key = kin[i];
+    const uint32_t val = vin[i];
+    const int own = i >> lrun, seg = own & ~(kWays - 1);
+    int pos[kWays];
+#pragma unroll
+    for (int j = 0; j < kWays; j++) pos[j] = 0;
+    for (int step = 1 << lrun; step > 0; step >>= 1) {
+        uint64_t k[kWays];
+#pragma unroll
+        for (int j = 0; j < kWays; j++) k[j] = kin[min(((seg + j) << lrun) + pos[j] + step - 1, n - 1)];
+#pragma unroll
+        for (int j = 0; j < kWays; j++) {
+            const int p = pos[j] + step;
+            if (seg + j != own && p <= 1 << lrun && ((seg + j) << lrun) + p <= n && (seg + j < own ? k[j] <= key : k[j] < key))
+                pos[j] = p;
+        }
+    }
+    int at = (seg << lrun) + (i - (own << lrun));
+#pragma unroll
+    for (int j = 0; j < kWays; j++) at += pos[j];
+    kout[at] = key;
+    vout[at] = val;
 }
 
 // ---- gather sorted bodies ----------------------------------------------------
@@ -1144,16 +1199,18 @@ __device__ __forceinline__ void clamp_cells(const CellClamp &c, unsigned long lo
 // over 64 and 4096 entries (a wave's round and the block; the range-end search
 // reads them).  One pass over the keys in the place of four launches.
 static_assert(kScanChunk == 4096, "a block's bodies are one m2 entry");
-__global__ __launch_bounds__(kTpb) void k_cpl(const uint64_t *__restrict__ keys, int nb, int8_t *cpl, uint8_t *cq,
+constexpr int kCplTpb = 1024, kCplItems = kScanChunk / kCplTpb;
+__global__ __launch_bounds__(kCplTpb) void k_cpl(const uint64_t *__restrict__ keys, int nb, int8_t *cpl, uint8_t *cq,
                                               uint32_t *ccnt, uint32_t *part, uint8_t *m1, uint8_t *m2)
 {
-    __shared__ int wmin[kTpb / 64];
+    __shared__ int wmin[kCplTpb / 64];
+    __shared__ uint32_t wsum[kCplTpb / 64];
     const int lane = lane_id(), w = threadIdx.x >> 6;
     const int base = blockIdx.x * kScanChunk + (int)threadIdx.x;
-    uint64_t key[kScanItems], edge[kScanItems];
+    uint64_t key[kCplItems], edge[kCplItems];
 #pragma unroll
-    for (int r = 0; r < kScanItems; r++) {
-        const int i = base + r * kTpb;
+    for (int r = 0; r < kCplItems; r++) {
+        const int i = base + r * kCplTpb;
         key[r] = i < nb ? keys[i] : 0;
         // lane 0 also needs the key before the wave's, lane 63 the one after
         const int j = lane == 0 ? i - 1 : i + 1;
@@ -1162,8 +1219,8 @@ __global__ __launch_bounds__(kTpb) void k_cpl(const uint64_t *__restrict__ keys,
     uint32_t sum = 0;
     int low = 255;
 #pragma unroll
-    for (int r = 0; r < kScanItems; r++) {
-        const int i = base + r * kTpb;
+    for (int r = 0; r < kCplItems; r++) {
+        const int i = base + r * kCplTpb;
         const uint64_t after = __shfl_down(key[r], 1, 64);
         int c = -1;
         if (i + 1 < nb) c = min(kMaxLevel, (__clzll(key[r] ^ (lane == 63 ? edge[r] : after)) - 1) / 3);
@@ -1182,13 +1239,20 @@ __global__ __launch_bounds__(kTpb) void k_cpl(const uint64_t *__restrict__ keys,
         if (lane == 0 && i < nb) m1[i >> 6] = (uint8_t)m;
         low = min(low, m);
     }
-    if (lane == 0) wmin[w] = low;
-    uint32_t tot;
-    block_excl_scan(sum, &tot);
-    if (threadIdx.x == 0) {
-        part[blockIdx.x] = tot;
 #pragma unroll
-        for (int k = 1; k < kTpb / 64; k++) low = min(low, wmin[k]);
+    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+    if (lane == 0) {
+        wmin[w] = low;
+        wsum[w] = sum;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int k = 1; k < kCplTpb / 64; k++) {
+            low = min(low, wmin[k]);
+            sum += wsum[k];
+        }
+        part[blockIdx.x] = sum;
         m2[blockIdx.x] = (uint8_t)low;
     }
 }
@@ -2472,10 +2536,13 @@ void radix_sort_pairs(bh_ctx *ctx, uint64_t *k0, uint64_t *k1, uint32_t *v0, uin
     *vout = va;
 }
 
-// Merge passes over sorted tiles up to this many keys, radix passes beyond: 75
-// against 102 us at 10^5, 103 against 129 at 3 10^5, 174 against 166 at 2^20, 303
-// against 236 at 2^21 (keys and sort; a merge pass more per doubling, where the
-// radix passes stream).
+// Merge passes over sorted tiles up to kMergeMax keys, radix passes beyond (keys
+// and sort, us): 73 against 102 at 10^5, 98 against 129 at 3 10^5, 144 against
+// 166 at 2^20; a merge pass more per doubling, where the radix passes stream (at
+// 2^21, with an earlier k_merge, 303 against 236).  Up to kRankMax four runs at a
+// time: 44 against 53 at 2 10^4, 59 against 73 at 10^5, 105 against 111 at 5.2
+// 10^5, but 146 against 138 at 7 10^5.
+constexpr int64_t kRankMax = 1 << 19;
 constexpr int64_t kMergeMax = 1 << 20;
 
 // Sorts n Morton keys with their indices: of the bodies at pos (mass and pk as
@@ -2488,11 +2555,17 @@ static void sort_keys(bh_ctx *ctx, const double *pos, const double *mass, int64_
     hipStream_t st = ctx->stream;
     unsigned long long *stat = ptr<unsigned long long>(ctx->counters);
     if (n <= kMergeMax) {
-        const int tiles = (int)((n + kSortTile - 1) / kSortTile);
+        const int tiles = (int)((n + kMergeRun - 1) / kMergeRun);
         uint64_t *ka = k1, *kb = k0;
         uint32_t *va = v1, *vb = v0;
-        k_tile_sort<<<tiles, kSortTpb, 0, st>>>(pos, mass, n, box, k0, ka, va, pk, boxi, stat);
-        for (int64_t run = kSortTile; run < n; run *= 2) {
+        k_tile_sort<<<tiles, kTileTpb, 0, st>>>(pos, mass, n, box, k0, ka, va, pk, boxi, stat);
+        if (n <= kRankMax)
+            for (int lrun = kLogRun; 1 << lrun < n; lrun += 2) {
+                k_rank_merge<<<nblocks(n), kTpb, 0, st>>>(ka, va, kb, vb, (int)n, lrun);
+                std::swap(ka, kb);
+                std::swap(va, vb);
+            }
+        else for (int64_t run = kMergeRun; run < n; run *= 2) {
             k_merge<<<(int)((n + kMergeTile - 1) / kMergeTile), kTpb, 0, st>>>(ka, va, kb, vb, n, run);
             std::swap(ka, kb);
             std::swap(va, vb);
@@ -2569,7 +2642,7 @@ static void topo_scan(bh_ctx *ctx, const TopoBufs &b, const uint64_t *keys)
 {
     hipStream_t st = ctx->stream;
     const int n2 = (b.n + kScanChunk - 1) / kScanChunk;
-    k_cpl<<<n2, kTpb, 0, st>>>(keys, b.n, b.t.cpl, b.cq, b.ccnt, b.part, b.m1, b.m2);
+    k_cpl<<<n2, kCplTpb, 0, st>>>(keys, b.n, b.t.cpl, b.cq, b.ccnt, b.part, b.m1, b.m2);
     const bool scanned = n2 > kScanFewParts;
     if (scanned) k_scan_top<<<1, kTpb, 0, st>>>(b.part, n2, b.part + n2 + 1, 0);
     k_cbase<<<n2, kTpb, 0, st>>>(b.ccnt, b.t.cbase, b.n, b.part, scanned, b.m2, n2, b.m3, b.clamp);

@@ -89,7 +89,8 @@ def test_build_at_the_lines(eng, n, kind):
     check(eng, m, x, 4.0)
 
 
-@pytest.mark.parametrize("n", [(1 << 20) - 1, 1 << 20, (1 << 20) + 1])
+@pytest.mark.parametrize("n", [4097, 8191, 8192, 16385, 65535, 65536, 65537, 262145, 1 << 19, (1 << 19) + 1, (1 << 20) - 1, 1 << 20,
+                               (1 << 20) + 1])
 def test_merge_and_radix_sort_at_their_line(eng, n):
     m, x = bodies(n, "massless")
     eng.upload(m, x)
