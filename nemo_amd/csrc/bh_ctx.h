@@ -32,7 +32,7 @@ struct bh_ctx {
     // second stream of the tree build (same priority): branches that no
     // kernel of the main stream needs until the matching join
     hipStream_t side = nullptr;
-    hipEvent_t fork_ev[4] = {};
+    hipEvent_t fork_ev[6] = {};
     std::string err;
     int inject = 0;
 

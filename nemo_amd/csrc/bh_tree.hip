@@ -2548,11 +2548,11 @@ constexpr int64_t kMergeMax = 1 << 20;
 // Sorts n Morton keys with their indices: of the bodies at pos (mass and pk as
 // in k_tile_sort) in the box, or (pos null) the keys in k0.  k0/k1, v0/v1: two
 // buffers each; the sorted arrays are one of each.
-static void sort_keys(bh_ctx *ctx, const double *pos, const double *mass, int64_t n, const double4 *box, double4 *pk,
+// (radix passes run on the main stream only: they share its scratch)
+static void sort_keys(bh_ctx *ctx, hipStream_t st, const double *pos, const double *mass, int64_t n, const double4 *box, double4 *pk,
                       const int *boxi, uint64_t *k0, uint64_t *k1, uint32_t *v0, uint32_t *v1, uint64_t **kout,
                       uint32_t **vout)
 {
-    hipStream_t st = ctx->stream;
     unsigned long long *stat = ptr<unsigned long long>(ctx->counters);
     if (n <= kMergeMax) {
         const int tiles = (int)((n + kMergeRun - 1) / kMergeRun);
@@ -2665,7 +2665,7 @@ static void topo_cells(bh_ctx *ctx, const TopoBufs &b)
 constexpr int kSmallMax = kSmallTpb * 6;
 
 template <bool BOX>
-static void small_front(bh_ctx *ctx, const double *pos, const double *mass, int n, int nb, const BoxStart &start, int rounds,
+static void small_front(bh_ctx *ctx, hipStream_t st, const double *pos, const double *mass, int n, int nb, const BoxStart &start, int rounds,
                         double4 *box, uint32_t *lwork, int nlwork, uint64_t *keys, uint32_t *vals, const TopoBufs *b)
 {
     unsigned long long *stat = ptr<unsigned long long>(ctx->counters);
@@ -2679,7 +2679,7 @@ static void small_front(bh_ctx *ctx, const double *pos, const double *mass, int 
         cc = b->clamp;
     }
     auto go = [&](auto kernel) {
-        kernel<<<1, kSmallTpb, 0, ctx->stream>>>(pos, mass, n, b ? nb : 0, start, rounds, box, stat, S_ZERO, lwork, nlwork,
+        kernel<<<1, kSmallTpb, 0, st>>>(pos, mass, n, b ? nb : 0, start, rounds, box, stat, S_ZERO, lwork, nlwork,
                                                  out, cc);
     };
     if (n <= 2 * kSmallTpb) go(k_front<2, BOX>);
@@ -2751,7 +2751,7 @@ void fill_moments(bh_ctx *ctx)
 // far on ctx->side; main_wait(k): the main stream waits for that mark.
 // Under graph capture the side stream joins the capture through the forked
 // event and every branch is joined back before the build returns.
-enum { kForkSort = 0, kMarkGather = 1, kForkTopo = 2, kMarkLevels = 3 };
+enum { kForkSort = 0, kMarkGather = 1, kForkTopo = 2, kMarkLevels = 3, kForkBox = 4, kMarkTest = 5 };
 
 static void side_fork(bh_ctx *ctx, int k)
 {
@@ -2792,6 +2792,41 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
     const BoxStart start{r0, r1, r2, p.rsize, keep ? 1 : 0};
     const int rounds = std::max(1, keep ? ctx->box_rounds_keep : ctx->box_rounds);
 
+    // -- the test set's own keys and order in the tree's box (and its cells, when
+    //    one block does it all): on the second stream beside the mass set's, so
+    //    far as both need no scratch in common
+    const int64_t nt = ctx->ntest;
+    const bool alias = ctx->self_test && nt == nb;
+    const double *d_tpos = ctx->self_test ? d_pos : ptr<double>(ctx->tpos);
+    // groups of a test set with its own order (fast mode): at most G points
+    // are one group (a cell only cuts groups for children of a cell holding
+    // more than G points; batches, whose test set is the tree's, keep one
+    // group per system); more are cut from the topology of their own keys
+    const int G = p.mode == BH_MODE_FAST ? (p.group_size > 0 ? p.group_size : 64) : 0;
+    const bool tset_topo = !alias && G > 0 && nt > G && nt >= 2;
+    TopoBufs ttb{};
+    if (tset_topo && ctx->tcell_cap == 0) ctx->tcell_cap = (int)std::min<int64_t>(2 * nt + 64, INT32_MAX / 2);
+    uint64_t *tks = nullptr;
+    uint32_t *tvs = nullptr;
+    const bool beside = nt <= kMergeMax;
+    auto sort_tests = [&]() {
+        if (alias) return;
+        uint64_t *tk0 = ensure<uint64_t>(ctx->tkeys0, nt), *tk1 = ensure<uint64_t>(ctx->tkeys1, nt);
+        uint32_t *tv0 = ensure<uint32_t>(ctx->tvals0, nt), *tv1 = ensure<uint32_t>(ctx->tvals1, nt);
+        if (tset_topo && nt <= kSmallMax) ttb = topo_alloc(ctx, (int)nt, ctx->tcell_cap, true);
+        if (beside) side_fork(ctx, kForkBox);
+        hipStream_t ts = beside ? ctx->side : st;
+        if (nt <= kSmallMax) {
+            small_front<false>(ctx, ts, d_tpos, nullptr, (int)nt, (int)nt, start, 0, d_box, nullptr, 0, tk0, tv0,
+                               tset_topo ? &ttb : nullptr);
+            tks = tk0;
+            tvs = tv0;
+        } else {
+            sort_keys(ctx, ts, d_tpos, nullptr, nt, d_box, nullptr, nullptr, tk0, tk1, tv0, tv1, &tks, &tvs);
+        }
+        if (beside) side_mark(ctx, kMarkTest);
+    };
+
     // -- box, keys and sort of the mass set (massless bodies sort last); small
     //    sets in one launch, with the scans of the topology
     uint64_t *k0 = ensure<uint64_t>(ctx->keys0, n), *k1 = ensure<uint64_t>(ctx->keys1, n);
@@ -2805,10 +2840,11 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
     uint32_t *vs;
     if (small) {
         if (timing) BH_HIP(hipEventRecord(ctx->ev[6], st));
-        small_front<true>(ctx, d_pos, d_mass, (int)n, nb, start, 16 * rounds, d_box, lwork, nlwork, k0, v0,
+        small_front<true>(ctx, st, d_pos, d_mass, (int)n, nb, start, 16 * rounds, d_box, lwork, nlwork, k0, v0,
                           nb > 1 ? &tb : nullptr);
         ks = k0;
         vs = v0;
+        sort_tests();
     } else if (nsys) {
         k_build_start<<<1, 128, 0, st>>>(stat, S_ZERO, lwork, nlwork);
         k_sys_box<<<nsys, kTpb, 0, st>>>(d_pos, sysoff, sysbox, d_box, r0, r1, r2, p.rsize, keep ? 1 : 0,
@@ -2817,7 +2853,8 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
         k_keys_batch<<<grid_n, kTpb, 0, st>>>(d_pos, n, sysoff, nsys, sysbox, ctx->sysbits, k0);
         k_sysroot_init<<<nblocks(nsys), kTpb, 0, st>>>(sysoff, nsys, ensure<int>(ctx->sysroot, nsys));
         if (timing) BH_HIP(hipEventRecord(ctx->ev[6], st));
-        sort_keys(ctx, nullptr, nullptr, n, d_box, nullptr, nullptr, k0, k1, v0, v1, &ks, &vs);
+        sort_tests();
+        sort_keys(ctx, st, nullptr, nullptr, n, d_box, nullptr, nullptr, k0, k1, v0, v1, &ks, &vs);
     } else {
         // from a fresh box the first bodies are expanded for by one block, the
         // others by passes over all
@@ -2831,7 +2868,8 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
                                                  pass == 1 ? kBoxFew : kBoxShort, stat);
         pk = ensure<double4>(ctx->bpk, n);
         if (timing) BH_HIP(hipEventRecord(ctx->ev[6], st));
-        sort_keys(ctx, d_pos, d_mass, n, d_box, pk, d_boxi, k0, k1, v0, v1, &ks, &vs);
+        sort_tests();
+        sort_keys(ctx, st, d_pos, d_mass, n, d_box, pk, d_boxi, k0, k1, v0, v1, &ks, &vs);
     }
     if (timing) BH_HIP(hipEventRecord(ctx->ev[7], st));
 
@@ -2890,9 +2928,7 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
     T.keys = ks;
     T.dbox = d_box;
 
-    // -- test set, sorted by its own keys in the same box
-    const int64_t nt = ctx->ntest;
-    const bool alias = ctx->self_test && nt == nb;
+    // -- test set in its own order
     float4 *thi = alias ? nullptr : ensure<float4>(ctx->thi, nt), *tlo = alias ? nullptr : ensure<float4>(ctx->tlo, nt);
     double4 *td = alias || p.mode == BH_MODE_FAST ? nullptr : ensure<double4>(ctx->td, nt);   // (the strict walk's)
     int *tself = alias ? nullptr : ensure<int>(ctx->tself, nt);
@@ -2903,14 +2939,6 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
     T.tself = tself;
     T.tinv = nullptr;
     T.selfmode = ctx->self_test ? 2 : 0;
-    // groups of a test set with its own order (fast mode): at most G points
-    // are one group (a cell only cuts groups for children of a cell holding
-    // more than G points; batches, whose test set is the tree's, keep one
-    // group per system); more are cut from the topology of their own keys
-    const int G = p.mode == BH_MODE_FAST ? (p.group_size > 0 ? p.group_size : 64) : 0;
-    const bool tset_topo = !alias && G > 0 && nt > G && nt >= 2;
-    TopoBufs ttb{};
-    if (tset_topo && ctx->tcell_cap == 0) ctx->tcell_cap = (int)std::min<int64_t>(2 * nt + 64, INT32_MAX / 2);
     if (alias) {
         // the test set is the tree's body set in the same order
         T.thi = bhi;
@@ -2926,20 +2954,7 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
         // tree's order), so each group stays compact in space; a test point
         // finds its tree body (self pair) through the inverse of the tree's
         // sort, and each tree body its test index through tinv.
-        uint64_t *tk0 = ensure<uint64_t>(ctx->tkeys0, nt), *tk1 = ensure<uint64_t>(ctx->tkeys1, nt);
-        uint32_t *tv0 = ensure<uint32_t>(ctx->tvals0, nt), *tv1 = ensure<uint32_t>(ctx->tvals1, nt);
-        const double *d_tpos = ctx->self_test ? d_pos : ptr<double>(ctx->tpos);
-        uint64_t *tks;
-        uint32_t *tvs;
-        if (nt <= kSmallMax) {
-            if (tset_topo) ttb = topo_alloc(ctx, (int)nt, ctx->tcell_cap, true);
-            small_front<false>(ctx, d_tpos, nullptr, (int)nt, (int)nt, start, 0, d_box, nullptr, 0, tk0, tv0,
-                               tset_topo ? &ttb : nullptr);
-            tks = tk0;
-            tvs = tv0;
-        } else {
-            sort_keys(ctx, d_tpos, nullptr, nt, d_box, nullptr, nullptr, tk0, tk1, tv0, tv1, &tks, &tvs);
-        }
+        if (beside) main_wait(ctx, kMarkTest);
         tks_for_groups = tks;
         T.tperm = tvs;
         int *tmap = nullptr, *tinv = nullptr;
