@@ -139,100 +139,10 @@ struct TmpDev {
     T *as() const { return static_cast<T *>(p); }
 };
 
-// Copies of small pageable host arrays go through page-locked memory of the
-// context: the runtime's own path for pageable memory takes 18 to 28 us for 16
-// to 48 KB and 110 us for 256 KB, a copy to or from page-locked memory 10 to 14
-// us and the host's memcpy 1 to 7.  Larger arrays (from kStageMax on the two are
-// alike) and arrays the caller has page-locked are copied directly.
-constexpr size_t kStageBytes = 2 << 20, kStageMax = 512 << 10;
-
-bool pageable(const void *p)
-{
-    hipPointerAttribute_t a;
-    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
-    (void)hipGetLastError();
-    return true;
-}
-
-// Room for a staged copy of the caller's array p, or null.
-char *stage_room(bh_ctx *ctx, const void *p, size_t bytes)
-{
-    if (!ctx->stage || bytes > kStageMax || ctx->stage_used + bytes > kStageBytes || !pageable(p)) return nullptr;
-    char *s = ctx->stage + ctx->stage_used;
-    ctx->stage_used += (bytes + 255) & ~(size_t)255;
-    return s;
-}
-
-void to_device(bh_ctx *ctx, void *dst, const void *src, size_t bytes)
-{
-    if (char *s = stage_room(ctx, src, bytes)) {
-        memcpy(s, src, bytes);
-        src = s;
-    }
-    BH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
-}
-
-// Device arrays on their way to the caller's (null: left out): start() queues
-// the staged copies, finish() hands them over after the stream has been waited
-// for and copies the others.
-struct Fetch {
-    struct Item {
-        void *to;
-        const void *from;
-        size_t bytes;
-        char *staged;
-    };
-    bh_ctx *ctx;
-    Item item[4];
-    int n = 0;
-    size_t base;               // of the staging memory left to start()
-
-    explicit Fetch(bh_ctx *c) : ctx(c), base(c->stage_used) {}
-    void add(void *to, const void *from, size_t bytes)
-    {
-        if (to) item[n++] = Item{to, from, bytes, nullptr};
-    }
-    void results(double *phi, double *acc)
-    {
-        add(phi, ctx->phi.p, ctx->ntest * sizeof(double));
-        add(acc, ctx->acc.p, 3 * ctx->ntest * sizeof(double));
-    }
-    void start()
-    {
-        ctx->stage_used = base;
-        for (int k = 0; k < n; k++) {
-            Item &i = item[k];
-            i.staged = stage_room(ctx, i.to, i.bytes);
-            if (i.staged) BH_HIP(hipMemcpyAsync(i.staged, i.from, i.bytes, hipMemcpyDeviceToHost, ctx->stream));
-        }
-    }
-    void finish()
-    {
-        bool wait = false;
-        for (int k = 0; k < n; k++)
-            if (!item[k].staged) {
-                BH_HIP(hipMemcpyAsync(item[k].to, item[k].from, item[k].bytes, hipMemcpyDeviceToHost, ctx->stream));
-                wait = true;
-            }
-        for (int k = 0; k < n; k++)
-            if (item[k].staged) memcpy(item[k].to, item[k].staged, item[k].bytes);
-        if (wait) BH_HIP(hipStreamSynchronize(ctx->stream));
-    }
-    void now()
-    {
-        start();
-        BH_HIP(hipStreamSynchronize(ctx->stream));
-        finish();
-        ctx->stage_used = base;
-    }
-};
-
 // A new upload replaces the bodies a leapfrog integrates: its state (vel,
 // acc_old sized for the old set) and captured step graph are void, and the
 // bh_lf_* calls report BH_ERR_STATE until bh_lf_init runs again.
-// wait: return with the copies done (else the caller waits for the stream).
-void upload(bh_ctx *ctx, int64_t nmass, const double *mass, const double *pos, int64_t ntest, const double *tpos,
-            bool wait = true)
+void upload(bh_ctx *ctx, int64_t nmass, const double *mass, const double *pos, int64_t ntest, const double *tpos)
 {
     if (nmass < 1) throw ApiFail(BH_ERR_ARG, "nmass must be >= 1");
     if (nmass > (int64_t)INT32_MAX / 2) throw ApiFail(BH_ERR_ARG, "nmass too large (max 2^30)");
@@ -252,28 +162,22 @@ void upload(bh_ctx *ctx, int64_t nmass, const double *mass, const double *pos, i
     ctx->ntest = self ? nmass : ntest;
     double *dm = bh::ensure<double>(ctx->mass, nmass);
     double *dp = bh::ensure<double>(ctx->pos, 3 * nmass);
-    if (ctx->stage_used) BH_HIP(hipStreamSynchronize(ctx->stream));   // (an upload that failed half way)
-    ctx->stage_used = 0;
-    to_device(ctx, dm, mass, nmass * sizeof(double));
-    to_device(ctx, dp, pos, 3 * nmass * sizeof(double));
+    BH_HIP(hipMemcpyAsync(dm, mass, nmass * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    BH_HIP(hipMemcpyAsync(dp, pos, 3 * nmass * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
     if (!self) {
         double *dt = bh::ensure<double>(ctx->tpos, 3 * ntest);
-        to_device(ctx, dt, tpos, 3 * ntest * sizeof(double));
+        BH_HIP(hipMemcpyAsync(dt, tpos, 3 * ntest * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
     }
     bh::ensure<double>(ctx->phi, ctx->ntest);
     bh::ensure<double>(ctx->acc, 3 * ctx->ntest);
-    if (wait) {
-        BH_HIP(hipStreamSynchronize(ctx->stream));
-        ctx->stage_used = 0;
-    }
+    BH_HIP(hipStreamSynchronize(ctx->stream));
     ctx->uploaded = true;
 }
 
 // One evaluation without host synchronisation, then one read-back of the
 // device status.  A capacity overflow (cells, walk frontier) or a box that
 // needed more expansion rounds grows the capacity and evaluates again.
-// res: results to fetch with the status.
-void eval(bh_ctx *ctx, const bh_params *p, bh_stats *st, Fetch *res = nullptr)
+void eval(bh_ctx *ctx, const bh_params *p, bh_stats *st)
 {
     check_params(p);
     if (!ctx->uploaded) throw ApiFail(BH_ERR_STATE, "bh_eval before bh_upload");
@@ -287,12 +191,7 @@ void eval(bh_ctx *ctx, const bh_params *p, bh_stats *st, Fetch *res = nullptr)
     if (ctx->nsys && q.criterion != BH_CRIT_HACK)
         throw ApiFail(BH_ERR_ARG, "batches use the hackcode1 criterion");
     if (ctx->cell_cap == 0) ctx->cell_cap = (int)std::min<int64_t>(2 * ctx->nb + 64, INT32_MAX / 2);
-    unsigned long long local[bh::S_NSLOTS + 4];
-    unsigned long long *stat = local;
-    if (ctx->stage && ctx->stage_used + sizeof local <= kStageBytes) {
-        stat = reinterpret_cast<unsigned long long *>(ctx->stage + ctx->stage_used);
-        if (res) res->base += (sizeof local + 255) & ~(size_t)255;
-    }
+    unsigned long long stat[bh::S_NSLOTS];
     double box[4];
     // plain fast walk: the tree-end event also starts the walk kernel and the
     // walk kernel's end event also ends the phase (fewer event records)
@@ -312,10 +211,9 @@ void eval(bh_ctx *ctx, const bh_params *p, bh_stats *st, Fetch *res = nullptr)
             bh::walk_fast(ctx, q);
         }
         if (!plain_fast) BH_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
-        BH_HIP(hipMemcpyAsync(stat, ctx->counters.p, sizeof local, hipMemcpyDeviceToHost, ctx->stream));
-        if (res) res->start();
+        BH_HIP(hipMemcpyAsync(stat, ctx->counters.p, sizeof stat, hipMemcpyDeviceToHost, ctx->stream));
+        BH_HIP(hipMemcpyAsync(box, ctx->dbox.p, sizeof box, hipMemcpyDeviceToHost, ctx->stream));
         BH_HIP(hipStreamSynchronize(ctx->stream));
-        memcpy(box, stat + bh::S_NSLOTS, sizeof box);
         ctx->box_valid = true;
         const unsigned long long f = stat[bh::S_FLAGS];
         if (f & bh::F_NONFINITE)
@@ -433,12 +331,11 @@ void lf_upload_state(bh_ctx *ctx, int64_t n, const double *vel)
 {
     double *dv = bh::ensure<double>(ctx->vel, 3 * n);
     double *da = bh::ensure<double>(ctx->acc_old, 3 * n);
-    to_device(ctx, dv, vel, 3 * n * sizeof(double));
+    BH_HIP(hipMemcpyAsync(dv, vel, 3 * n * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
     BH_HIP(hipMemsetAsync(da, 0, 3 * n * sizeof(double), ctx->stream));
     bh::ensure<int>(ctx->lfstep, 2);
     bh::lf_reset(ctx);
     BH_HIP(hipStreamSynchronize(ctx->stream));
-    ctx->stage_used = 0;
 }
 
 // Parameters of one leapfrog force pass: after the first step the box is kept.
@@ -506,10 +403,6 @@ bh_status bh_create(bh_ctx **out, int device)
     if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0)
         ctx->ncu = prop.multiProcessorCount;
     for (auto &e : ctx->ev) (void)hipEventCreate(&e);
-    if (hipHostMalloc(reinterpret_cast<void **>(&ctx->stage), kStageBytes) != hipSuccess) {
-        (void)hipGetLastError();
-        ctx->stage = nullptr;       // (small copies then go the runtime's way)
-    }
     *out = ctx;
     return BH_OK;
 }
@@ -521,7 +414,7 @@ void bh_destroy(bh_ctx *ctx)
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipStreamSynchronize(ctx->side);
     lf_drop_graph(ctx);
-    bh::DevBuf *bufs[] = {&ctx->mass,   &ctx->pos,    &ctx->tpos,   &ctx->dboxi,  &ctx->keys0,
+    bh::DevBuf *bufs[] = {&ctx->mass,   &ctx->pos,    &ctx->tpos,   &ctx->dbox,    &ctx->dboxi,  &ctx->keys0,
                           &ctx->keys1,  &ctx->vals0,  &ctx->vals1,  &ctx->hist,    &ctx->scan_tmp, &ctx->tkeys0,
                           &ctx->tkeys1, &ctx->tvals0, &ctx->tvals1, &ctx->bd,    &ctx->bpk,   &ctx->bhi,
                           &ctx->blo,    &ctx->thi,    &ctx->tlo,    &ctx->td,      &ctx->tself, &ctx->tinv, &ctx->tmap,
@@ -542,7 +435,6 @@ void bh_destroy(bh_ctx *ctx)
                           &ctx->mlp.res, &ctx->mlp.smeta};
     for (auto *b : bufs)
         if (b->p) (void)hipFree(b->p);
-    if (ctx->stage) (void)hipHostFree(ctx->stage);
     for (auto &e : ctx->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto &e : ctx->fork_ev)
@@ -582,9 +474,8 @@ bh_status bh_download(bh_ctx *ctx, double *phi, double *acc)
 {
     return guarded(ctx, [&] {
         if (!ctx->uploaded) throw ApiFail(BH_ERR_STATE, "bh_download before bh_upload");
-        Fetch f(ctx);
-        f.results(phi, acc);
-        f.now();
+        if (phi) BH_HIP(hipMemcpy(phi, ctx->phi.p, ctx->ntest * sizeof(double), hipMemcpyDeviceToHost));
+        if (acc) BH_HIP(hipMemcpy(acc, ctx->acc.p, 3 * ctx->ntest * sizeof(double), hipMemcpyDeviceToHost));
     });
 }
 
@@ -599,24 +490,13 @@ bh_status bh_force(bh_ctx *ctx, const bh_params *p, int64_t nmass, const double 
     return guarded(ctx, [&] {
         check_params(p);
         if (!phi || !acc) throw ApiFail(BH_ERR_ARG, "phi/acc is NULL");
-        // the uploads, the evaluation and the small results with one wait (also
-        // when a step fails: the caller's arrays are free again on return)
-        struct Wait {
-            bh_ctx *ctx;
-            ~Wait()
-            {
-                (void)hipStreamSynchronize(ctx->stream);
-                ctx->stage_used = 0;
-            }
-        } wait{ctx};
-        upload(ctx, nmass, mass, pos, ntest, tpos, false);
+        upload(ctx, nmass, mass, pos, ntest, tpos);
         ctx->box_valid = false;
         bh_params q = *p;
         q.keep_box = 0;
-        Fetch res(ctx);
-        res.results(phi, acc);
-        eval(ctx, &q, st, &res);
-        res.finish();
+        eval(ctx, &q, st);
+        BH_HIP(hipMemcpy(phi, ctx->phi.p, ctx->ntest * sizeof(double), hipMemcpyDeviceToHost));
+        BH_HIP(hipMemcpy(acc, ctx->acc.p, 3 * ctx->ntest * sizeof(double), hipMemcpyDeviceToHost));
     });
 }
 
@@ -758,11 +638,15 @@ bh_status bh_lf_force(bh_ctx *ctx, double *diag, int64_t *n2b, int64_t *nbc)
         double *dd = bh::ensure<double>(ctx->diag_buf, nd);
         long long *d2 = bh::ensure<long long>(ctx->n2b_buf, 1), *dc = bh::ensure<long long>(ctx->nbc_buf, 1);
         bh::lf_after_force(ctx, dd, d2, dc, false);
-        Fetch f(ctx);
-        f.add(diag, dd, nd * sizeof(double));
-        f.add(n2b, d2, sizeof(int64_t));
-        f.add(nbc, dc, sizeof(int64_t));
-        f.now();
+        std::vector<double> h(nd);
+        long long c[2];
+        BH_HIP(hipMemcpyAsync(h.data(), dd, nd * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+        BH_HIP(hipMemcpyAsync(&c[0], d2, sizeof(long long), hipMemcpyDeviceToHost, ctx->stream));
+        BH_HIP(hipMemcpyAsync(&c[1], dc, sizeof(long long), hipMemcpyDeviceToHost, ctx->stream));
+        BH_HIP(hipStreamSynchronize(ctx->stream));
+        if (diag) memcpy(diag, h.data(), nd * sizeof(double));
+        if (n2b) *n2b = c[0];
+        if (nbc) *nbc = c[1];
     });
 }
 
@@ -834,21 +718,19 @@ bh_status bh_lf_run(bh_ctx *ctx, int64_t nsteps, int use_graph, double *diag, in
                 bh::lf_after_force(ctx, dd, d2, dc, true);
             }
         }
-        unsigned long long h[bh::S_NSLOTS + 4];
+        unsigned long long h[bh::S_NSLOTS];
         double box[4];
-        Fetch f(ctx);
-        f.add(h, stat, sizeof h);
-        f.add(diag, dd, nd * nsteps * sizeof(double));
-        f.add(n2b, d2, nsteps * sizeof(int64_t));
-        f.add(nbc, dc, nsteps * sizeof(int64_t));
-        f.now();
-        memcpy(box, h + bh::S_NSLOTS, sizeof box);
+        BH_HIP(hipMemcpyAsync(h, stat, sizeof h, hipMemcpyDeviceToHost, st));
+        BH_HIP(hipMemcpyAsync(box, ctx->dbox.p, sizeof box, hipMemcpyDeviceToHost, st));
+        if (diag) BH_HIP(hipMemcpyAsync(diag, dd, nd * nsteps * sizeof(double), hipMemcpyDeviceToHost, st));
+        if (n2b) BH_HIP(hipMemcpyAsync(n2b, d2, nsteps * sizeof(int64_t), hipMemcpyDeviceToHost, st));
+        if (nbc) BH_HIP(hipMemcpyAsync(nbc, dc, nsteps * sizeof(int64_t), hipMemcpyDeviceToHost, st));
+        BH_HIP(hipStreamSynchronize(st));
         for (int k = 0; k < 4; k++) ctx->box[k] = box[k];
         ctx->lf_nstep += nsteps;
-        const unsigned long long flags = h[bh::S_STICKY] | h[bh::S_FLAGS];
-        if (flags & bh::F_NONFINITE)
-            throw ApiFail(BH_ERR_NONFINITE, "non-finite position of a massive body during the run");
-        if (flags & (bh::F_CELL_OVF | bh::F_TCELL_OVF | bh::F_BOX_OPEN | bh::F_FRONTIER)) {
+        const unsigned long long f = h[bh::S_STICKY] | h[bh::S_FLAGS];
+        if (f & bh::F_NONFINITE) throw ApiFail(BH_ERR_NONFINITE, "non-finite position of a massive body during the run");
+        if (f & (bh::F_CELL_OVF | bh::F_TCELL_OVF | bh::F_BOX_OPEN | bh::F_FRONTIER)) {
             lf_drop_graph(ctx);
             throw ApiFail(BH_ERR_CAPACITY, "a step of the batch exceeded a capacity (cells, frontier or box rounds); "
                                            "the state is invalid: restart with bh_lf_init");
@@ -861,12 +743,10 @@ bh_status bh_lf_get(bh_ctx *ctx, double *pos, double *vel, double *acc, double *
     return guarded(ctx, [&] {
         if (!ctx->lf_ready) throw ApiFail(BH_ERR_STATE, "bh_lf_get before bh_lf_init");
         const int64_t n = ctx->nmass;
-        Fetch f(ctx);
-        f.add(pos, ctx->pos.p, 3 * n * sizeof(double));
-        f.add(vel, ctx->vel.p, 3 * n * sizeof(double));
-        f.add(acc, ctx->acc.p, 3 * n * sizeof(double));
-        f.add(phi, ctx->phi.p, n * sizeof(double));
-        f.now();
+        if (pos) BH_HIP(hipMemcpy(pos, ctx->pos.p, 3 * n * sizeof(double), hipMemcpyDeviceToHost));
+        if (vel) BH_HIP(hipMemcpy(vel, ctx->vel.p, 3 * n * sizeof(double), hipMemcpyDeviceToHost));
+        if (acc) BH_HIP(hipMemcpy(acc, ctx->acc.p, 3 * n * sizeof(double), hipMemcpyDeviceToHost));
+        if (phi) BH_HIP(hipMemcpy(phi, ctx->phi.p, n * sizeof(double), hipMemcpyDeviceToHost));
         if (nstep) *nstep = ctx->lf_nstep;
     });
 }
@@ -890,9 +770,8 @@ bh_status bh_batch_force(bh_ctx *ctx, const bh_params *p, int nsys, const int64_
         bh_params q = *p;
         q.keep_box = 0;
         eval(ctx, &q, st);
-        Fetch f(ctx);
-        f.results(phi, acc);
-        f.now();
+        BH_HIP(hipMemcpy(phi, ctx->phi.p, ctx->ntest * sizeof(double), hipMemcpyDeviceToHost));
+        BH_HIP(hipMemcpy(acc, ctx->acc.p, 3 * ctx->ntest * sizeof(double), hipMemcpyDeviceToHost));
     });
 }
 
@@ -1003,7 +882,7 @@ bh_status bh_lf_restore(bh_ctx *ctx, const double *acc, int64_t nstep, const dou
         ctx->lf_nstep = nstep;
         if (rmin) {
             const double b[4] = {rmin[0], rmin[1], rmin[2], rsize};
-            BH_HIP(hipMemcpy(bh::box_of(ctx), b, sizeof b, hipMemcpyHostToDevice));
+            BH_HIP(hipMemcpy(bh::ensure<double4>(ctx->dbox, 1), b, sizeof b, hipMemcpyHostToDevice));
             for (int k = 0; k < 4; k++) ctx->box[k] = b[k];
             ctx->box_valid = true;
         }
