@@ -142,7 +142,9 @@ struct TmpDev {
 // A new upload replaces the bodies a leapfrog integrates: its state (vel,
 // acc_old sized for the old set) and captured step graph are void, and the
 // bh_lf_* calls report BH_ERR_STATE until bh_lf_init runs again.
-void upload(bh_ctx *ctx, int64_t nmass, const double *mass, const double *pos, int64_t ntest, const double *tpos)
+// wait: return with the copies done (else the caller waits for the stream).
+void upload(bh_ctx *ctx, int64_t nmass, const double *mass, const double *pos, int64_t ntest, const double *tpos,
+            bool wait = true)
 {
     if (nmass < 1) throw ApiFail(BH_ERR_ARG, "nmass must be >= 1");
     if (nmass > (int64_t)INT32_MAX / 2) throw ApiFail(BH_ERR_ARG, "nmass too large (max 2^30)");
@@ -170,7 +172,7 @@ void upload(bh_ctx *ctx, int64_t nmass, const double *mass, const double *pos, i
     }
     bh::ensure<double>(ctx->phi, ctx->ntest);
     bh::ensure<double>(ctx->acc, 3 * ctx->ntest);
-    BH_HIP(hipStreamSynchronize(ctx->stream));
+    if (wait) BH_HIP(hipStreamSynchronize(ctx->stream));
     ctx->uploaded = true;
 }
 
@@ -191,7 +193,7 @@ void eval(bh_ctx *ctx, const bh_params *p, bh_stats *st)
     if (ctx->nsys && q.criterion != BH_CRIT_HACK)
         throw ApiFail(BH_ERR_ARG, "batches use the hackcode1 criterion");
     if (ctx->cell_cap == 0) ctx->cell_cap = (int)std::min<int64_t>(2 * ctx->nb + 64, INT32_MAX / 2);
-    unsigned long long stat[bh::S_NSLOTS];
+    unsigned long long stat[bh::S_NSLOTS + 4];
     double box[4];
     // plain fast walk: the tree-end event also starts the walk kernel and the
     // walk kernel's end event also ends the phase (fewer event records)
@@ -212,8 +214,8 @@ void eval(bh_ctx *ctx, const bh_params *p, bh_stats *st)
         }
         if (!plain_fast) BH_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
         BH_HIP(hipMemcpyAsync(stat, ctx->counters.p, sizeof stat, hipMemcpyDeviceToHost, ctx->stream));
-        BH_HIP(hipMemcpyAsync(box, ctx->dbox.p, sizeof box, hipMemcpyDeviceToHost, ctx->stream));
         BH_HIP(hipStreamSynchronize(ctx->stream));
+        memcpy(box, stat + bh::S_NSLOTS, sizeof box);
         ctx->box_valid = true;
         const unsigned long long f = stat[bh::S_FLAGS];
         if (f & bh::F_NONFINITE)
@@ -414,7 +416,7 @@ void bh_destroy(bh_ctx *ctx)
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipStreamSynchronize(ctx->side);
     lf_drop_graph(ctx);
-    bh::DevBuf *bufs[] = {&ctx->mass,   &ctx->pos,    &ctx->tpos,   &ctx->dbox,    &ctx->dboxi,  &ctx->keys0,
+    bh::DevBuf *bufs[] = {&ctx->mass,   &ctx->pos,    &ctx->tpos,   &ctx->dboxi,  &ctx->keys0,
                           &ctx->keys1,  &ctx->vals0,  &ctx->vals1,  &ctx->hist,    &ctx->scan_tmp, &ctx->tkeys0,
                           &ctx->tkeys1, &ctx->tvals0, &ctx->tvals1, &ctx->bd,    &ctx->bpk,   &ctx->bhi,
                           &ctx->blo,    &ctx->thi,    &ctx->tlo,    &ctx->td,      &ctx->tself, &ctx->tinv, &ctx->tmap,
@@ -490,11 +492,18 @@ bh_status bh_force(bh_ctx *ctx, const bh_params *p, int64_t nmass, const double 
     return guarded(ctx, [&] {
         check_params(p);
         if (!phi || !acc) throw ApiFail(BH_ERR_ARG, "phi/acc is NULL");
-        upload(ctx, nmass, mass, pos, ntest, tpos);
-        ctx->box_valid = false;
-        bh_params q = *p;
-        q.keep_box = 0;
-        eval(ctx, &q, st);
+        // (the evaluation waits for the uploads; when it fails they are waited
+        // for here, so that the caller's arrays are free again)
+        try {
+            upload(ctx, nmass, mass, pos, ntest, tpos, false);
+            ctx->box_valid = false;
+            bh_params q = *p;
+            q.keep_box = 0;
+            eval(ctx, &q, st);
+        } catch (...) {
+            (void)hipStreamSynchronize(ctx->stream);
+            throw;
+        }
         BH_HIP(hipMemcpy(phi, ctx->phi.p, ctx->ntest * sizeof(double), hipMemcpyDeviceToHost));
         BH_HIP(hipMemcpy(acc, ctx->acc.p, 3 * ctx->ntest * sizeof(double), hipMemcpyDeviceToHost));
     });
@@ -721,7 +730,7 @@ bh_status bh_lf_run(bh_ctx *ctx, int64_t nsteps, int use_graph, double *diag, in
         unsigned long long h[bh::S_NSLOTS];
         double box[4];
         BH_HIP(hipMemcpyAsync(h, stat, sizeof h, hipMemcpyDeviceToHost, st));
-        BH_HIP(hipMemcpyAsync(box, ctx->dbox.p, sizeof box, hipMemcpyDeviceToHost, st));
+        BH_HIP(hipMemcpyAsync(box, bh::box_of(ctx), sizeof box, hipMemcpyDeviceToHost, st));
         if (diag) BH_HIP(hipMemcpyAsync(diag, dd, nd * nsteps * sizeof(double), hipMemcpyDeviceToHost, st));
         if (n2b) BH_HIP(hipMemcpyAsync(n2b, d2, nsteps * sizeof(int64_t), hipMemcpyDeviceToHost, st));
         if (nbc) BH_HIP(hipMemcpyAsync(nbc, dc, nsteps * sizeof(int64_t), hipMemcpyDeviceToHost, st));
@@ -882,7 +891,7 @@ bh_status bh_lf_restore(bh_ctx *ctx, const double *acc, int64_t nstep, const dou
         ctx->lf_nstep = nstep;
         if (rmin) {
             const double b[4] = {rmin[0], rmin[1], rmin[2], rsize};
-            BH_HIP(hipMemcpy(bh::ensure<double4>(ctx->dbox, 1), b, sizeof b, hipMemcpyHostToDevice));
+            BH_HIP(hipMemcpy(bh::box_of(ctx), b, sizeof b, hipMemcpyHostToDevice));
             for (int k = 0; k < 4; k++) ctx->box[k] = b[k];
             ctx->box_valid = true;
         }

@@ -46,8 +46,7 @@ struct bh_ctx {
 
     // inputs (device, input order)
     bh::DevBuf mass, pos, tpos;
-    // box state: double4 box, ints {first, start, changed, nonfinite}
-    bh::DevBuf dbox, dboxi, bcand;
+    bh::DevBuf dboxi, bcand;   // box expansion: its words (bh_tree.hip) and the bodies outside
     // sorting
     bh::DevBuf keys0, keys1, vals0, vals1, hist, scan_tmp;
     bh::DevBuf tkeys0, tkeys1, tvals0, tvals1;
@@ -143,6 +142,11 @@ T *ensure(DevBuf &b, size_t count)
 
 template <class T>
 T *ptr(DevBuf &b) { return static_cast<T *>(b.p); }
+
+// The status words and, behind them, the root box: one read-back for both (a
+// copy to pageable memory takes ~20 us, however small).
+inline unsigned long long *status_of(bh_ctx *ctx) { return ensure<unsigned long long>(ctx->counters, S_NSLOTS + 4); }
+inline double4 *box_of(bh_ctx *ctx) { return reinterpret_cast<double4 *>(status_of(ctx) + S_NSLOTS); }
 
 // bh_tree.hip
 void build_tree(bh_ctx *ctx, const bh_params &p);

@@ -276,7 +276,7 @@ void lf_reset_record(bh_ctx *ctx)
 {
     double *partial = ensure<double>(ctx->diag_partial, 36 * (size_t)kDiagBlocks + 1);
     k_lf_begin<<<1, 1, 0, ctx->stream>>>(ptr<int>(ctx->lfstep) + 1,
-                                         ensure<unsigned long long>(ctx->counters, S_NSLOTS),
+                                         status_of(ctx),
                                          reinterpret_cast<unsigned *>(partial + 36 * (size_t)kDiagBlocks));
     BH_HIP(hipGetLastError());
 }

@@ -2727,7 +2727,7 @@ static void one_group(bh_ctx *ctx, int64_t n, int G)
 // Morton keys of the mass set in input order, in the current box.
 void debug_keys(bh_ctx *ctx, uint64_t *d_out)
 {
-    double4 *d_box = ensure<double4>(ctx->dbox, 1);
+    double4 *d_box = box_of(ctx);
     k_keys<<<nblocks(ctx->nmass), kTpb, 0, ctx->stream>>>(ptr<double>(ctx->pos), ptr<double>(ctx->mass), ctx->nmass,
                                                           d_box, d_out, nullptr);
     BH_HIP(hipStreamSynchronize(ctx->stream));
@@ -2772,9 +2772,9 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
     const int64_t n = ctx->nmass;
     const int nb = (int)ctx->nb;
     double *d_pos = ptr<double>(ctx->pos), *d_mass = ptr<double>(ctx->mass);
-    double4 *d_box = ensure<double4>(ctx->dbox, 1);
+    double4 *d_box = box_of(ctx);
     int *d_boxi = ensure<int>(ctx->dboxi, 8);
-    unsigned long long *stat = ensure<unsigned long long>(ctx->counters, S_NSLOTS);
+    unsigned long long *stat = status_of(ctx);
     const bool timing = !ctx->capturing;
     // -- box: start from the caller's box (or the previous one) and expand in
     //    input order; a fixed number of rounds, checked afterwards
