@@ -326,37 +326,45 @@ __global__ void k_build_start(unsigned long long *stat, int nzero, uint32_t *lwo
 
 // Start of a build and, from a fresh box, expandbox over the first kBoxFirst
 // bodies by one block: in input order these already reach most of a system's
-// extent, so few of the others are candidates for k_box_compact.
-constexpr int kFirstTpb = 1024, kFirstPer = 8, kBoxFirst = kFirstTpb * kFirstPer;
+// extent, so few of the others are candidates for k_box_compact.  solo: over all
+// bodies, from a kept box too (a chunk takes ~3 us, k_box_compact 9 and its
+// launch 2 to 4).
+constexpr int kFirstTpb = 1024, kFirstPer = 8, kBoxFirst = kFirstTpb * kFirstPer, kBoxSolo = 3 * kBoxFirst;
 __global__ __launch_bounds__(kFirstTpb) void k_box_first(const double *__restrict__ pos, const double *__restrict__ mass,
-                                                         int64_t n, BoxStart st, int rounds, double4 *box, int *boxi,
-                                                         unsigned long long *stat, int nzero, uint32_t *lwork, int nlwork)
+                                                         int64_t n, BoxStart st, int rounds, bool solo, double4 *box,
+                                                         int *boxi, unsigned long long *stat, int nzero, uint32_t *lwork,
+                                                         int nlwork)
 {
     __shared__ BoxPick pick;
     build_start(stat, nzero, lwork, nlwork);
     __syncthreads();
     double4 b = st.keep ? *box : make_double4(st.rx, st.ry, st.rz, st.rsize);
-    if (!st.keep) {
-        double x[kFirstPer][3];
+    const int64_t end = solo ? n : st.keep ? 0 : min(n, (int64_t)kBoxFirst);
+    bool closed = true;
+    for (int64_t base = 0; base < end && closed; base += kBoxFirst) {
+        double x[kFirstPer][3], m[kFirstPer];
         unsigned mask = 0;
-        const int first = (threadIdx.x >> 6) * kFirstPer * 64 + lane_id();
+        const int first = (int)base + (threadIdx.x >> 6) * kFirstPer * 64 + lane_id();
 #pragma unroll
         for (int r = 0; r < kFirstPer; r++) {
             const int64_t i = min<int64_t>(first + r * 64, n - 1);
-            if (first + r * 64 < n && mass[i] != 0.0) mask |= 1u << r;
+            m[r] = mass[i];
 #pragma unroll
             for (int k = 0; k < 3; k++) x[r][k] = pos[3 * i + k];
         }
-        // (not closed within the rounds: the bodies left outside stay
-        // candidates only if k_box_compact starts over, so flag it)
-        if (!box_rounds<kFirstTpb, kFirstPer>(x, mask, first, b, rounds, pick, stat) && threadIdx.x == 0)
-            atomicOr(&stat[S_FLAGS], (unsigned long long)F_BOX_OPEN);
+#pragma unroll
+        for (int r = 0; r < kFirstPer; r++)
+            if (first + r * 64 < n && m[r] != 0.0) mask |= 1u << r;
+        closed = box_rounds<kFirstTpb, kFirstPer>(x, mask, first, b, rounds, pick, stat);
     }
     if (threadIdx.x == 0) {
-        if (!st.keep) *box = b;
+        // (not closed within the rounds: the host grows their number)
+        if (!closed) atomicOr(&stat[S_FLAGS], (unsigned long long)F_BOX_OPEN);
+        if (!st.keep || solo) *box = b;
         boxi[0] = INT32_MAX;
-        boxi[1] = st.keep ? 0 : (int)min(n, (int64_t)kBoxFirst);
+        boxi[1] = (int)end;
         for (int k = 2; k < 7; k++) boxi[k] = 0;
+        if (solo) boxi[5] = 1;
     }
 }
 
@@ -1338,41 +1346,58 @@ __device__ __forceinline__ uint64_t below(const uint8_t *__restrict__ a, int k, 
     return (x - nl) & ~x & 0x8080808080808080ULL;
 }
 
-// First j >= s with cpl[j] < L (exists: cpl[nb-1] = -1), i.e. cq[j] < L + 1.
-// Each level of the minima pyramid (m1: 64 bodies, m2: 4096, m3: 262144 per
-// entry; all in the cq domain, 8-byte aligned, one word of padding) is read
-// eight entries at a time: at an aligned position the word either lets the
-// search skip up to eight blocks whose minimum is >= L, or names the first
-// block holding an entry below L, which the next finer level then searches.
-// At most ~8 words per level going up and down.
+// First entry from k on, within k's aligned block of 64, that is below L + 1
+// (nl), or -1: one round trip for the block (a is 64-byte aligned).
+__device__ __forceinline__ int below64(const uint8_t *__restrict__ a, int k, uint64_t nl)
+{
+    const int base = k & ~63, w0 = (k & 63) >> 3;
+    uint64_t x[8];
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+        const ulonglong2 q = reinterpret_cast<const ulonglong2 *>(a + base)[w];
+        x[2 * w] = q.x;
+        x[2 * w + 1] = q.y;
+    }
+    const int sh = (k & 7) * 8;
+    const uint64_t head = sh ? 0x7f7f7f7f7f7f7f7fULL & ((1ULL << sh) - 1) : 0;
+    int r = -1;
+#pragma unroll
+    for (int w = 7; w >= 0; w--) {
+        const uint64_t v = w == w0 ? x[w] | head : x[w];
+        const uint64_t t = (v - nl) & ~v & 0x8080808080808080ULL;
+        if (w >= w0 && t) r = base + 8 * w + (__builtin_ctzll(t) >> 3);
+    }
+    return r;
+}
+
+// First j >= s with cpl[j] < L (exists: cpl[nb-1] = -1), i.e. cq[j] < L + 1: in
+// s's word (most cells end there), then in its block of 64, then in the blocks
+// that the minima pyramid names (m1: 64 bodies, m2: 4096, m3: 262144 per entry;
+// all in the cq domain, 64-byte aligned with a block of padding; what lies in the
+// padding is never reached, the last entry of every level being 0).  A chain of
+// at most 5 round trips up to 262144 bodies; reading the blocks a word at a time
+// made it 20, and k_cells 15 us at 10^4 bodies, where few waves hide them.
 __device__ int range_end(const uint8_t *__restrict__ cq, const uint8_t *__restrict__ m1,
                          const uint8_t *__restrict__ m2, const uint8_t *__restrict__ m3, int s, int L)
 {
     const uint64_t nl = 0x0101010101010101ULL * (uint64_t)(L + 1);
-    int j = s;
-    for (;;) {
-        if ((j & 262143) == 0) {
-            const int k = j >> 18;
-            const uint64_t t = below(m3, k, nl);
-            if (!t) { j = ((k | 7) + 1) << 18; continue; }
-            j = ((k & ~7) + (__builtin_ctzll(t) >> 3)) << 18;
+    const uint64_t t = below(cq, s, nl);
+    if (t) return (s & ~7) + (__builtin_ctzll(t) >> 3);
+    int r = (s & 63) < 56 ? below64(cq, (s | 7) + 1, nl) : -1;
+    if (r >= 0) return r;
+    const int k = (s >> 6) + 1;
+    r = below64(m1, k, nl);
+    if (r < 0) {
+        const int k2 = (k >> 6) + 1;
+        int r2 = below64(m2, k2, nl);
+        if (r2 < 0) {
+            int k3 = (k2 >> 6) + 1, r3;
+            while ((r3 = below64(m3, k3, nl)) < 0) k3 = (k3 | 63) + 1;
+            r2 = below64(m2, r3 << 6, nl);
         }
-        if ((j & 4095) == 0) {
-            const int k = j >> 12;
-            const uint64_t t = below(m2, k, nl);
-            if (!t) { j = ((k | 7) + 1) << 12; continue; }
-            j = ((k & ~7) + (__builtin_ctzll(t) >> 3)) << 12;
-        }
-        if ((j & 63) == 0) {
-            const int k = j >> 6;
-            const uint64_t t = below(m1, k, nl);
-            if (!t) { j = ((k | 7) + 1) << 6; continue; }
-            j = ((k & ~7) + (__builtin_ctzll(t) >> 3)) << 6;
-        }
-        const uint64_t t = below(cq, j, nl);
-        if (t) return (j & ~7) + (__builtin_ctzll(t) >> 3);
-        j = (j | 7) + 1;
+        r = below64(m1, r2 << 6, nl);
     }
+    return below64(cq, r << 6, nl);
 }
 
 // The whole front of a small build in one block (n <= T * I): BOX: the start of
@@ -1384,10 +1409,10 @@ constexpr int kSmallTpb = 1024;
 template <int I>
 struct SmallFront {
     BlockSort<kSmallTpb, I, uint16_t> S;
-    // cpl + 1 and its minima, read eight entries at a time (range_end)
-    __attribute__((aligned(8))) uint8_t cq[kSmallTpb * I + 64];
-    __attribute__((aligned(8))) uint8_t m1[kSmallTpb * I / 64 + 8];
-    __attribute__((aligned(8))) uint8_t m2[16], m3[16];
+    // cpl + 1 and its minima, read 64 entries at a time (range_end)
+    __attribute__((aligned(64))) uint8_t cq[kSmallTpb * I + 64];
+    __attribute__((aligned(64))) uint8_t m1[(kSmallTpb * I / 64 + 127) & ~63];
+    __attribute__((aligned(64))) uint8_t m2[64], m3[64];
     uint32_t wsum[kSmallTpb / 64];
     BoxPick pick;
 };
@@ -1656,8 +1681,10 @@ __device__ __forceinline__ int child_end(int c, int s, int e, int t, int L, cons
                                          int *cc)
 {
     *cc = -1;
-    if (cpl[t] < L + 1) return t + 1;
-    const int k = (t == s) ? c + 1 : (int)cbase[t];
+    const int shared = cpl[t], first = (int)cbase[t];   // (one round trip: both loads before the branch)
+    __builtin_amdgcn_sched_barrier(0);
+    if (shared < L + 1) return t + 1;
+    const int k = (t == s) ? c + 1 : first;
     if (k >= ncell) return e + 1;
     *cc = k;
     const int tn = clast[k] + 1;
@@ -2611,17 +2638,16 @@ static TopoBufs topo_alloc(bh_ctx *ctx, int n, int cap, bool tset)
     b.n = n;
     b.t.cap = cap;
     b.t.ncellp = stat + (tset ? S_TNCELL : S_NCELL);
-    b.t.cpl = ensure<int8_t>(tset ? ctx->gcpl : ctx->cpl, 2 * (size_t)n + 32);
-    b.cq = reinterpret_cast<uint8_t *>(b.t.cpl) + ((n + 15) & ~7);   // 8-aligned, n + 8 bytes
+    // the bytes that range_end reads: 64-byte aligned, a block of padding behind
+    auto blocks = [](int v) { return ((size_t)v + 127) & ~(size_t)63; };
+    b.t.cpl = ensure<int8_t>(tset ? ctx->gcpl : ctx->cpl, 2 * blocks(n));
+    b.cq = reinterpret_cast<uint8_t *>(b.t.cpl) + blocks(n);
     b.ccnt = ensure<uint32_t>(tset ? ctx->gccnt : ctx->ccnt, n + 1);
     b.t.cbase = ensure<uint32_t>(tset ? ctx->gcbase : ctx->cbase, n + 1);
     const int n1 = (n + 63) / 64, n2 = (n1 + 63) / 64, n3 = (n2 + 63) / 64;
-    // each level 8-byte aligned with at least one word of padding (the
-    // search reads whole words; it stops at the entry holding cpl[n-1] = -1)
-    auto words = [](int v) { return (v + 15) & ~7; };
-    b.m1 = reinterpret_cast<uint8_t *>(ensure<int8_t>(tset ? ctx->gm1 : ctx->cmin1, words(n1) + words(n2) + words(n3)));
-    b.m2 = b.m1 + words(n1);
-    b.m3 = b.m2 + words(n2);
+    b.m1 = reinterpret_cast<uint8_t *>(ensure<int8_t>(tset ? ctx->gm1 : ctx->cmin1, blocks(n1) + blocks(n2) + blocks(n3)));
+    b.m2 = b.m1 + blocks(n1);
+    b.m3 = b.m2 + blocks(n2);
     b.part = ensure<uint32_t>(ctx->scan_tmp, n2 + 2);
     b.t.first = ensure<int>(tset ? ctx->gcf : ctx->cfirst, cap);
     b.t.last = ensure<int>(tset ? ctx->gcl : ctx->clast, cap);
@@ -2858,12 +2884,13 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
     } else {
         // from a fresh box the first bodies are expanded for by one block, the
         // others by passes over all
-        k_box_first<<<1, kFirstTpb, 0, st>>>(d_pos, d_mass, n, start, 16 * rounds, d_box, d_boxi, stat, S_ZERO, lwork,
-                                             nlwork);
+        const bool solo = n <= kBoxSolo;
+        k_box_first<<<1, kFirstTpb, 0, st>>>(d_pos, d_mass, n, start, 16 * rounds, solo, d_box, d_boxi, stat, S_ZERO,
+                                             lwork, nlwork);
         const int64_t i0 = keep ? 0 : std::min<int64_t>(n, kBoxFirst);
         double4 *cand = ensure<double4>(ctx->bcand, n);
         const int grid = std::max(1, (int)((n - i0 + kBoxChunk - 1) / kBoxChunk));
-        for (int pass = n - i0 > kBoxOne ? std::max(2, rounds / 4) : 1; pass > 0; pass--)
+        for (int pass = solo ? 0 : n - i0 > kBoxOne ? std::max(2, rounds / 4) : 1; pass > 0; pass--)
             k_box_compact<<<grid, kTpb, 0, st>>>(d_pos, d_mass, i0, n, d_box, cand, d_boxi, 16 * rounds,
                                                  pass == 1 ? kBoxFew : kBoxShort, stat);
         pk = ensure<double4>(ctx->bpk, n);
