@@ -371,64 +371,36 @@ __global__ __launch_bounds__(kFirstTpb) void k_box_first(const double *__restric
 // ---- batched ensembles: one box per system -----------------------------------
 
 // expandbox for every system of a batch (one block each): from the caller's
-// box, or the system's previous box, take the first body in input order that
-// lies outside, double the box towards it (load.c:68-95), and go on from the
-// next body; every body of a batch is massive.  All threads compute the same
-// box.  A round scans forward from its start in chunks of kTpb * kSysBoxPer
-// bodies (all loads of a chunk in flight) and stops at the first chunk that
-// holds a body outside; the next round starts after that body, so all rounds
-// together read each body about once.  At most `rounds` expansions; a box
-// still open is flagged.
-constexpr int kSysBoxPer = 8;
+// box, or the system's previous box, over chunks of bodies held in registers
+// (box_rounds; every body of a batch is massive).  A box still open after
+// `rounds` expansions for one chunk is flagged.  The block of the largest system
+// is a chain of chunks: 1024 threads for systems of kSysWide bodies on average
+// (512 systems of 256 to 65536 bodies: 245 us with 256 threads), 256 for the
+// others, whose blocks share a CU.
+constexpr int kSysBoxPer = 8, kSysWide = 4096;
 
-__global__ __launch_bounds__(kTpb) void k_sys_box(const double *__restrict__ pos, const int64_t *__restrict__ off,
-                                                  double4 *sysbox, double4 *box0, double rx, double ry, double rz,
-                                                  double rsize, int keep, int rounds, unsigned long long *stat)
+template <int T>
+__global__ __launch_bounds__(T) void k_sys_box(const double *__restrict__ pos, const int64_t *__restrict__ off,
+                                               double4 *sysbox, double4 *box0, double rx, double ry, double rz,
+                                               double rsize, int keep, int rounds, unsigned long long *stat)
 {
-    __shared__ int red[kTpb / 64];
+    __shared__ BoxPick pick;
     const int s = blockIdx.x;
     const int lo = (int)off[s], hi = (int)off[s + 1];
     double4 b = keep ? sysbox[s] : make_double4(rx, ry, rz, rsize);
-    int start = lo;
-    bool closed = false;
-    for (int round = 0; round <= rounds; round++) {
-        const BoxTest bt = box_test(b);
-        int f = hi;
-        for (int c0 = start; c0 < hi && f == hi; c0 += kTpb * kSysBoxPer) {
-            int first = hi;
+    bool closed = true;
+    for (int base = lo; base < hi && closed; base += T * kSysBoxPer) {
+        double x[kSysBoxPer][3];
+        unsigned mask = 0;
+        const int first = base + (int)(threadIdx.x >> 6) * kSysBoxPer * 64 + lane_id();
 #pragma unroll
-            for (int k = 0; k < kSysBoxPer; k++) {
-                const int i = c0 + k * kTpb + (int)threadIdx.x;
-                if (i < hi && !fits(pos + 3 * (int64_t)i, bt)) first = min(first, i);
-            }
+        for (int r = 0; r < kSysBoxPer; r++) {
+            const int64_t i = min(first + r * 64, hi - 1);
+            if (first + r * 64 < hi) mask |= 1u << r;
 #pragma unroll
-            for (int d = 32; d >= 1; d >>= 1) first = min(first, __shfl_xor(first, d, 64));
-            if (lane_id() == 0) red[threadIdx.x >> 6] = first;
-            __syncthreads();
-            f = red[0];
-#pragma unroll
-            for (int k = 1; k < kTpb / 64; k++) f = min(f, red[k]);
-            __syncthreads();
+            for (int k = 0; k < 3; k++) x[r][k] = pos[3 * i + k];
         }
-        if (f == hi) {
-            closed = true;
-            break;
-        }
-        if (round == rounds) break;
-        const double *x = pos + 3 * (int64_t)f;
-        if (!(isfinite(x[0]) && isfinite(x[1]) && isfinite(x[2]))) {
-            if (threadIdx.x == 0) atomicOr(&stat[S_FLAGS], (unsigned long long)F_NONFINITE);
-            closed = true;
-            break;
-        }
-        for (int guard = 0; guard < 2000 && !fits(x, b); guard++) {
-            double rmid0 = b.x + 0.5 * b.w, rmid1 = b.y + 0.5 * b.w, rmid2 = b.z + 0.5 * b.w;
-            if (x[0] < rmid0) b.x -= b.w;
-            if (x[1] < rmid1) b.y -= b.w;
-            if (x[2] < rmid2) b.z -= b.w;
-            b.w = 2.0 * b.w;
-        }
-        start = f + 1;
+        closed = box_rounds<T, kSysBoxPer>(x, mask, first, b, rounds, pick, stat);
     }
     if (threadIdx.x == 0) {
         sysbox[s] = b;
@@ -2873,8 +2845,12 @@ void build_tree(bh_ctx *ctx, const bh_params &p)
         sort_tests();
     } else if (nsys) {
         k_build_start<<<1, 128, 0, st>>>(stat, S_ZERO, lwork, nlwork);
-        k_sys_box<<<nsys, kTpb, 0, st>>>(d_pos, sysoff, sysbox, d_box, r0, r1, r2, p.rsize, keep ? 1 : 0,
-                                         16 * ctx->box_rounds, stat);
+        if (n / nsys >= kSysWide)
+            k_sys_box<1024><<<nsys, 1024, 0, st>>>(d_pos, sysoff, sysbox, d_box, r0, r1, r2, p.rsize, keep ? 1 : 0,
+                                                   16 * ctx->box_rounds, stat);
+        else
+            k_sys_box<256><<<nsys, 256, 0, st>>>(d_pos, sysoff, sysbox, d_box, r0, r1, r2, p.rsize, keep ? 1 : 0,
+                                                 16 * ctx->box_rounds, stat);
         const int grid_n = (int)std::min<int64_t>(nblocks(n), (int64_t)ctx->ncu * 16);
         k_keys_batch<<<grid_n, kTpb, 0, st>>>(d_pos, n, sysoff, nsys, sysbox, ctx->sysbits, k0);
         k_sysroot_init<<<nblocks(nsys), kTpb, 0, st>>>(sysoff, nsys, ensure<int>(ctx->sysroot, nsys));

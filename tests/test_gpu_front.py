@@ -127,3 +127,25 @@ def test_separate_test_points(eng, nt):
     # the fast walk opens at least what the strict one opens per group: their
     # difference is within the tree's own error at this tolerance
     assert np.abs(phi / phi0 - 1).max() < 2e-2
+
+
+# (a mean of 4096 bodies is the line between the two widths of a system's block)
+@pytest.mark.parametrize("sizes", [(1, 2, 255, 2047, 2048, 2049, 300), (8191, 8192, 8193, 20000, 1, 64, 5000)])
+def test_systems_of_a_batch_get_the_box_of_their_own(eng, sizes):
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    parts = [bodies(k, "spread") for k in sizes]
+    for _, q in parts:          # grows the box late, to 2^7 (a batch has a level less: far from its depth)
+        for j, i in enumerate(range(len(q) - 1, len(q) // 2, -max(1, len(q) // 8))):
+            q[i] *= 2.0 ** (5 - j)
+    m, x = np.concatenate([q[0] for q in parts]), np.concatenate([q[1] for q in parts])
+    eng.batch_upload(off, m, x, np.full(len(sizes), 0.05), np.full(len(sizes), 0.8))
+    eng.eval(E.default_params())
+    phi, acc = eng.download()
+    for k, (ms, xs) in enumerate(parts):
+        if len(ms) < 3:
+            continue
+        eng.upload(ms, xs)
+        eng.eval(E.default_params(eps=0.05, tol=0.8))
+        p1, a1 = eng.download()
+        a, b = off[k], off[k + 1]
+        assert np.array_equal(phi[a:b], p1) and np.array_equal(acc[a:b], a1)
