@@ -104,7 +104,7 @@ typedef struct {
     double t_walk_ms;    /* device time: walk + interactions (+ MLP) */
     int64_t n_mlp;       /* learned corrections applied */
     double t_walk_kernel_ms; /* device time of the walk kernel launch alone */
-    double t_sort_ms;    /* device time of the mass-set key sort */
+    double t_sort_ms;    /* device time of the mass-set keys and their sort */
     int64_t ngroups;     /* fast mode: groups of test points walked */
     double t_mlp_ms;     /* learned mode: device time of the learned-correction kernel (MLP inference
                             and the per-group apply) */

@@ -946,10 +946,12 @@ void launch(bh_ctx *ctx, WalkArgs &a, int grid, bool crit)
 // against the device's CUs; walk times in us, quadrupole cells in brackets:
 //   one row per 8-wave team while the rows of all groups stay near one per CU
 //     (N = 10^4, groups of 128: 76 [87]; 8 waves per group 86 [111], one wave 391 [450]);
-//   8 waves per group up to 3 groups per CU (N = 5 10^4: 139 [191]; 4 waves
-//     190 [262], a row per team 177 [230], one wave 461 [626]);
-//   4 waves up to 16 per CU (N = 4 10^5: 683 [982]; 8 waves 737 [1013], one
-//     wave 749 [1028]; N = 2^20, groups of 256: 1541; one wave 1671);
+//   8 waves per group up to 6 groups per CU (N = 5 10^4: 139 [191]; 4 waves
+//     190 [262], a row per team 177 [230], one wave 461 [626]; 1.6 10^5: 349 [494],
+//     4 waves 373 [520]; 2 10^5: 413 [571], 422 [570]);
+//   4 waves up to 16 per CU (N = 3 10^5: 563 [775], 8 waves 572 [797]; 4 10^5: 683
+//     [982]; 8 waves 737 [1013], one wave 749 [1028]; N = 2^20, groups of 256:
+//     1541; one wave 1671);
 //   then one wave, whose tiles never wait for another's (N = 2^20, groups of
 //     128: 1559 [2090]; 4 waves 1595 [2251]; N = 2^22: 5640 [7070]; 6090 [8740]).
 struct Walkers {
@@ -961,7 +963,7 @@ Walkers walkers(const bh_ctx *ctx, const bh_params &p, int64_t nt, int K)
     if (K > 1) return {0, false};
     const int64_t e = std::max<int64_t>(nt / p.group_size, ctx->nsys), ncu = ctx->ncu;
     if (2 * e * (p.group_size / 64) <= 3 * ncu) return {8, p.group_size > 64};
-    if (e <= 3 * ncu) return {8, false};
+    if (e <= 6 * ncu) return {8, false};
     if (e <= 16 * ncu) return {4, false};
     return {0, false};
 }
