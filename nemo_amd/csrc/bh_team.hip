@@ -166,17 +166,20 @@ __global__ __launch_bounds__(64 * W) void k_walk_team(WalkArgs a)
     const int split = rows < a.grows ? a.grows : 1;     // teams per group
     const int nitem = (int)a.stat[S_NGROUPS] * split;
 
-    if (threadIdx.x == 0) *next = atomicAdd(a.gctr, 1);
-    __syncthreads();
-    int item = *next;
+    // The first item by the block's number, the others by tickets; an item's
+    // group is loaded before the item is begun (the loads at a group's start are
+    // round trips in a row that a small problem shows in full).
+    int item = blockIdx.x;
+    const bool nocell = *a.ncellp == 0;
+    int gfirst = a.gfirst[item / split], gsize = a.gcount[item / split];
     while (item < nitem) {
         // (read by every thread before the barrier below that precedes this
         // group's end; the atomic's round trip hides behind the walk)
         int gnext = 0;
-        if (threadIdx.x == 0) gnext = atomicAdd(a.gctr, 1);
+        if (threadIdx.x == 0) gnext = (int)gridDim.x + atomicAdd(a.gctr, 1);
         const int g = item / split, r0 = item % split;  // group, and this team's first row
-        const int64_t gbase = a.gfirst[g];
-        const int gcount = a.gcount[g];
+        const int64_t gbase = gfirst;
+        const int gcount = gsize;
         const int nq = (gcount + 63) >> 6;
         const int nr = split > 1 ? 1 : nq;              // this team's rows and points
         const int mine0 = 64 * r0, mcount = min(gcount - mine0, 64 * nr);
@@ -184,6 +187,8 @@ __global__ __launch_bounds__(64 * W) void k_walk_team(WalkArgs a)
             if (threadIdx.x == 0) *next = gnext;
             __syncthreads();
             item = *next;
+            gfirst = a.gfirst[min(item, nitem - 1) / split];
+            gsize = a.gcount[min(item, nitem - 1) / split];
             __syncthreads();
             continue;
         }
@@ -296,7 +301,7 @@ __global__ __launch_bounds__(64 * W) void k_walk_team(WalkArgs a)
         nf = 1;
         if (sys >= 0) {
             root = a.sysroot[sys];
-        } else if (*a.ncellp == 0) {
+        } else if (nocell) {
             root = 0;
             nf = a.nb == 1 ? 1 : 0;
         }
@@ -309,6 +314,8 @@ __global__ __launch_bounds__(64 * W) void k_walk_team(WalkArgs a)
         for (int t = 0; t < kTasks; t++) ahi[t] = alo[t] = 0.f;
         __syncthreads();
         const int gn = *next;
+        gfirst = a.gfirst[min(gn, nitem - 1) / split];
+        gsize = a.gcount[min(gn, nitem - 1) / split];
 
         // Evaluates the first min(W, ne) waiting tiles, one per wave, and folds
         // their sums in order.  Ends with a barrier.
@@ -369,7 +376,7 @@ __global__ __launch_bounds__(64 * W) void k_walk_team(WalkArgs a)
                 const bool busy = base + 64 * w < nf;
                 int node = 0, c = 0, nk = 0, off = 0, wk = 0, bfirst = -1;
                 bool isBody = false, open = false, accept = false, take = false, far = false;
-                float4 A = make_float4(0.f, 0.f, 0.f, 0.f), bl = A;
+                float4 A = make_float4(0.f, 0.f, 0.f, 0.f), bl = A, q0 = A, q1 = A;
                 float rx = 0.f, ry = 0.f, rz = 0.f, size2 = 0.f;
                 int4 s0 = make_int4(kNoChild, kNoChild, kNoChild, kNoChild), s1 = s0;
                 unsigned long long mP = 0, mC = 0, mF = 0, mR = 0;
@@ -389,6 +396,10 @@ __global__ __launch_bounds__(64 * W) void k_walk_team(WalkArgs a)
                         s1 = reinterpret_cast<const int4 *>(a.sub)[2 * (int64_t)c + 1];
                         A = a.cA[c];
                         const float4 B = a.cB[c];
+                        if (QUAD) {      // (with the record: after the decision they are a round trip more per step)
+                            q0 = a.cQ0[c];
+                            q1 = a.cQ1[c];
+                        }
                         const int2 fn = a.fnb[c];
                         const int lv = a.level[c];
                         size2 = B.w;
@@ -487,8 +498,8 @@ __global__ __launch_bounds__(64 * W) void k_walk_team(WalkArgs a)
                     slot -= slot >= T::kC ? T::kC : 0;
                     Cl[S * slot] = make_float4(rx, ry, rz, A.w);
                     if (QUAD) {
-                        Cl[S * slot + 1] = a.cQ0[c];
-                        Cl[S * slot + 2] = a.cQ1[c];
+                        Cl[S * slot + 1] = q0;
+                        Cl[S * slot + 2] = q1;
                     }
                 }
                 nc += pct >> 16;
