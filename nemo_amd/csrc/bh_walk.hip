@@ -945,15 +945,18 @@ void launch(bh_ctx *ctx, WalkArgs &a, int grid, bool crit)
 // the points fill at least, e = points / group_size (a third more are cut),
 // against the device's CUs; walk times in us, quadrupole cells in brackets:
 //   one row per 8-wave team while the rows of all groups stay near one per CU
-//     (N = 10^4, groups of 128: 76 [87]; 8 waves per group 86 [111], one wave 391 [450]);
-//   8 waves per group up to 6 groups per CU (N = 5 10^4: 139 [191]; 4 waves
-//     190 [262], a row per team 177 [230], one wave 461 [626]; 1.6 10^5: 349 [494],
-//     4 waves 373 [520]; 2 10^5: 413 [571], 422 [570]);
-//   4 waves up to 16 per CU (N = 3 10^5: 563 [775], 8 waves 572 [797]; 4 10^5: 683
-//     [982]; 8 waves 737 [1013], one wave 749 [1028]; N = 2^20, groups of 256:
-//     1541; one wave 1671);
-//   then one wave, whose tiles never wait for another's (N = 2^20, groups of
-//     128: 1559 [2090]; 4 waves 1595 [2251]; N = 2^22: 5640 [7070]; 6090 [8740]).
+//     (N = 10^4, groups of 128: 64 [78]; 8 waves per group, before both took
+//     their loads early, 86 [111] against 76 [87]; one wave 391 [450]);
+//   8 waves per group up to 6 groups per CU (N = 5 10^4: 128 [169]; 4 waves
+//     181 [237], a row per team 176 [215], one wave 461 [626]; 2 10^5: 398 [549],
+//     4 waves 402 [572]);
+//   4 waves up to 16 per CU (N = 3 10^5: 533 [760], 8 waves 557 [767]; 4 10^5: 668
+//     [954], 8 waves 717 [985], one wave 746 [1013]), and to 32 for monopole
+//     cells and groups of at most 128 (8 10^5: 1206, one wave 1257; 2^20: 1535 and
+//     1604; 1.5 10^6: 2164 and 2179; but quadrupoles 1340 and 1255 at 6 10^5,
+//     groups of 192 1170 and 1127 at 8 10^5, local expansions 1211 and 1071);
+//   then one wave, whose tiles never wait for another's (N = 2^22, groups of
+//     128: 5617 [7037]; 4 waves 5676 [8612]).
 struct Walkers {
     int waves;
     bool split;
@@ -964,7 +967,8 @@ Walkers walkers(const bh_ctx *ctx, const bh_params &p, int64_t nt, int K)
     const int64_t e = std::max<int64_t>(nt / p.group_size, ctx->nsys), ncu = ctx->ncu;
     if (2 * e * (p.group_size / 64) <= 3 * ncu) return {8, p.group_size > 64};
     if (e <= 6 * ncu) return {8, false};
-    if (e <= 16 * ncu) return {4, false};
+    const bool light = !p.usequad && !p.learned && p.local_alpha == 0.0 && p.group_size <= 128;
+    if (e <= (light ? 32 : 16) * ncu) return {4, false};
     return {0, false};
 }
 
