@@ -166,17 +166,25 @@ __global__ __launch_bounds__(64 * W) void k_walk_team(WalkArgs a)
     const int split = rows < a.grows ? a.grows : 1;     // teams per group
     const int nitem = (int)a.stat[S_NGROUPS] * split;
 
-    // The first item by the block's number, the others by tickets; an item's
-    // group is loaded before the item is begun (the loads at a group's start are
-    // round trips in a row that a small problem shows in full).
+    // The first item by the block's number, the others by tickets, drawn as late
+    // in a group as the round trip can still be hidden (a team that holds its
+    // next ticket through a long walk leaves work waiting: 2 10^5 bodies 390 us,
+    // now 343); the range of the next group is loaded before it is begun.
     int item = blockIdx.x;
-    const bool nocell = *a.ncellp == 0;
+    const bool nocell = *a.ncellp == 0, once = nitem <= (int)gridDim.x;
     int gfirst = a.gfirst[item / split], gsize = a.gcount[item / split];
+    auto enter = [&](int to) {
+        item = to;
+        gfirst = a.gfirst[min(to, nitem - 1) / split];
+        gsize = a.gcount[min(to, nitem - 1) / split];
+    };
+    auto advance = [&]() {
+        if (threadIdx.x == 0) *next = once ? nitem : (int)gridDim.x + atomicAdd(a.gctr, 1);
+        __syncthreads();
+        enter(*next);
+        __syncthreads();
+    };
     while (item < nitem) {
-        // (read by every thread before the barrier below that precedes this
-        // group's end; the atomic's round trip hides behind the walk)
-        int gnext = 0;
-        if (threadIdx.x == 0) gnext = (int)gridDim.x + atomicAdd(a.gctr, 1);
         const int g = item / split, r0 = item % split;  // group, and this team's first row
         const int64_t gbase = gfirst;
         const int gcount = gsize;
@@ -184,12 +192,7 @@ __global__ __launch_bounds__(64 * W) void k_walk_team(WalkArgs a)
         const int nr = split > 1 ? 1 : nq;              // this team's rows and points
         const int mine0 = 64 * r0, mcount = min(gcount - mine0, 64 * nr);
         if (mcount <= 0) {
-            if (threadIdx.x == 0) *next = gnext;
-            __syncthreads();
-            item = *next;
-            gfirst = a.gfirst[min(item, nitem - 1) / split];
-            gsize = a.gcount[min(item, nitem - 1) / split];
-            __syncthreads();
+            advance();
             continue;
         }
         float tolsq = a.tolsq, eps2 = a.eps2;
@@ -305,17 +308,11 @@ __global__ __launch_bounds__(64 * W) void k_walk_team(WalkArgs a)
             root = 0;
             nf = a.nb == 1 ? 1 : 0;
         }
-        if (threadIdx.x == 0) {
-            lf0[0] = root;
-            *next = gnext;
-        }
+        if (threadIdx.x == 0) lf0[0] = root;
         float ahi[kTasks], alo[kTasks];                 // this wave's (row, component) sums
 #pragma unroll
         for (int t = 0; t < kTasks; t++) ahi[t] = alo[t] = 0.f;
         __syncthreads();
-        const int gn = *next;
-        gfirst = a.gfirst[min(gn, nitem - 1) / split];
-        gsize = a.gcount[min(gn, nitem - 1) / split];
 
         // Evaluates the first min(W, ne) waiting tiles, one per wave, and folds
         // their sums in order.  Ends with a barrier.
@@ -552,17 +549,26 @@ __global__ __launch_bounds__(64 * W) void k_walk_team(WalkArgs a)
         if (overflow) {
             if (threadIdx.x == 0) atomicOr(&a.counters[S_FLAGS], (unsigned long long)F_FRONTIER);
             __syncthreads();
-            item = gn;
+            advance();
             continue;
         }
         // the last full tiles, then the two partial ones (bodies first)
+        // and the next ticket
+        int ticket = 0;
         if (threadIdx.x == 0) {
+            if (!once) ticket = (int)gridDim.x + atomicAdd(a.gctr, 1);
             int at = eh + ne;
             if (np & 63) ev[at++ & (T::kEv - 1)] = ((np & 63) << 1) | (((np >> 6) % (T::kP / 64)) << 8);
             if (nc & 63) ev[at & (T::kEv - 1)] = 1 | ((nc & 63) << 1) | (((nc >> 6) % (T::kC / 64)) << 8);
         }
         ne += ((np & 63) != 0) + ((nc & 63) != 0);
         __syncthreads();
+        if (!once) {
+            if (ne > 0) eval_tiles();
+            if (threadIdx.x == 0) *next = ticket;
+            __syncthreads();
+            enter(*next);
+        }
         while (ne > 0) eval_tiles();
         if (LOCAL && nfl > 0) {
             for (int rest = nfl - 64 * df; rest > 0; rest -= 64 * W) eval_far(min(64 * W, rest));
@@ -623,8 +629,8 @@ __global__ __launch_bounds__(64 * W) void k_walk_team(WalkArgs a)
                 if (LOCAL) atomicAdd(&a.counters[S_NLOC], (unsigned long long)((long long)nfl * mcount));
             }
         }
+        if (once) break;
         __syncthreads();   // the lists, positions and self flags are reused
-        item = gn;
     }
 }
 
