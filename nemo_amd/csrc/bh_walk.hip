@@ -945,18 +945,32 @@ void launch(bh_ctx *ctx, WalkArgs &a, int grid, bool crit)
 // the points fill at least, e = points / group_size (a third more are cut),
 // against the device's CUs; walk times in us, quadrupole cells in brackets:
 //   one row per 8-wave team while the rows of all groups stay near one per CU
-//     (N = 10^4, groups of 128: 64 [78]; 8 waves per group, before both took
+//     (N = 10^4, groups of 128: 64 [77]; 8 waves per group, before both took
 //     their loads early, 86 [111] against 76 [87]; one wave 391 [450]);
-//   8 waves per group up to 6 groups per CU (N = 5 10^4: 128 [169]; 4 waves
-//     181 [237], a row per team 176 [215], one wave 461 [626]; 2 10^5: 398 [549],
-//     4 waves 402 [572]);
-//   4 waves up to 16 per CU (N = 3 10^5: 533 [760], 8 waves 557 [767]; 4 10^5: 668
-//     [954], 8 waves 717 [985], one wave 746 [1013]), and to 32 for monopole
-//     cells and groups of at most 128 (8 10^5: 1206, one wave 1257; 2^20: 1535 and
-//     1604; 1.5 10^6: 2164 and 2179; but quadrupoles 1340 and 1255 at 6 10^5,
-//     groups of 192 1170 and 1127 at 8 10^5, local expansions 1211 and 1071);
+//   8 waves per group up to 6 groups per CU (N = 5 10^4: 127 [169]; 4 waves
+//     181 [237], a row per team 176 [215], one wave 461 [626]; 2 10^5: 350 [520],
+//     4 waves 354 [521]);
+//   4 waves up to four_waves() groups per CU (N = 4 10^5: 622 [903], 8 waves 694
+//     [942], one wave 737 [994]);
 //   then one wave, whose tiles never wait for another's (N = 2^22, groups of
-//     128: 5617 [7037]; 4 waves 5676 [8612]).
+//     128: 5564 [7158]; 4 waves 5601 [8619]).
+// four_waves: what a team gains shrinks with the rows of a group and with the
+// cost of its tiles (4 waves against one, us): monopole cells, groups of 64
+// 2424 / 4217 at 1.5 10^6 (92 per CU), of 128 2058 / 2152 there (46; tol 0.5
+// 3817 / 3673), of 192 1381 / 1414 at 2^20 and 1938 / 1853 at 1.5 10^6 (21, 31),
+// of 256 2104 / 2245 there (23); quadrupoles at tol 0.5, groups of 128 4203 /
+// 4444 at 2^20 (32), of 192 4788 / 4927 at 10^6 (20); at tol 0.7, 1649 / 1653 at
+// 8 10^5 (24) and 2145 / 1942 at 2^20, of 192 1531 / 1486 at 6 10^5 and 1971 /
+// 1856 at 8 10^5 (12, 16); local expansions, groups of 192 926 / 953 at 6 10^5
+// and 1169 / 1060 at 8 10^5.
+int four_waves(const bh_params &p)
+{
+    const int g = p.group_size;
+    if (p.learned || p.local_alpha > 0.0 || p.criterion != BH_CRIT_HACK) return 16;
+    if (!p.usequad) return g == 64 ? 96 : g == 128 ? 48 : 24;
+    if (p.tol <= 0.6) return g <= 128 ? 36 : 20;
+    return g <= 128 ? 20 : 14;
+}
 struct Walkers {
     int waves;
     bool split;
@@ -967,8 +981,7 @@ Walkers walkers(const bh_ctx *ctx, const bh_params &p, int64_t nt, int K)
     const int64_t e = std::max<int64_t>(nt / p.group_size, ctx->nsys), ncu = ctx->ncu;
     if (2 * e * (p.group_size / 64) <= 3 * ncu) return {8, p.group_size > 64};
     if (e <= 6 * ncu) return {8, false};
-    const bool light = !p.usequad && !p.learned && p.local_alpha == 0.0 && p.group_size <= 128;
-    if (e <= (light ? 32 : 16) * ncu) return {4, false};
+    if (e <= four_waves(p) * ncu) return {4, false};
     return {0, false};
 }
 
