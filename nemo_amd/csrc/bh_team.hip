@@ -3,7 +3,7 @@
 // k_walk (bh_walk.hip) gives a group to one wave.  That fills the device when
 // there are several groups for each of its ~4096 resident waves; below that
 // the walk's time is one wave's serial walk of its group (N = 10^4, quadrupole
-// cells: 120 groups, 0.45 ms; here 0.087 ms).  Here the W waves of a block
+// cells: 120 groups, 0.45 ms; here 0.077 ms).  Here the W waves of a block
 // share the group's work:
 //   traversal  each step tests 64 W frontier nodes, 64 per wave, and appends
 //              bodies, accepted cells and children at offsets from a scan of
