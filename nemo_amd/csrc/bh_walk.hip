@@ -944,9 +944,11 @@ void launch(bh_ctx *ctx, WalkArgs &a, int grid, bool crit)
 // (k_walk_team), which may take one 64-point row of it (split).  By the groups
 // the points fill at least, e = points / group_size (a third more are cut),
 // against the device's CUs; walk times in us, quadrupole cells in brackets:
-//   one row per 8-wave team while the rows of all groups stay near one per CU
-//     (N = 10^4, groups of 128: 64 [77]; 8 waves per group, before both took
-//     their loads early, 86 [111] against 76 [87]; one wave 391 [450]);
+//   one row per 8-wave team while the teams of all rows are resident together
+//     (two per CU; N = 10^4, groups of 128: 64 [77]; 8 waves per group, before
+//     both took their loads early, 86 [111] against 76 [87]; one wave 391 [450];
+//     2.8 10^4: 80 [95], 8 waves per group 100 [131]; 3.6 10^4: 122 [147], 109
+//     [146]);
 //   8 waves per group up to 6 groups per CU (N = 5 10^4: 127 [169]; 4 waves
 //     181 [237], a row per team 176 [215], one wave 461 [626]; 2 10^5: 350 [520],
 //     4 waves 354 [521]);
@@ -979,7 +981,7 @@ Walkers walkers(const bh_ctx *ctx, const bh_params &p, int64_t nt, int K)
 {
     if (K > 1) return {0, false};
     const int64_t e = std::max<int64_t>(nt / p.group_size, ctx->nsys), ncu = ctx->ncu;
-    if (2 * e * (p.group_size / 64) <= 3 * ncu) return {8, p.group_size > 64};
+    if (4 * e * (p.group_size / 64) <= 7 * ncu) return {8, p.group_size > 64};
     if (e <= 6 * ncu) return {8, false};
     if (e <= four_waves(p) * ncu) return {4, false};
     return {0, false};
